@@ -81,6 +81,11 @@ void launch_embed_q8_0(const uint8_t* table, const int32_t* ids, float* out, int
 void launch_quant_q8_0(const float* x, uint8_t* y, int64_t n_elements, hipStream_t s);
 void launch_q8_0_dispatch_T(const uint8_t* Wq, const uint8_t* Xq, float* out, int m_weight, int m_tokens, int K,
                             hipStream_t s);
+// Up to 3 matrices of M[i] >= 1 rows sharing the activation rows Xq in order T, one launch
+// (q8_0_t.hip): out[i][token * M[i] + row]; false (nothing launched) where the per-token
+// GEMVs are the faster ones.
+bool launch_q8_0_gemm_T_multi(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq,
+                              int m_tokens, int K, hipStream_t s);
 void launch_q8_pad64(const float* x, uint8_t* out, int N, int K, hipStream_t s);
 void launch_q8_pad64_dispatch_T(const uint8_t* Wp, const uint8_t* Xq, float* out, int m_weight, int m_tokens, int K,
                                 hipStream_t s);

@@ -2037,8 +2037,8 @@ void mt_gemm(const MtCtx& c, const uint8_t* W, float* out, int mw, int K, const 
         launch_q8_0_dispatch_T(W, xq, out, mw, c.T, K, c.s);
 }
 
-// n GEMMs of the same activation rows (Q/K/V, gate/up): order S in one launch,
-// order T one dispatch each.  (Q/K/V of 512 tokens of a Mistral-7B layer, 6144
+// n GEMMs of the same activation rows (Q/K/V, gate/up) in one launch; order T with
+// few cells one dispatch each.  (Q/K/V of 512 tokens of a Mistral-7B layer, 6144
 // rows in all: 76 us in one launch against 174 us in three, each of which left
 // most CUs idle.)
 void mt_gemm3(const MtCtx& c, std::initializer_list<const uint8_t*> W, std::initializer_list<float*> out,
@@ -2053,6 +2053,7 @@ void mt_gemm3(const MtCtx& c, std::initializer_list<const uint8_t*> W, std::init
         launch_q8_0_gemm_S_multi(w, o, m, n, c.xq, c.T, K, 1, c.s);
         return;
     }
+    if (launch_q8_0_gemm_T_multi(w, o, m, n, c.xq, c.T, K, c.s)) return;
     for (int i = 0; i < n; i++) mt_gemm(c, w[i], o[i], m[i], K);
 }
 

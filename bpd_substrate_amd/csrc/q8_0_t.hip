@@ -1,0 +1,575 @@
+// q8_0_t.hip — Q8_0 x Q8_0 for several activation rows in the AVX1 tile order T
+// (bench/bpd_gemm_q8_0_cpu.c:32-86), on f16 MFMA.
+#include "bpdq_device.h"
+#include "bpdq_launch.h"
+#include "bpdq_q8_0.h"
+
+namespace bpdq {
+
+// ----------------------------------------------------------------------------
+// k_q8_0_gemm_TM.  Per cell and lane L = 0..7 of the reference's vector, over the
+// blocks b in order:  acc_L = RN(RN(RN(Ad*Bd) * p_L) + acc_L), p_L the exact dot of
+// elements 4L..4L+3 of the two blocks; the cell is
+// ((a0+a4)+(a2+a6))+((a1+a5)+(a3+a7)).  The 16 fp32 operations per cell and block
+// cannot be merged (each result is rounded), so the VALU bounds this product; the
+// kernel gives it nothing else to do:
+//  - v_mfma_f32_16x16x4_4b_f16 computes four independent 16x16 products of inner
+//    length 4: with the quants as f16 (exact) its "block" k gives p_L of 16 rows x
+//    16 tokens as the exact fp32 value (|p_L| <= 65,536), so there is no
+//    int-to-float conversion.  Two of them (L = 2k, L = 2k+1) cover a Q8_0 block.
+//  - the same instruction with the two f16 scales at inner index 0 and zeros
+//    elsewhere gives RN(Ad*Bd) (exact: 11 x 11 bits) of two blocks x two column
+//    tiles at once.
+// A workgroup owns R = 16 WRN weight rows x C = 16 CT WCN tokens; each of its WRN x
+// WCN waves 16 rows x 16 CT tokens: 32 CT accumulators per lane.  A stage is 2 blocks
+// (68 bytes of a row), staged by 4 threads per row: a thread loads half a block,
+// turns its 16 quants to f16 (0x6400 | (q ^ 0x80) is 1152 + q) and writes 32 bytes.
+// PF stages are in flight in registers, two LDS slots alternate, one barrier per
+// stage (LDS only, so the loads stay in flight across it).
+// LDS: [block][row][64 bytes]; the 16-byte chunk k of a row (quants 8k..8k+7) sits
+// at k ^ ((row >> 2) & 3) and a block's plane is padded by 16 bytes, so that 16
+// consecutive lanes reading (16 rows, one chunk) or writing (4 rows, two blocks, two
+// chunks) touch 16 different 16-byte groups modulo 256.
+// Blocks past the end of a row have zero scales: acc + 0 is acc (a chain that
+// starts at +0.0 never is -0.0).  Rows and tokens past the end repeat the last one.
+// ----------------------------------------------------------------------------
+typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
+typedef float tf32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t tu32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t tu32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
+typedef uint32_t tu32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int WRN, int WCN, int CT>
+struct TmGeo {
+    static constexpr int R = 16 * WRN, C = 16 * CT * WCN, ROWS = R + C;
+    static constexpr int NT = 64 * WRN * WCN, UNITS = 4 * ROWS;  // staging threads (UNITS % 64 == 0)
+    static constexpr int PASSES = (UNITS + NT - 1) / NT;
+    static constexpr int PLANE = ROWS * 64 + 16;                 // bytes of one block's quants
+    static constexpr int SLOT = 2 * PLANE + 2 * ROWS * 4;        // quants, then the scales [block][row]
+};
+
+struct TmRaw {
+    tu32x4 q;    // AL: the dwords at the half block's (aligned) start; else its 16 quants
+    uint32_t e;  // AL: the dword after them; else the block's scale
+};
+
+// 4 int8 quants -> 4 f16.
+__device__ __forceinline__ uint2 tm_f16(uint32_t q) {
+    const uint32_t u = q ^ 0x80808080u;  // q + 128 per byte
+    const h16x2 bias = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    const h16x2 lo = __builtin_bit_cast(h16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) + bias;
+    const h16x2 hi = __builtin_bit_cast(h16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) + bias;
+    return make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+}
+
+// AL: W, X 4-byte aligned and nb even: part p of a stage's 68 bytes is loaded from
+// dword offset {0, 16, 36, 52} (block 0's quants start 2 bytes into a dword).
+template <bool AL>
+__device__ __forceinline__ void tm_load(TmRaw& t, const uint8_t* __restrict__ src, int p, int st, int nst, int nb) {
+    if constexpr (AL) {
+        const uint8_t* s = src + (int64_t)min(st, nst - 1) * (2 * kQ80Bytes) + 16 * p + (p >= 2 ? 4 : 0);
+        t.q = *reinterpret_cast<const tu32x4_a4*>(s);
+        t.e = *reinterpret_cast<const uint32_t*>(s + (p >= 2 ? 12 : 16));
+    } else {
+        const uint8_t* s = src + (int64_t)min(2 * st + (p >> 1), nb - 1) * kQ80Bytes;
+        t.q = *reinterpret_cast<const tu32x4_a1*>(s + 2 + 16 * (p & 1));
+        t.e = ld_u16(s);
+    }
+}
+
+// Stage st of one staging thread into a slot; returns the OR of has_m128 of its quants.
+template <bool AL, int ROWS, int PLANE>
+__device__ __forceinline__ uint32_t tm_store(uint8_t* slot, const TmRaw& t, int row, int p, int st, int nb, bool want) {
+    uint32_t q[4], d;
+    if constexpr (AL) {
+        const uint32_t sh = p >= 2 ? 0u : 16u;
+        q[0] = __builtin_amdgcn_alignbit(t.q[1], t.q[0], sh);
+        q[1] = __builtin_amdgcn_alignbit(t.q[2], t.q[1], sh);
+        q[2] = __builtin_amdgcn_alignbit(t.q[3], t.q[2], sh);
+        q[3] = __builtin_amdgcn_alignbit(t.e, t.q[3], sh);
+        d = p == 0 ? (t.q[0] & 0xFFFFu) : (t.e >> 16);  // block 1's scale: high half of part 1's last dword
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; i++) q[i] = t.q[i];
+        d = t.e;
+    }
+    const int u = p >> 1, h = p & 1, swz = (row >> 2) & 3;
+    uint8_t* base = slot + u * PLANE + row * 64;
+    const uint2 a = tm_f16(q[0]), b = tm_f16(q[1]), c = tm_f16(q[2]), e = tm_f16(q[3]);
+    *reinterpret_cast<uint4*>(base + 16 * ((2 * h) ^ swz)) = make_uint4(a.x, a.y, b.x, b.y);
+    *reinterpret_cast<uint4*>(base + 16 * ((2 * h + 1) ^ swz)) = make_uint4(c.x, c.y, e.x, e.y);
+    uint32_t* sc = reinterpret_cast<uint32_t*>(slot + 2 * PLANE);
+    if constexpr (AL) {
+        if (p < 2) sc[p * ROWS + row] = d;
+    } else {
+        if (h == 0) sc[u * ROWS + row] = 2 * st + u < nb ? d : 0u;
+    }
+    if (!want) return 0u;
+    return has_m128(q[0]) | has_m128(q[1]) | has_m128(q[2]) | has_m128(q[3]);
+}
+
+template <int WRN, int WCN, int CT, int PF, bool AL>
+__global__ __launch_bounds__(64 * WRN * WCN) void k_q8_0_gemm_TM(GemmW gw, const uint8_t* __restrict__ X, int m_tokens,
+                                                                 int nb) {
+    using G = TmGeo<WRN, WCN, CT>;
+    static_assert(PF % 2 == 0 && (CT == 1 || CT == 2), "slot parity; one scale product per stage");
+    __shared__ __align__(16) uint8_t lds[2 * G::SLOT];
+    __shared__ uint32_t m128[G::C];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = wave / WCN, wc = wave % WCN;
+    int bx, by;
+    sh_tile(blockIdx.x, gw.first[kGemmMulti], (m_tokens + G::C - 1) / G::C, bx, by);
+    const int mi = (bx >= gw.first[1]) + (bx >= gw.first[2]);
+    const uint8_t* __restrict__ W = gw.w[mi];
+    float* __restrict__ out = gw.out[mi];
+    const int m_weight = gw.m[mi];
+    const int m0 = (bx - gw.first[mi]) * G::R, n0 = by * G::C;
+    const int64_t bpr = (int64_t)nb * kQ80Bytes;
+    const int nst = (nb + 1) / 2;
+
+    // staging: unit tid + ps * NT is part p of staged row (the R weight rows, then the C tokens)
+    const uint8_t* src[G::PASSES];
+    int srow[G::PASSES];
+    const int p = tid & 3;
+#pragma unroll
+    for (int ps = 0; ps < G::PASSES; ps++) {
+        const int row = min((tid + ps * G::NT) >> 2, G::ROWS - 1);
+        srow[ps] = row;
+        src[ps] = row < G::R ? W + (int64_t)min(m0 + row, m_weight - 1) * bpr
+                             : X + (int64_t)min(n0 + row - G::R, m_tokens - 1) * bpr;
+    }
+    for (int i = tid; i < G::C; i += G::NT) m128[i] = 0u;
+
+    TmRaw raw[PF][G::PASSES];
+    uint32_t bad[G::PASSES] = {};
+    const auto load = [&](TmRaw (&r)[G::PASSES], int st) {
+#pragma unroll
+        for (int ps = 0; ps < G::PASSES; ps++)
+            if ((ps + 1) * G::NT <= G::UNITS || tid + ps * G::NT < G::UNITS) tm_load<AL>(r[ps], src[ps], p, st, nst, nb);
+    };
+    const auto store = [&](const TmRaw (&r)[G::PASSES], int slot, int st) {
+#pragma unroll
+        for (int ps = 0; ps < G::PASSES; ps++)
+            if ((ps + 1) * G::NT <= G::UNITS || tid + ps * G::NT < G::UNITS)
+                bad[ps] |= tm_store<AL, G::ROWS, G::PLANE>(lds + slot * G::SLOT, r[ps], srow[ps], p, st, nb,
+                                                           srow[ps] >= G::R);
+    };
+#pragma unroll
+    for (int i = 0; i < PF; i++) load(raw[i], i);
+    store(raw[0], 0, 0);
+    load(raw[0], PF);
+    lds_barrier();
+
+    float acc[CT][8][4];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++)
+#pragma unroll
+        for (int L = 0; L < 8; L++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) acc[ct][L][r] = 0.0f;
+
+    const int j = lane & 15, k = lane >> 4;
+    const int frag = j * 64 + 16 * (k ^ (j >> 2));  // this lane's chunk in a 16-row tile
+    const int arow = wr * 16, brow = G::R + wc * 16 * CT;
+    // scale operands: lane group k gives block k & 1, column tile k >> 1
+    const int asc = (k & 1) * G::ROWS + arow + j, bsc = (k & 1) * G::ROWS + brow + (CT == 2 ? 16 * (k >> 1) : 0) + j;
+    const tf32x16 zero = {0.0f};
+
+    for (int s0 = 0; s0 < nst; s0 += PF) {
+#pragma unroll
+        for (int i = 0; i < PF; i++) {
+            const int st = s0 + i;
+            if (st >= nst) break;
+            if (st + 1 < nst) {  // the other slot was last read before the previous barrier
+                store(raw[(i + 1) % PF], (i + 1) & 1, st + 1);
+                load(raw[(i + 1) % PF], st + 1 + PF);
+            }
+            const uint8_t* slot = lds + (i & 1) * G::SLOT;
+            const uint32_t* sc = reinterpret_cast<const uint32_t*>(slot + 2 * G::PLANE);
+            const h16x4 sa = __builtin_bit_cast(h16x4, make_uint2(sc[asc], 0u));
+            const h16x4 sb = __builtin_bit_cast(h16x4, make_uint2(sc[bsc], 0u));
+            const tf32x16 delta = __builtin_amdgcn_mfma_f32_16x16x4f16(sa, sb, zero, 0, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const uint4 fa = *reinterpret_cast<const uint4*>(slot + u * G::PLANE + arow * 64 + frag);
+                const h16x4 a0 = __builtin_bit_cast(h16x4, make_uint2(fa.x, fa.y));
+                const h16x4 a1 = __builtin_bit_cast(h16x4, make_uint2(fa.z, fa.w));
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) {
+                    const uint4 fb = *reinterpret_cast<const uint4*>(slot + u * G::PLANE + (brow + 16 * ct) * 64 + frag);
+                    const h16x4 b0 = __builtin_bit_cast(h16x4, make_uint2(fb.x, fb.y));
+                    const h16x4 b1 = __builtin_bit_cast(h16x4, make_uint2(fb.z, fb.w));
+                    const tf32x16 p0 = __builtin_amdgcn_mfma_f32_16x16x4f16(a0, b0, zero, 0, 0, 0);
+                    const tf32x16 p1 = __builtin_amdgcn_mfma_f32_16x16x4f16(a1, b1, zero, 0, 0, 0);
+#pragma unroll
+                    for (int g = 0; g < 4; g++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const float d = delta[4 * (u + 2 * ct) + r];
+                            acc[ct][2 * g][r] = d * p0[4 * g + r] + acc[ct][2 * g][r];
+                            acc[ct][2 * g + 1][r] = d * p1[4 * g + r] + acc[ct][2 * g + 1][r];
+                        }
+                }
+            }
+            lds_barrier();
+        }
+    }
+
+#pragma unroll
+    for (int ps = 0; ps < G::PASSES; ps++)
+        if (bad[ps] != 0) m128[srow[ps] - G::R] = 1u;
+    __syncthreads();
+    // register r of lane l: row 4 (l / 16) + r of the wave's 16, token l % 16 of column tile ct
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+        const int tl = wc * 16 * CT + 16 * ct + j, tok = n0 + tl;
+        if (tok >= m_tokens) continue;
+        const int r0 = m0 + arow + 4 * k;
+        float y[4];
+        bool odd = m128[tl] != 0;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const float(&a)[8][4] = acc[ct];
+            y[r] = ((a[0][r] + a[4][r]) + (a[2][r] + a[6][r])) + ((a[1][r] + a[5][r]) + (a[3][r] + a[7][r]));
+            odd |= __builtin_isnan(y[r]);
+        }
+        if (odd) {  // the reference's own arithmetic: NaN bits, -128 activation quants
+            for (int r = 0; r < 4; r++)
+                if (r0 + r < m_weight && (m128[tl] != 0 || __builtin_isnan(y[r])))
+                    y[r] = t_order_cell(W + (r0 + r) * bpr, kQ80Bytes, 2, X + tok * bpr, nb, r0 + r, tok, m_weight,
+                                        m_tokens);
+        }
+        float* o = out + (int64_t)tok * m_weight + r0;
+        if ((reinterpret_cast<uintptr_t>(o) & 15) == 0 && r0 + 4 <= m_weight) {
+            *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (r0 + r < m_weight) o[r] = y[r];
+        }
+    }
+}
+
+// ----------------------------------------------------------------------------
+// k_q8_0_gemm_TQ: the same cells on v_mfma_f32_4x4x4_16b_f16, 16 independent 4x4
+// products of inner length 4, for few tokens.  A wave owns 8 rows; "block" L + 8 rg
+// of the instruction gives p_L of rows 4 rg .. 4 rg + 3 x 4 tokens, so a lane holds
+// the chains of 4 rows for one (L, token), and the accumulators of 4 NQ tokens are
+// 4 NQ registers.  Each wave streams its own rows in chunks of CB blocks through
+// registers (two chunks in flight) and its own LDS slot as 16-byte pieces; the
+// workgroup shares only the activation chunk (f16, two slots), so there is one
+// barrier per CB blocks.  Needs nb % 8 == 0 and W 16-byte aligned.
+// LDS: rows at an odd multiple of 8 dwords (8 rows x 8 quant dwords of a block touch
+// 64 different banks); the quants of 4 tokens of a block are 256 contiguous bytes.
+// ----------------------------------------------------------------------------
+typedef float tf32x4 __attribute__((ext_vector_type(4)));
+
+template <int NQ, int NW, int CB>
+struct TqGeo {
+    static constexpr int C = 4 * NQ, R = 8 * NW, NT = 64 * NW;
+    static constexpr int PIECES = CB * 17 / 8;  // 16-byte pieces of a row's chunk
+    static constexpr int WP = 8 * PIECES, PER = (WP + 63) / 64;
+    static constexpr int PITCH = CB == 8 ? 288 : CB == 16 ? 544 : 1120;
+    static constexpr int PLANE = C * 64 + 32;             // one block's activation quants
+    static constexpr int XSLOT = CB * PLANE + CB * C * 4;  // quants, then the scales [block pair][token][2]
+    static constexpr int UX = C * CB * 2, XP = (UX + NT - 1) / NT;
+    static constexpr int LDS = 2 * XSLOT + NW * 8 * PITCH;
+    static_assert(PITCH >= 16 * PIECES && PITCH % 16 == 0 && (PITCH / 32) % 2 == 1 && PITCH % 32 == 0 && CB % 8 == 0 &&
+                      XSLOT % 16 == 0, "LDS geometry");
+};
+
+struct TqX {
+    tu32x4 q;
+    uint32_t d;
+};
+
+// The operands of blocks 2t and 2t + 1 of a chunk: this lane's weight dwords, the
+// scales of its row, and per 4 tokens the quants and both scales.
+template <int NQ>
+struct TqOps {
+    uint32_t lo, hi, q1, d0, d1;
+    uint2 b0[NQ], b1[NQ];
+    float2 s[NQ];
+};
+
+template <int NQ, int C, int PLANE>
+__device__ __forceinline__ void tq_read(TqOps<NQ>& o, const uint8_t* wq, const uint8_t* wd, const uint8_t* xq,
+                                        const float2* xd, int t) {
+    o.lo = *reinterpret_cast<const uint32_t*>(wq + 68 * t);  // block 2t: quants 2 bytes into a dword
+    o.hi = *reinterpret_cast<const uint32_t*>(wq + 68 * t + 4);
+    o.q1 = *reinterpret_cast<const uint32_t*>(wq + 68 * t + 36);
+    o.d0 = *reinterpret_cast<const uint16_t*>(wd + 68 * t);
+    o.d1 = *reinterpret_cast<const uint16_t*>(wd + 68 * t + 34);
+#pragma unroll
+    for (int n = 0; n < NQ; n++) {
+        o.b0[n] = *reinterpret_cast<const uint2*>(xq + 2 * t * PLANE + 256 * n);
+        o.b1[n] = *reinterpret_cast<const uint2*>(xq + (2 * t + 1) * PLANE + 256 * n);
+        o.s[n] = xd[t * C + 4 * n];
+    }
+}
+
+template <int NQ>
+__device__ __forceinline__ void tq_pair(const TqOps<NQ>& o, float (&acc)[NQ][4]) {
+    const tf32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const h16x4 a0 = __builtin_bit_cast(h16x4, tm_f16(__builtin_amdgcn_alignbit(o.hi, o.lo, 16)));
+    const h16x4 a1 = __builtin_bit_cast(h16x4, tm_f16(o.q1));
+    const float d0 = f16_ieee(o.d0), d1 = f16_ieee(o.d1);
+    tf32x4 p0[NQ], p1[NQ], e0[NQ], e1[NQ];
+#pragma unroll
+    for (int n = 0; n < NQ; n++) {
+        e0[n] = __builtin_amdgcn_mfma_f32_4x4x1f32(d0, o.s[n].x, zero, 0, 0, 0);
+        p0[n] = __builtin_amdgcn_mfma_f32_4x4x4f16(a0, __builtin_bit_cast(h16x4, o.b0[n]), zero, 0, 0, 0);
+        e1[n] = __builtin_amdgcn_mfma_f32_4x4x1f32(d1, o.s[n].y, zero, 0, 0, 0);
+        p1[n] = __builtin_amdgcn_mfma_f32_4x4x4f16(a1, __builtin_bit_cast(h16x4, o.b1[n]), zero, 0, 0, 0);
+    }
+#pragma unroll
+    for (int n = 0; n < NQ; n++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[n][r] = e0[n][r] * p0[n][r] + acc[n][r];
+    }
+#pragma unroll
+    for (int n = 0; n < NQ; n++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[n][r] = e1[n][r] * p1[n][r] + acc[n][r];
+    }
+}
+
+template <int NQ, int NW, int CB>
+__global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_t* __restrict__ X, int m_tokens, int nb) {
+    using G = TqGeo<NQ, NW, CB>;
+    __shared__ __align__(16) uint8_t lds[G::LDS];
+    __shared__ uint32_t m128[G::C];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int bx, by;
+    sh_tile(blockIdx.x, gw.first[kGemmMulti], (m_tokens + G::C - 1) / G::C, bx, by);
+    const int mi = (bx >= gw.first[1]) + (bx >= gw.first[2]);
+    const uint8_t* __restrict__ W = gw.w[mi];
+    float* __restrict__ out = gw.out[mi];
+    const int m_weight = gw.m[mi];
+    const int row0 = (bx - gw.first[mi]) * G::R + wave * 8, n0 = by * G::C;
+    const int64_t bpr = (int64_t)nb * kQ80Bytes;
+    const int nch = (nb + CB - 1) / CB, npc = nb * 17 / 8;  // chunks, 16-byte pieces of a row
+
+    // weights: piece k of this lane is piece f % PIECES of row f / PIECES of the chunk
+    const uint8_t* wbase = W + (int64_t)min(row0, m_weight - 1) * bpr;
+    uint32_t off[G::PER], dst[G::PER];
+    int pc[G::PER];
+#pragma unroll
+    for (int k = 0; k < G::PER; k++) {
+        const int f = min(lane + 64 * k, G::WP - 1), r = f / G::PIECES;
+        pc[k] = f % G::PIECES;
+        off[k] = (uint32_t)((min(row0 + r, m_weight - 1) - min(row0, m_weight - 1)) * bpr);
+        dst[k] = (uint32_t)(r * G::PITCH + 16 * pc[k]);
+    }
+    uint8_t* slot = lds + 2 * G::XSLOT + wave * 8 * G::PITCH;
+    const auto wload = [&](tu32x4 (&v)[G::PER], int c) {
+#pragma unroll
+        for (int k = 0; k < G::PER; k++) {
+            const uint8_t* s = wbase + off[k] + 16 * min(c * G::PIECES + pc[k], npc - 1);
+            v[k] = *reinterpret_cast<const tu32x4*>(s);
+        }
+    };
+    // activations: unit i is half i & 1 of block (i / 2) % CB of token i / (2 CB)
+    TqX xr[G::XP];
+    const auto xload = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < G::XP; u++) {
+            const int i = min(tid + u * G::NT, G::UX - 1), t = i / (2 * CB), b = (i >> 1) % CB;
+            const uint8_t* s = X + (int64_t)min(n0 + t, m_tokens - 1) * bpr + (int64_t)min(c * CB + b, nb - 1) * kQ80Bytes;
+            xr[u].q = *reinterpret_cast<const tu32x4_a1*>(s + 2 + 16 * (i & 1));
+            xr[u].d = ld_u16(s);
+        }
+    };
+    uint32_t bad[G::XP] = {};
+    const auto xstore = [&](int xs) {
+        uint8_t* x = lds + xs * G::XSLOT;
+#pragma unroll
+        for (int u = 0; u < G::XP; u++) {
+            const int i = tid + u * G::NT, t = i / (2 * CB), b = (i >> 1) % CB;
+            if (G::UX % G::NT != 0 && i >= G::UX) continue;
+            const uint2 q0 = tm_f16(xr[u].q[0]), q1 = tm_f16(xr[u].q[1]), q2 = tm_f16(xr[u].q[2]), q3 = tm_f16(xr[u].q[3]);
+            uint4* d = reinterpret_cast<uint4*>(x + b * G::PLANE + t * 64 + 32 * (i & 1));
+            d[0] = make_uint4(q0.x, q0.y, q1.x, q1.y);
+            d[1] = make_uint4(q2.x, q2.y, q3.x, q3.y);
+            if ((i & 1) == 0)
+                reinterpret_cast<float*>(x + CB * G::PLANE)[2 * ((b >> 1) * G::C + t) + (b & 1)] = f16_ieee(xr[u].d);
+            bad[u] |= has_m128(xr[u].q[0]) | has_m128(xr[u].q[1]) | has_m128(xr[u].q[2]) | has_m128(xr[u].q[3]);
+        }
+    };
+
+    tu32x4 wv[2][G::PER];
+    xload(0);
+    wload(wv[0], 0);
+    wload(wv[1], 1);
+    for (int i = tid; i < G::C; i += G::NT) m128[i] = 0u;
+    xstore(0);
+    lds_barrier();
+
+    float acc[NQ][4];
+#pragma unroll
+    for (int q = 0; q < NQ; q++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[q][r] = 0.0f;
+    const int j = lane & 3, L = (lane >> 2) & 7, rg = lane >> 5;
+    const uint8_t* wq = slot + (4 * rg + j) * G::PITCH + 4 * L;   // this lane's row, dword L
+    const uint8_t* wd = slot + (4 * rg + j) * G::PITCH;
+
+    const auto step = [&](tu32x4 (&v)[G::PER], int xs, int c) {
+#pragma unroll
+        for (int k = 0; k < G::PER; k++)
+            if (k < G::PER - 1 || G::WP % 64 == 0 || lane + 64 * k < G::WP) *reinterpret_cast<tu32x4*>(slot + dst[k]) = v[k];
+        xload(min(c + 1, nch - 1));  // before the weights: loads return in order
+        wload(v, c + 2);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        const uint8_t* x = lds + xs * G::XSLOT;
+        const uint8_t* xq = x + j * 64 + 8 * L;
+        const float2* xd = reinterpret_cast<const float2*>(x + CB * G::PLANE) + j;
+        // pairs of blocks, the next pair's operands read before this one's arithmetic
+        TqOps<NQ> o[2];
+        tq_read<NQ, G::C, G::PLANE>(o[0], wq, wd, xq, xd, 0);
+        if (CB == 8 || (c + 1) * CB <= nb) {
+#pragma unroll
+            for (int t = 0; t < CB / 2; t++) {
+                if (t + 1 < CB / 2) tq_read<NQ, G::C, G::PLANE>(o[(t + 1) & 1], wq, wd, xq, xd, t + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                tq_pair<NQ>(o[t & 1], acc);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            const int npair = (nb - c * CB) / 2;
+#pragma unroll 1
+            for (int t = 0; t < npair; t++) {
+                tq_read<NQ, G::C, G::PLANE>(o[0], wq, wd, xq, xd, t);
+                tq_pair<NQ>(o[0], acc);
+            }
+        }
+        xstore(xs ^ 1);  // last read before the previous barrier
+        lds_barrier();
+    };
+    int c0 = 0;
+    for (; c0 + 1 < nch; c0 += 2) {
+        step(wv[0], 0, c0);
+        step(wv[1], 1, c0 + 1);
+    }
+    if (c0 < nch) step(wv[0], 0, c0);
+
+#pragma unroll
+    for (int u = 0; u < G::XP; u++) {
+        const int t = min(tid + u * G::NT, G::UX - 1) / (2 * CB);
+        if (bad[u] != 0) m128[t] = 1u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NQ; n++) {
+        float y[4];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            float a = acc[n][r];
+            a = a + xor_f(a, 16);
+            a = a + xor_f(a, 8);
+            y[r] = a + xor_f(a, 4);
+        }
+        const int tl = 4 * n + j, tok = n0 + tl, r0 = row0 + 4 * rg;
+        if (L != 0 || tok >= m_tokens) continue;
+        bool odd = m128[tl] != 0;
+#pragma unroll
+        for (int r = 0; r < 4; r++) odd |= __builtin_isnan(y[r]);
+        if (odd) {
+            for (int r = 0; r < 4; r++)
+                if (r0 + r < m_weight && (m128[tl] != 0 || __builtin_isnan(y[r])))
+                    y[r] = t_order_cell(W + (r0 + r) * bpr, kQ80Bytes, 2, X + tok * bpr, nb, r0 + r, tok, m_weight,
+                                        m_tokens);
+        }
+        float* o = out + (int64_t)tok * m_weight + r0;
+        if ((reinterpret_cast<uintptr_t>(o) & 15) == 0 && r0 + 4 <= m_weight) {
+            *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (r0 + r < m_weight) o[r] = y[r];
+        }
+    }
+}
+
+template <int R>
+static GemmW gemm_args(const uint8_t* const* W, float* const* out, const int* M, int n) {
+    GemmW g{};
+    int blocks = 0;
+    for (int i = 0; i < kGemmMulti; i++) {
+        const int q = i < n ? i : 0;
+        g.first[i] = blocks;
+        g.w[i] = W[q];
+        g.out[i] = out[q];
+        g.m[i] = M[q];
+        if (i < n) blocks += (M[i] + R - 1) / R;
+    }
+    g.first[kGemmMulti] = blocks;
+    return g;
+}
+
+template <int WRN, int WCN, int CT, int PF>
+static void launch_tm(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq, int m_tokens,
+                      int nb, bool aligned, hipStream_t s) {
+    using G = TmGeo<WRN, WCN, CT>;
+    const GemmW g = gemm_args<G::R>(W, out, M, n);
+    const dim3 grid(g.first[kGemmMulti] * ((m_tokens + G::C - 1) / G::C));
+    if (aligned)
+        hipLaunchKernelGGL((k_q8_0_gemm_TM<WRN, WCN, CT, PF, true>), grid, dim3(G::NT), 0, s, g, Xq, m_tokens, nb);
+    else
+        hipLaunchKernelGGL((k_q8_0_gemm_TM<WRN, WCN, CT, PF, false>), grid, dim3(G::NT), 0, s, g, Xq, m_tokens, nb);
+}
+
+template <int NQ, int NW, int CB>
+static void launch_tq(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq, int m_tokens,
+                      int nb, hipStream_t s) {
+    using G = TqGeo<NQ, NW, CB>;
+    const GemmW g = gemm_args<G::R>(W, out, M, n);
+    hipLaunchKernelGGL((k_q8_0_gemm_TQ<NQ, NW, CB>), dim3(g.first[kGemmMulti] * ((m_tokens + G::C - 1) / G::C)),
+                       dim3(G::NT), 0, s, g, Xq, m_tokens, nb);
+}
+
+// Which kernel, by the cells M * m_tokens (every one costs about the same per block,
+// so K does not enter).  Measured on MI355X at K = 4096, weights beyond the MALL, us
+// per call, the per-token GEMVs they replace in brackets:
+//   TQ   14336x2 18.9 (22.3), 14336x4 19.0 (39.7), 14336x8 26 (73), 4096x4 13.5
+//        (14.1), 4096x8 13.8 (22.7), 4096x16 17.8 (41), 4096x32 25.9 (75);
+//        1024x8 12.6 (7.5: the GEMVs stay below 16,384 cells);
+//   TM   32 rows x 64 tokens: 4096x64 45.6 (TQ 48), 4096x128 46.7 (TQ 89), 1024x512
+//        50 (304); 64 x 64: 14336x32 67 (TQ 80), 14336x64 69 (650), 4096x512 137
+//        (1,360), 14336x512 434 (4,890: 84 % of the 382 us that 16 VALU operations
+//        per cell and block take).
+// 4 tokens per wave (NQ 1) while 8 would leave SIMDs without a wave: 4096x8 13.8
+// against 17.5, 14336x8 31 against 26.
+bool launch_q8_0_gemm_T_multi(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq,
+                              int m_tokens, int K, hipStream_t s) {
+    const int nb = K / 32;
+    bool al4 = nb % 2 == 0 && (reinterpret_cast<uintptr_t>(Xq) & 3) == 0, al16 = nb % 8 == 0;
+    int64_t rows = 0;
+    for (int i = 0; i < n; i++) {
+        rows += M[i];
+        al4 = al4 && (reinterpret_cast<uintptr_t>(W[i]) & 3) == 0;
+        al16 = al16 && (reinterpret_cast<uintptr_t>(W[i]) & 15) == 0;
+    }
+    if (nb == 0 || m_tokens < 2) return false;
+    if (al16 && rows * m_tokens < 16384) return false;
+    // without 16-byte rows the few-token kernel does not apply, and the GEMVs take the
+    // dword form: 18 us per token at 14336x4096 against 46 for the smallest TM launch
+    if (!al16 && rows * m_tokens < 40960) return false;
+    const int64_t w8 = (rows + 7) / 8 * ((m_tokens + 7) / 8);  // waves of 8 rows x 8 tokens
+    if (al16 && w8 <= 4096) {
+        if (w8 < 1024)
+            launch_tq<1, 4, 16>(W, out, M, n, Xq, m_tokens, nb, s);
+        else
+            launch_tq<2, 4, 16>(W, out, M, n, Xq, m_tokens, nb, s);
+    } else if ((rows + 31) / 32 * ((m_tokens + 63) / 64) <= 256) {
+        launch_tm<2, 4, 1, 4>(W, out, M, n, Xq, m_tokens, nb, al4, s);
+    } else {
+        launch_tm<4, 4, 1, 4>(W, out, M, n, Xq, m_tokens, nb, al4, s);
+    }
+    return true;
+}
+
+}  // namespace bpdq
