@@ -90,6 +90,18 @@ void launch_q8_pad64(const float* x, uint8_t* out, int N, int K, hipStream_t s);
 void launch_q8_pad64_dispatch_T(const uint8_t* Wp, const uint8_t* Xq, float* out, int m_weight, int m_tokens, int K,
                                 hipStream_t s);
 
+// The padded layout (q8_pad.hip): up to 3 matrices of N[i] >= 1 rows sharing the activation
+// rows Xq; false (nothing launched) where the activation does not fit in LDS, or where
+// k_q8_pad64_gemv_TP is faster and ring_fits says that it can run.
+bool launch_pad_gemv(const uint8_t* const* W, float* const* y, const int* N, int n, const uint8_t* Xq, int m_tokens,
+                     int K, bool ring_fits, hipStream_t s);
+// Up to 3 matrices sharing one activation row: y[i][N[i]].
+void launch_q8_pad64_multi(const uint8_t* const* W, float* const* y, const int* N, int n, const uint8_t* Xq, int K,
+                           hipStream_t s);
+// Gate and up with SwiGLU and the Q8_0 blocks of y; false (nothing launched) if K does not fit.
+bool launch_pad_swiglu(const uint8_t* Wg, const uint8_t* Wu, float* y, uint8_t* yq, int F, const uint8_t* Xq, int K,
+                       hipStream_t s);
+
 // nan_mode: which reference form's NaN bits the NaN cells take: 0 = the scalar
 // tiles of the dispatcher, 1 = bpd_qdot_q8_0_q8_0_cpu (the scalar build's llamafile).
 void launch_q8_0_gemm_S(const uint8_t* Wq, const uint8_t* Xq, float* out, int m_weight, int m_tokens, int K,

@@ -1638,7 +1638,7 @@ bool validate(V& v, const StepOpts& o, const LayerWeights* layers, const ModelCo
 }
 
 // The GEMVs y_i[N_i] = W_i[N_i][K] a[K] of matrices that share one activation.
-// Padded Q8 reads the Q8_0 bytes aq of a.  The K-quants read a's Q8_K: xk when
+// Padded Q8 reads the Q8_0 bytes aq of a, in one launch.  The K-quants read a's Q8_K: xk when
 // the norm wrote it, else Q4_K quantizes inside the kernel (K <= fused_max_k())
 // and Q6_K (or a longer Q4_K) reads q8k, written here once per group.  Q4_K
 // matrices of one element map share a launch.
@@ -1648,8 +1648,9 @@ struct Gemv {
     void run(int n, const void* const* w, const int* fmt, float* const* y, const int* N, const float* a,
              const uint8_t* aq, const uint8_t* xk, int K) const {
         if (fmt[0] == BPDQ_W_Q8_PAD64) {
-            for (int i = 0; i < n; i++)
-                launch_q8_pad64_dispatch_T(static_cast<const uint8_t*>(w[i]), aq, y[i], N[i], 1, K, s);
+            const uint8_t* wl[3];
+            for (int i = 0; i < n; i++) wl[i] = static_cast<const uint8_t*>(w[i]);
+            launch_q8_pad64_multi(wl, y, N, n, aq, K, s);
             return;
         }
         bool need_q8k = false;
@@ -1818,6 +1819,10 @@ void run_layers(const StepCtx& c, const Gemv& gemv, const LayerWeights* layers, 
         } else if (fused && g.E <= fused_max_k()) {
             launch_qmatmul_q4k_fused_swiglu(static_cast<const uint8_t*>(w.gate), static_cast<const uint8_t*>(w.up),
                                             c.gate, g.F, c.h, g.E, format_order(f[4]), c.s);
+        } else if (f[4] == BPDQ_W_Q8_PAD64 &&
+                   launch_pad_swiglu(static_cast<const uint8_t*>(w.gate), static_cast<const uint8_t*>(w.up), c.gate,
+                                     c.xq_f, g.F, c.xq_e, g.E, c.s)) {
+            // y in gate and its Q8_0 blocks in xq_f
         } else {
             const void* wgu[2] = {w.gate, w.up};
             float* ygu[2] = {c.gate, c.up};

@@ -109,14 +109,14 @@ struct WBatch {
 // wbase: wave-uniform pointer to the wave's first row; voff: this lane's row
 // offset within the wave plus 2 + 4L (lane-constant).  Addresses are then
 // "scalar base + 32-bit lane offset + immediate", one instruction per load.
-template <int U, int LAYOUT>
+template <int U>
 __device__ __forceinline__ void load_batch(WBatch<U>& w, const uint8_t* __restrict__ wbase, uint32_t voff,
-                                           uint32_t doff, int b0, int nb, int64_t bstride) {
+                                           uint32_t doff, int b0, int nb) {
     // Blocks past the end of the row repeat block nb-1 (their steps are skipped).
     // The clamp is wave-uniform, so each address stays scalar base + lane offset.
 #pragma unroll
     for (int u = 0; u < U; u++) {
-        const uint8_t* bu = wbase + (int64_t)min(b0 + u, nb - 1) * (LAYOUT == 0 ? (int64_t)kQ80Bytes : bstride);
+        const uint8_t* bu = wbase + (int64_t)min(b0 + u, nb - 1) * kQ80Bytes;
         w.q[u] = ld_u32(bu + voff);
         w.d[u] = ld_u16(bu + doff);
     }
@@ -172,11 +172,7 @@ __device__ __forceinline__ uint32_t stage_x(uint32_t* __restrict__ xs, float* __
     return any_m128;
 }
 
-// LAYOUT 0: W is rows of 34-byte Q8_0 blocks.  LAYOUT 1: W is the padded
-// block-major layout of inference/llamatov_c_inference.py:88-100, records of 64
-// bytes [block][row] with d at bytes 0-1 and the quants at 4-35; the cells and
-// their order are the same.
-template <int U, int WPB, int LAYOUT = 0>
+template <int U, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_q8_0_gemv_T(const uint8_t* __restrict__ W, const uint8_t* __restrict__ Xq,
                                                           float* __restrict__ out, int m_weight, int nb) {
     extern __shared__ uint32_t lds[];
@@ -188,26 +184,25 @@ __global__ __launch_bounds__(64 * WPB) void k_q8_0_gemv_T(const uint8_t* __restr
     const int row = (blockIdx.x * WPB + wave) * 8 + (lane >> 3);
     const int tok = blockIdx.y;
     const int64_t bpr = (int64_t)nb * kQ80Bytes;
-    const int64_t wrow = LAYOUT == 0 ? bpr : 64, bstride = LAYOUT == 0 ? kQ80Bytes : (int64_t)m_weight * 64;
     // A wave past the last row (the workgroup's spare waves) reads row m_weight-1;
     // base and lane offsets are clamped so every address stays inside W.
     const int row0 = min((blockIdx.x * WPB + wave) * 8, m_weight - 1);
-    const uint8_t* wbase = W + (int64_t)row0 * wrow;
-    const uint32_t doff = (uint32_t)((max(min(row, m_weight - 1), row0) - row0) * wrow);
-    const uint32_t voff = doff + (LAYOUT == 0 ? 2 : 4) + 4 * L;
+    const uint8_t* wbase = W + (int64_t)row0 * bpr;
+    const uint32_t doff = (uint32_t)((max(min(row, m_weight - 1), row0) - row0) * bpr);
+    const uint32_t voff = doff + 2 + 4 * L;
 
     __shared__ uint32_t wave_m128[WPB];
     WBatch<U> a, b;
-    load_batch<U, LAYOUT>(a, wbase, voff, doff, 0, nb, bstride);
+    load_batch<U>(a, wbase, voff, doff, 0, nb);
     note_m128(wave_m128, stage_x<64 * WPB>(xs, xd, Xq + (int64_t)tok * bpr, nb));
     __syncthreads();
     const bool xm128 = __builtin_amdgcn_readfirstlane((int)row_m128(wave_m128, WPB)) != 0;
 
     float acc = 0.0f;
     for (int b0 = 0; b0 < nb; b0 += 2 * U) {
-        if (b0 + U < nb) load_batch<U, LAYOUT>(b, wbase, voff, doff, b0 + U, nb, bstride);
+        if (b0 + U < nb) load_batch<U>(b, wbase, voff, doff, b0 + U, nb);
         acc = accumulate_batch<U>(a, xs, xd, L, b0, nb, acc);
-        if (b0 + 2 * U < nb) load_batch<U, LAYOUT>(a, wbase, voff, doff, b0 + 2 * U, nb, bstride);
+        if (b0 + 2 * U < nb) load_batch<U>(a, wbase, voff, doff, b0 + 2 * U, nb);
         acc = accumulate_batch<U>(b, xs, xd, L, b0 + U, nb, acc);
     }
     acc = acc + xor_f(acc, 4);
@@ -215,8 +210,8 @@ __global__ __launch_bounds__(64 * WPB) void k_q8_0_gemv_T(const uint8_t* __restr
     acc = acc + xor_f(acc, 1);
     if (L == 0 && row < m_weight) {
         if (__builtin_isnan(acc) || xm128)
-            acc = t_order_cell(W + (int64_t)row * wrow, bstride, LAYOUT == 0 ? 2 : 4, Xq + (int64_t)tok * bpr, nb,
-                               row, tok, m_weight, (int)gridDim.y);
+            acc = t_order_cell(W + (int64_t)row * bpr, kQ80Bytes, 2, Xq + (int64_t)tok * bpr, nb, row, tok, m_weight,
+                               (int)gridDim.y);
         out[(int64_t)tok * m_weight + row] = acc;
     }
 }
@@ -323,13 +318,13 @@ __device__ __forceinline__ void tp_step(TpLoad (&regs)[kTpAhead], const TpLane& 
 }
 
 template <int LAYOUT>
-__global__ __launch_bounds__(320) void k_q8_0_gemv_TP(const uint8_t* __restrict__ W, const uint8_t* __restrict__ Xq,
-                                                       float* __restrict__ out, int m_weight, int nb) {
+__device__ __forceinline__ void tp_gemv(const uint8_t* __restrict__ W, const uint8_t* __restrict__ Xq,
+                                        float* __restrict__ out, int m_weight, int nb, int bx) {
     extern __shared__ uint32_t lds[];
     uint32_t* xs = lds;                                   // [nb][8] activation quants
     float* xd = reinterpret_cast<float*>(lds + nb * 8);   // [nb] activation scales
     __shared__ __align__(16) float prod[2][64 * kTpLd];
-    const int tid = threadIdx.x, tok = blockIdx.y, row0 = blockIdx.x * 8;
+    const int tid = threadIdx.x, tok = blockIdx.y, row0 = bx * 8;
     const bool producer = tid >= 64;
     const int pp = producer ? tid - 64 : 0;
     TpLane p;
@@ -385,6 +380,17 @@ __global__ __launch_bounds__(320) void k_q8_0_gemv_TP(const uint8_t* __restrict_
             out[(int64_t)tok * m_weight + orow] = acc;
         }
     }
+}
+
+__global__ __launch_bounds__(320) void k_q8_0_gemv_TP(const uint8_t* __restrict__ W, const uint8_t* __restrict__ Xq,
+                                                      float* __restrict__ out, int m_weight, int nb) {
+    tp_gemv<0>(W, Xq, out, m_weight, nb, blockIdx.x);
+}
+
+// The padded layout; up to 3 matrices that share the activation (a decode step's Q, K and V).
+__global__ __launch_bounds__(320) void k_q8_pad64_gemv_TP(GemmW gw, const uint8_t* __restrict__ Xq, int nb) {
+    const int bx = blockIdx.x, mi = (bx >= gw.first[1]) + (bx >= gw.first[2]);
+    tp_gemv<1>(gw.w[mi], Xq, gw.out[mi], gw.m[mi], nb, bx - gw.first[mi]);
 }
 
 // ----------------------------------------------------------------------------
@@ -701,21 +707,19 @@ static bool launch_wide(const uint8_t* Wq, const uint8_t* Xq, float* out, int m_
     return true;
 }
 
-template <int LAYOUT>
-static void dispatch_T(const uint8_t* Wq, const uint8_t* Xq, float* out, int m_weight, int m_tokens, int K,
-                       hipStream_t s) {
+void launch_q8_0_dispatch_T(const uint8_t* Wq, const uint8_t* Xq, float* out, int m_weight, int m_tokens, int K,
+                            hipStream_t s) {
     const int nb = K / 32;
     if (nb == 0) {  // the kernels below index block nb-1
         launch_fill_zero(out, (int64_t)m_weight * m_tokens, s);
         return;
     }
-    if (LAYOUT == 0 && launch_q8_0_gemm_T_multi(&Wq, &out, &m_weight, 1, Xq, m_tokens, K, s)) return;
-    if (LAYOUT == 0 && launch_wide(Wq, Xq, out, m_weight, m_tokens, nb, s)) return;
+    if (launch_q8_0_gemm_T_multi(&Wq, &out, &m_weight, 1, Xq, m_tokens, K, s)) return;
+    if (launch_wide(Wq, Xq, out, m_weight, m_tokens, nb, s)) return;
     const int waves = (m_weight + 7) / 8;
     const size_t lds = (size_t)nb * 36;
     if (lds > 64 * 1024) {
-        hipLaunchKernelGGL(k_q8_0_gemm_T<LAYOUT>, dim3((waves + 3) / 4, m_tokens), dim3(256), 0, s, Wq, Xq, out,
-                           m_weight, nb);
+        hipLaunchKernelGGL(k_q8_0_gemm_T<0>, dim3((waves + 3) / 4, m_tokens), dim3(256), 0, s, Wq, Xq, out, m_weight, nb);
         return;
     }
     // shapes measured on MI355X (graph, weights beyond the MALL): with many waves
@@ -724,24 +728,57 @@ static void dispatch_T(const uint8_t* Wq, const uint8_t* Xq, float* out, int m_w
     // waves the producer/consumer kernel (4096x14336: 24.2 us vs 38.4 for 32-block
     // batches; 4096x4096: 9.2 vs 13.0; 1024x4096: 6.7 vs 12.5)
     if (waves * m_tokens >= 1024)
-        hipLaunchKernelGGL((k_q8_0_gemv_T<16, 4, LAYOUT>), dim3((waves + 3) / 4, m_tokens), dim3(256), lds, s, Wq, Xq,
-                           out, m_weight, nb);
-    else if (lds + sizeof(float) * 2 * 64 * kTpLd <= 64 * 1024)
-        hipLaunchKernelGGL((k_q8_0_gemv_TP<LAYOUT>), dim3((m_weight + 7) / 8, m_tokens), dim3(320), lds, s, Wq, Xq, out,
+        hipLaunchKernelGGL((k_q8_0_gemv_T<16, 4>), dim3((waves + 3) / 4, m_tokens), dim3(256), lds, s, Wq, Xq, out,
                            m_weight, nb);
+    else if (lds + sizeof(float) * 2 * 64 * kTpLd <= 64 * 1024)
+        hipLaunchKernelGGL(k_q8_0_gemv_TP, dim3((m_weight + 7) / 8, m_tokens), dim3(320), lds, s, Wq, Xq, out, m_weight,
+                           nb);
     else
-        hipLaunchKernelGGL((k_q8_0_gemv_T<32, 2, LAYOUT>), dim3((waves + 1) / 2, m_tokens), dim3(128), lds, s, Wq,
-                           Xq, out, m_weight, nb);
+        hipLaunchKernelGGL((k_q8_0_gemv_T<32, 2>), dim3((waves + 1) / 2, m_tokens), dim3(128), lds, s, Wq, Xq, out,
+                           m_weight, nb);
 }
 
-void launch_q8_0_dispatch_T(const uint8_t* Wq, const uint8_t* Xq, float* out, int m_weight, int m_tokens, int K,
-                            hipStream_t s) {
-    dispatch_T<0>(Wq, Xq, out, m_weight, m_tokens, K, s);
+// The padded layout: m_tokens rows of Xq, or (m_tokens == 1) up to 3 matrices in one launch.
+// Few rows take the producer/consumer kernel while its ring and the activation fit in 64 KB of
+// LDS, the rest launch_pad_gemv; k_q8_0_gemm_T where the activation does not fit in LDS at all.
+static void pad64_T(const uint8_t* const* W, float* const* out, const int* N, int n, const uint8_t* Xq, int m_tokens,
+                    int K, hipStream_t s) {
+    const int nb = K / 32;
+    const size_t lds = (size_t)nb * 36;
+    const bool ring = lds + sizeof(float) * 2 * 64 * kTpLd <= 64 * 1024;
+    if (nb > 0 && launch_pad_gemv(W, out, N, n, Xq, m_tokens, K, ring, s)) return;
+    if (nb > 0 && ring) {
+        GemmW g{};
+        int blocks = 0;
+        for (int i = 0; i < kGemmMulti; i++) {
+            const int q = i < n ? i : 0;
+            g.w[i] = W[q];
+            g.out[i] = out[q];
+            g.m[i] = N[q];
+            g.first[i] = blocks;
+            if (i < n) blocks += (N[i] + 7) / 8;
+        }
+        g.first[kGemmMulti] = blocks;
+        hipLaunchKernelGGL(k_q8_pad64_gemv_TP, dim3(blocks, m_tokens), dim3(320), lds, s, g, Xq, nb);
+        return;
+    }
+    for (int i = 0; i < n; i++) {
+        if (nb == 0)
+            launch_fill_zero(out[i], (int64_t)N[i] * m_tokens, s);
+        else
+            hipLaunchKernelGGL(k_q8_0_gemm_T<1>, dim3((N[i] + 31) / 32, m_tokens), dim3(256), 0, s, W[i], Xq, out[i],
+                               N[i], nb);
+    }
 }
 
 void launch_q8_pad64_dispatch_T(const uint8_t* Wp, const uint8_t* Xq, float* out, int m_weight, int m_tokens, int K,
                                 hipStream_t s) {
-    dispatch_T<1>(Wp, Xq, out, m_weight, m_tokens, K, s);
+    pad64_T(&Wp, &out, &m_weight, 1, Xq, m_tokens, K, s);
+}
+
+void launch_q8_pad64_multi(const uint8_t* const* W, float* const* y, const int* N, int n, const uint8_t* Xq, int K,
+                           hipStream_t s) {
+    pad64_T(W, y, N, n, Xq, 1, K, s);
 }
 
 // ----------------------------------------------------------------------------

@@ -4,9 +4,10 @@ bit for bit against the Q8_0 dispatcher on the same blocks."""
 import numpy as np
 import pytest
 
-from bpd_substrate_amd import gpu, synth
+from bpd_substrate_amd import formats, gpu, synth
 from helpers import assert_bits_equal, special_f32_blocks, to_np
 from oracle import oracle as O
+from test_gpu_q8_0 import _q8_full_range, _q8_nan_heavy
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +55,18 @@ def test_pad64_product_equals_q8_0_dispatch(dev, mw, mt, K):
     assert np.array_equal(got.view(np.uint32), ref_gpu.view(np.uint32))
     if mw * K <= 4096 * 4096:
         assert_bits_equal(got, O.dispatch_q8_0(rows, to_np(xq), mw, mt, K, "T", nthreads=8), f"pad64 {mw}x{K}")
+
+
+# q8_pad.hip's kernel at its edges: fewer blocks than it keeps in flight, a ragged last group,
+# rows that end inside a workgroup, both workgroup shapes, several tokens, an activation over
+# 64 KB of LDS and one that does not fit at all
+@pytest.mark.parametrize("mw,mt,K", [(3079, 1, 96), (3088, 1, 1056), (12300, 1, 352), (41, 77, 160), (37, 1, 45056),
+                                     (3, 2, 81920)])
+@pytest.mark.parametrize("kind", ["plain", "nan", "int8"])
+def test_pad64_product_edges(dev, mw, mt, K, kind):
+    nb = K // 32
+    make = {"plain": lambda r, k: synth.q8_0(r, K, k), "nan": lambda r, k: _q8_nan_heavy(r, nb, k),
+            "int8": lambda r, k: _q8_full_range(r, nb, k)}[kind]
+    W, X = make(mw, synth.key(83, mw)), make(mt, synth.key(84, mt))
+    got = to_np(gpu.qmatmul_q8_pad64(_d(formats.q8_0_rows_to_pad64(W, mw, K), dev), _d(X, dev), mw, mt, K))
+    assert_bits_equal(got, O.dispatch_q8_0(W, X, mw, mt, K, "T", nthreads=8), f"pad64 {kind} {mw}x{mt}x{K}")
