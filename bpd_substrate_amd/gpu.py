@@ -17,7 +17,7 @@ point raises.
 import ctypes
 
 from . import formats
-from ._native import load_hip
+from ._native import HIP_SIGNATURES, load_hip
 
 
 class BpdqError(RuntimeError):
@@ -42,25 +42,34 @@ def _ptr(a):
     raise TypeError(f"cannot pass {type(a).__name__} as a device pointer")
 
 
+# Entry points bound once per process (name -> ctypes function).  A decode-time GEMV is 3-7 us of
+# GPU work, so what a call does in Python sets its rate: a lookup of every name, an import per call
+# and a torch.cuda.Stream object (2.7 us) made the helpers 4.8 us slower than the bare ctypes call.
+_fns = {}
+
+
+def _fn(name):
+    fn = _fns.get(name)
+    if fn is None:
+        if name not in HIP_SIGNATURES:
+            raise KeyError(f"{name} has no ctypes signature in _native.HIP_SIGNATURES")
+        fn = _fns[name] = getattr(lib(), name)
+    return fn
+
+
 def check():
     """Raise BpdqError if the last call on this thread recorded an error."""
-    L = lib()
-    code = L.bpd_gpu_last_error()
+    code = _fn("bpd_gpu_last_error")()
     if code:
-        raise BpdqError(code, L.bpd_gpu_last_error_message().decode())
+        raise BpdqError(code, _fn("bpd_gpu_last_error_message")().decode())
 
 
 def call(name, *args):
     """Call an exported entry point by name; pointers may be tensors.  Only names with a
     declared ctypes signature are callable: without one, ctypes would pass each Python
     int as a 32-bit C int and cut 64-bit device pointers short."""
-    from ._native import HIP_SIGNATURES
-
-    if name not in HIP_SIGNATURES:
-        raise KeyError(f"{name} has no ctypes signature in _native.HIP_SIGNATURES")
-    fn = getattr(lib(), name)
-    conv = [_ptr(a) if not isinstance(a, (float,)) else a for a in args]
-    res = fn(*conv)
+    fn = _fn(name)
+    res = fn(*[a if isinstance(a, (int, float)) else _ptr(a) for a in args])
     check()
     return res
 
@@ -75,9 +84,8 @@ def _need(t, nbytes, what):
         return
     if not t.is_contiguous():
         raise BpdqError(BPDQ_ERR_SHAPE, f"{what} is not contiguous")
-    have = t.numel() * t.element_size()
-    if have < nbytes:
-        raise BpdqError(BPDQ_ERR_SHAPE, f"{what} holds {have} bytes, the call needs {nbytes}")
+    if t.nbytes < nbytes:
+        raise BpdqError(BPDQ_ERR_SHAPE, f"{what} holds {t.nbytes} bytes, the call needs {nbytes}")
 
 
 def _q4k_bytes(M, K):
@@ -93,25 +101,24 @@ def _q8_0_bytes(rows, K):
 
 
 def _use_torch_stream():
+    """Launch on torch's current stream (its handle, without the Stream object around it)."""
     import torch
 
-    lib().bpd_gpu_set_stream(torch.cuda.current_stream().cuda_stream)
+    _fn("bpd_gpu_set_stream")(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def _empty(n, dtype, like):
     import torch
 
-    return torch.empty(n, dtype=dtype, device=like.device)
+    return torch.empty(n, dtype=getattr(torch, dtype), device=like.device)
 
 
 # ---------------------------------------------------------------- Q4_K / Q8_K
 
 def dequant_q4k(q, order=formats.ORDER_BPD, out=None):
     """q: uint8 device tensor of n_blocks*144 bytes -> fp32 tensor [n_blocks*256]."""
-    import torch
-
     nb = q.numel() // formats.Q4K_BYTES
-    out = _empty(nb * 256, torch.float32, q) if out is None else out
+    out = _empty(nb * 256, "float32", q) if out is None else out
     _need(out, nb * 256 * 4, "out")
     _use_torch_stream()
     call("bpd_dequant_q4k_gpu" if order == formats.ORDER_BPD else "bpd_dequant_q4k_gguf_gpu", q, out, nb)
@@ -120,9 +127,7 @@ def dequant_q4k(q, order=formats.ORDER_BPD, out=None):
 
 def qmatmul_q4k(w, x, M, K, out=None):
     """Reference-order GEMV, fp32 x (bit-identical to bpd_qmatmul_q4k)."""
-    import torch
-
-    out = _empty(M, torch.float32, x) if out is None else out
+    out = _empty(M, "float32", x) if out is None else out
     _need(w, _q4k_bytes(M, K), "w")
     _need(x, max(K, 0) * 4, "x")
     _need(out, max(M, 0) * 4, "out")
@@ -132,10 +137,8 @@ def qmatmul_q4k(w, x, M, K, out=None):
 
 
 def quant_q8_k(x, out=None):
-    import torch
-
     n = x.numel()
-    out = _empty(n // formats.Q8K_ELEMS * formats.Q8K_BYTES, torch.uint8, x) if out is None else out
+    out = _empty(n // formats.Q8K_ELEMS * formats.Q8K_BYTES, "uint8", x) if out is None else out
     _need(out, _q8k_bytes(n), "out")
     _use_torch_stream()
     call("bpd_quant_q8_k_gpu", x, out, n)
@@ -143,9 +146,7 @@ def quant_q8_k(x, out=None):
 
 
 def qmatmul_q4k_q8k(w, xq, M, K, order=formats.ORDER_BPD, out=None):
-    import torch
-
-    out = _empty(M, torch.float32, xq) if out is None else out
+    out = _empty(M, "float32", xq) if out is None else out
     _need(w, _q4k_bytes(M, K), "w")
     _need(xq, _q8k_bytes(K), "xq")
     _need(out, max(M, 0) * 4, "out")
@@ -162,9 +163,7 @@ def qmatmul_q4k_q8k_multi(ws, xq, Ms, K, outs=None):
 
 def qmatmul_q4k_q8k_fused(w, x, M, K, out=None):
     """Q4_K x Q8_K(x) for fp32 x, quantized inside the GEMV kernel (bits equal quant + GEMV)."""
-    import torch
-
-    out = _empty(M, torch.float32, x) if out is None else out
+    out = _empty(M, "float32", x) if out is None else out
     _need(w, _q4k_bytes(M, K), "w")
     _need(x, max(K, 0) * 4, "x")
     _need(out, max(M, 0) * 4, "out")
@@ -179,10 +178,8 @@ def qmatmul_q4k_q8k_fused_multi(ws, x, Ms, K, outs=None):
 
 
 def _multi(name, ws, x, Ms, K, outs):
-    import torch
-
     n = len(ws)
-    outs = [_empty(m, torch.float32, x) for m in Ms] if outs is None else outs
+    outs = [_empty(m, "float32", x) for m in Ms] if outs is None else outs
     for i in range(n):
         _need(ws[i], _q4k_bytes(Ms[i], K), f"w[{i}]")
         _need(outs[i], max(Ms[i], 0) * 4, f"out[{i}]")
@@ -200,9 +197,7 @@ def _multi(name, ws, x, Ms, K, outs):
 def q8_pad64(x, N, K, out=None):
     """fp32 [N, K] -> uint8 [K/32 * N * 64] in the layout of q8_pad64_coalesced
     (inference/llamatov_c_inference.py:88-100)."""
-    import torch
-
-    out = _empty(K // 32 * N * 64, torch.uint8, x) if out is None else out
+    out = _empty(K // 32 * N * 64, "uint8", x) if out is None else out
     _need(x, max(N, 0) * max(K, 0) * 4, "x")
     _need(out, max(K, 0) // 32 * max(N, 0) * 64, "out")
     _use_torch_stream()
@@ -211,9 +206,7 @@ def q8_pad64(x, N, K, out=None):
 
 
 def qmatmul_q8_pad64(Wp, Xq, m_weight, m_tokens, K, out=None):
-    import torch
-
-    out = _empty(m_tokens * m_weight, torch.float32, Xq) if out is None else out
+    out = _empty(m_tokens * m_weight, "float32", Xq) if out is None else out
     _need(Wp, max(K, 0) // 32 * max(m_weight, 0) * 64, "W_pad64")
     _need(Xq, _q8_0_bytes(m_tokens, K), "Xq")
     _need(out, max(m_tokens * m_weight, 0) * 4, "out")
@@ -232,12 +225,10 @@ GGUF_PY_BLOCKS = {0: (1, 4), 1: (1, 2), 2: (32, 18), 10: (256, 84), 11: (256, 11
 def dequant_gguf_py(raw, n_elements, ggml_type, out=None):
     """raw: uint8 device tensor of a GGUF tensor's bytes -> fp32 [n_elements] with the
     reference Python loader's formula for ggml_type (bpd_dequant_gguf_py_gpu)."""
-    import torch
-
     if ggml_type not in GGUF_PY_BLOCKS:
         raise ValueError(f"ggml_type {ggml_type} has no loader formula")
     per, size = GGUF_PY_BLOCKS[ggml_type]
-    out = _empty(n_elements, torch.float32, raw) if out is None else out
+    out = _empty(n_elements, "float32", raw) if out is None else out
     _need(raw, n_elements // per * size, "raw")
     _need(out, n_elements * 4, "out")
     _use_torch_stream()
@@ -250,10 +241,8 @@ def dequant_gguf_py(raw, n_elements, ggml_type, out=None):
 def dequant_q6k(q, order=formats.ORDER_BPD, out=None):
     """q: uint8 device tensor of n_blocks*210 bytes -> fp32 [n_blocks*256].  ORDER_BPD is the
     reference's map (inference/llamatov_helpers.py:161-179), ORDER_GGUF llama.cpp's."""
-    import torch
-
     nb = q.numel() // 210
-    out = _empty(nb * 256, torch.float32, q) if out is None else out
+    out = _empty(nb * 256, "float32", q) if out is None else out
     _need(out, nb * 256 * 4, "out")
     _use_torch_stream()
     call("bpd_dequant_q6k_gpu" if order == formats.ORDER_BPD else "bpd_dequant_q6k_gguf_gpu", q, out, nb)
@@ -261,9 +250,7 @@ def dequant_q6k(q, order=formats.ORDER_BPD, out=None):
 
 
 def qmatmul_q6k_q8k(w, xq, M, K, order=formats.ORDER_BPD, out=None):
-    import torch
-
-    out = _empty(M, torch.float32, xq) if out is None else out
+    out = _empty(M, "float32", xq) if out is None else out
     _need(w, max(M, 0) * max(K, 0) // 256 * 210, "w")
     _need(xq, _q8k_bytes(K), "xq")
     _need(out, max(M, 0) * 4, "out")
@@ -276,10 +263,8 @@ def qmatmul_q6k_q8k(w, xq, M, K, order=formats.ORDER_BPD, out=None):
 # ---------------------------------------------------------------- Q8_0
 
 def dequant_q8_0(raw, out=None):
-    import torch
-
     nb = raw.numel() // formats.Q8_0_BYTES
-    out = _empty(nb * 32, torch.float32, raw) if out is None else out
+    out = _empty(nb * 32, "float32", raw) if out is None else out
     _need(out, nb * 32 * 4, "out")
     _use_torch_stream()
     call("bpd_dequant_q8_0_gpu", raw, out, nb)
@@ -287,10 +272,8 @@ def dequant_q8_0(raw, out=None):
 
 
 def embed_lookup_q8_0(table, ids, embed_dim, out=None):
-    import torch
-
     n = ids.numel()
-    out = _empty(n * embed_dim, torch.float32, table) if out is None else out
+    out = _empty(n * embed_dim, "float32", table) if out is None else out
     _need(table, _q8_0_bytes(1, embed_dim), "table")   # ids index rows on the device: 0 <= id < rows
     _need(out, n * max(embed_dim, 0) * 4, "out")
     _use_torch_stream()
@@ -299,10 +282,8 @@ def embed_lookup_q8_0(table, ids, embed_dim, out=None):
 
 
 def quant_q8_0(x, out=None):
-    import torch
-
     n = x.numel()
-    out = _empty(n // 32 * 34, torch.uint8, x) if out is None else out
+    out = _empty(n // 32 * 34, "uint8", x) if out is None else out
     _need(out, n // 32 * 34, "out")
     _use_torch_stream()
     call("bpd_quant_q8_0_gpu", x, out, n)
@@ -311,9 +292,7 @@ def quant_q8_0(x, out=None):
 
 def qmatmul_q8_0_dispatch(Wq, Xq, m_weight, m_tokens, K, out=None):
     """out[token * m_weight + row] in the AVX1 llamafile tile order."""
-    import torch
-
-    out = _empty(m_tokens * m_weight, torch.float32, Wq) if out is None else out
+    out = _empty(m_tokens * m_weight, "float32", Wq) if out is None else out
     _need(Wq, _q8_0_bytes(m_weight, K), "Wq")
     _need(Xq, _q8_0_bytes(m_tokens, K), "Xq")
     _need(out, max(m_tokens * m_weight, 0) * 4, "out")
@@ -323,9 +302,7 @@ def qmatmul_q8_0_dispatch(Wq, Xq, m_weight, m_tokens, K, out=None):
 
 
 def qmatmul_q8_0_llamafile(W, X, m_weight, m_tokens, K, out=None):
-    import torch
-
-    out = _empty(m_tokens * m_weight, torch.float32, W) if out is None else out
+    out = _empty(m_tokens * m_weight, "float32", W) if out is None else out
     _need(W, _q8_0_bytes(m_weight, K), "W")
     _need(X, max(m_tokens, 0) * max(K, 0) * 4, "X")
     _need(out, max(m_tokens * m_weight, 0) * 4, "out")
@@ -336,9 +313,7 @@ def qmatmul_q8_0_llamafile(W, X, m_weight, m_tokens, K, out=None):
 
 def qmatmul_q8_0_dispatch_s(Wq, Xq, m_weight, m_tokens, K, out=None):
     """out[token * m_weight + row] in the scalar order S (int8 MFMA prefill GEMM)."""
-    import torch
-
-    out = _empty(m_tokens * m_weight, torch.float32, Wq) if out is None else out
+    out = _empty(m_tokens * m_weight, "float32", Wq) if out is None else out
     _need(Wq, _q8_0_bytes(m_weight, K), "Wq")
     _need(Xq, _q8_0_bytes(m_tokens, K), "Xq")
     _need(out, max(m_tokens * m_weight, 0) * 4, "out")
@@ -348,9 +323,7 @@ def qmatmul_q8_0_dispatch_s(Wq, Xq, m_weight, m_tokens, K, out=None):
 
 
 def qmatmul_q8_0_llamafile_s(W, X, m_weight, m_tokens, K, out=None):
-    import torch
-
-    out = _empty(m_tokens * m_weight, torch.float32, W) if out is None else out
+    out = _empty(m_tokens * m_weight, "float32", W) if out is None else out
     _need(W, _q8_0_bytes(m_weight, K), "W")
     _need(X, max(m_tokens, 0) * max(K, 0) * 4, "X")
     _need(out, max(m_tokens * m_weight, 0) * 4, "out")
