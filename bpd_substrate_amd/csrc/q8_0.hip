@@ -320,7 +320,7 @@ __device__ __forceinline__ void tp_step(TpLoad (&regs)[kTpAhead], const TpLane& 
 template <int LAYOUT>
 __device__ __forceinline__ void tp_gemv(const uint8_t* __restrict__ W, const uint8_t* __restrict__ Xq,
                                         float* __restrict__ out, int m_weight, int nb, int bx) {
-    extern __shared__ uint32_t lds[];
+    extern __shared__ __align__(16) uint32_t lds[];
     uint32_t* xs = lds;                                   // [nb][8] activation quants
     float* xd = reinterpret_cast<float*>(lds + nb * 8);   // [nb] activation scales
     __shared__ __align__(16) float prod[2][64 * kTpLd];
