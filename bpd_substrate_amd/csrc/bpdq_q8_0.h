@@ -1,4 +1,4 @@
-// bpdq_q8_0.h — device helpers shared by the Q8_0 product kernels (q8_0.hip, q8_0_t.hip).
+// bpdq_q8_0.h — device helpers shared by the Q8_0 product kernels (q8_0.hip, q8_0_t.hip, q8_0_s.hip).
 #pragma once
 #include "bpdq_device.h"
 
@@ -97,6 +97,23 @@ struct GemmW {
     uint8_t* yq;                // SwiGLU pairs: Q8_0 rows of y = silu(gate) * up, m[0] / 32 blocks per token
 };
 
+// The launch arguments of n <= kGemmMulti matrices in row blocks of R.
+template <int R>
+static GemmW gemm_args(const uint8_t* const* W, float* const* out, const int* M, int n) {
+    GemmW g{};
+    int blocks = 0;
+    for (int i = 0; i < kGemmMulti; i++) {
+        const int q = i < n ? i : 0;
+        g.first[i] = blocks;
+        g.w[i] = W[q];
+        g.out[i] = out[q];
+        g.m[i] = M[q];
+        if (i < n) blocks += (M[i] + R - 1) / R;
+    }
+    g.first[kGemmMulti] = blocks;
+    return g;
+}
+
 // Workgroup b of nP * nT (row panels x token tiles) takes panel bx, token tile
 // by.  Workgroups go to the 8 XCDs round robin (b % 8), each with its own L2:
 // when nP divides into 8, panel p runs on XCD p % 8 and its nT token tiles are
@@ -113,6 +130,58 @@ __device__ __forceinline__ void sh_tile(int b, int nP, int nT, int& bx, int& by)
         bx = b % nP;
         by = b / nP;
     }
+}
+
+// ----------------------------------------------------------------------------
+// NaN cells of the scalar order S.  The reference computes
+//   acc = acc + float(S_b) * (Ad*Bd)   over blocks b in order
+// on x86, where the first NaN of the chain sticks (acc + p keeps acc's NaN), a
+// NaN factor comes out quieted (the first operand's when both are NaN) and
+// Inf*0, Inf-Inf give the default NaN.  Two reference forms differ in their NaN
+// bits:
+//   kSNanTile (the scalar tiles, bench/bpd_gemm_q8_0_cpu.c:112-128): scales by
+//     the ldexpf decode of :13-26 (an f16 NaN becomes +/-0x7FC00000, no payload);
+//     the build puts Bd first in Ad*Bd;
+//   kSNanQdot (bpd_qdot_q8_0_q8_0_cpu's scalar form, bench/bpd_cpu.c:4263-4280,
+//     which the scalar build's llamafile entry uses): the magic-number decode
+//     (payload kept); the weight scale first.
+// A finite scale product keeps a finite accumulator finite (|S_b*Ad*Bd| < 2^51)
+// and an infinite one unchanged, so only blocks with an Inf or NaN scale can
+// change the state, and the first NaN event fixes the bits.  Called only for a
+// cell whose sum came out NaN; NaN-ness itself is the same on every IEEE machine.
+// ----------------------------------------------------------------------------
+constexpr int kSNanTile = 0;
+constexpr int kSNanQdot = 1;
+static_assert(kSNanTile != kSNanQdot, "the two NaN forms");
+
+__device__ __forceinline__ float f16_ref(uint32_t h, int mode) {
+    if (!f16_is_nan(h)) return f16_ieee(h);
+    return mode == kSNanTile ? __uint_as_float(((h & 0x8000u) << 16) | 0x7FC00000u) : f16_nan_x86(h);
+}
+
+__device__ __noinline__ inline float s_order_nan_bits(const uint8_t* __restrict__ wrow,
+                                                      const uint8_t* __restrict__ xrow, int nb, int mode) {
+    float acc = 0.0f;  // stands for any finite value
+    for (int b = 0; b < nb; b++) {
+        const uint8_t* wb = wrow + (int64_t)b * kQ80Bytes;
+        const uint8_t* xb = xrow + (int64_t)b * kQ80Bytes;
+        const uint32_t hw = (uint32_t)wb[0] | ((uint32_t)wb[1] << 8);
+        const uint32_t hx = (uint32_t)xb[0] | ((uint32_t)xb[1] << 8);
+        if (!f16_exp31(hw) && !f16_exp31(hx)) continue;
+        const float fw = f16_ref(hw, mode), fx = f16_ref(hx, mode);
+        const float first = mode == kSNanTile ? fx : fw, second = mode == kSNanTile ? fw : fx;
+        const float delta = first * second;
+        // a NaN product: p = float(S_b) * delta is delta's NaN, and acc + p is p's
+        if (__builtin_isnan(delta)) return x86_nan_of(first, second);
+        // delta is +/-Inf: p = +/-Inf, or the default NaN when S_b = 0
+        int sumi = 0;
+        for (int j = 0; j < 32; j++) sumi += (int)(int8_t)wb[2 + j] * (int)(int8_t)xb[2 + j];
+        if (sumi == 0) return __uint_as_float(kX86NaN);
+        const float p = sumi < 0 ? -delta : delta;
+        if (__builtin_isinf(acc) && acc != p) return __uint_as_float(kX86NaN);  // Inf - Inf
+        acc = p;
+    }
+    return acc;
 }
 
 }  // namespace bpdq

@@ -850,58 +850,6 @@ typedef int i32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 h16x8 __attribute__((ext_vector_type(8)));
 
-// ----------------------------------------------------------------------------
-// NaN cells of the scalar order S.  The reference computes
-//   acc = acc + float(S_b) * (Ad*Bd)   over blocks b in order
-// on x86, where the first NaN of the chain sticks (acc + p keeps acc's NaN), a
-// NaN factor comes out quieted (the first operand's when both are NaN) and
-// Inf*0, Inf-Inf give the default NaN.  Two reference forms differ in their NaN
-// bits:
-//   kSNanTile (the scalar tiles, bench/bpd_gemm_q8_0_cpu.c:112-128): scales by
-//     the ldexpf decode of :13-26 (an f16 NaN becomes +/-0x7FC00000, no payload);
-//     the build puts Bd first in Ad*Bd;
-//   kSNanQdot (bpd_qdot_q8_0_q8_0_cpu's scalar form, bench/bpd_cpu.c:4263-4280,
-//     which the scalar build's llamafile entry uses): the magic-number decode
-//     (payload kept); the weight scale first.
-// A finite scale product keeps a finite accumulator finite (|S_b*Ad*Bd| < 2^51)
-// and an infinite one unchanged, so only blocks with an Inf or NaN scale can
-// change the state, and the first NaN event fixes the bits.  Called only for a
-// cell whose sum came out NaN; NaN-ness itself is the same on every IEEE machine.
-// ----------------------------------------------------------------------------
-constexpr int kSNanTile = 0;
-constexpr int kSNanQdot = 1;
-static_assert(kSNanTile != kSNanQdot, "the two NaN forms");
-
-__device__ __forceinline__ float f16_ref(uint32_t h, int mode) {
-    if (!f16_is_nan(h)) return f16_ieee(h);
-    return mode == kSNanTile ? __uint_as_float(((h & 0x8000u) << 16) | 0x7FC00000u) : f16_nan_x86(h);
-}
-
-__device__ __noinline__ float s_order_nan_bits(const uint8_t* __restrict__ wrow, const uint8_t* __restrict__ xrow,
-                                               int nb, int mode) {
-    float acc = 0.0f;  // stands for any finite value
-    for (int b = 0; b < nb; b++) {
-        const uint8_t* wb = wrow + (int64_t)b * kQ80Bytes;
-        const uint8_t* xb = xrow + (int64_t)b * kQ80Bytes;
-        const uint32_t hw = (uint32_t)wb[0] | ((uint32_t)wb[1] << 8);
-        const uint32_t hx = (uint32_t)xb[0] | ((uint32_t)xb[1] << 8);
-        if (!f16_exp31(hw) && !f16_exp31(hx)) continue;
-        const float fw = f16_ref(hw, mode), fx = f16_ref(hx, mode);
-        const float first = mode == kSNanTile ? fx : fw, second = mode == kSNanTile ? fw : fx;
-        const float delta = first * second;
-        // a NaN product: p = float(S_b) * delta is delta's NaN, and acc + p is p's
-        if (__builtin_isnan(delta)) return x86_nan_of(first, second);
-        // delta is +/-Inf: p = +/-Inf, or the default NaN when S_b = 0
-        int sumi = 0;
-        for (int j = 0; j < 32; j++) sumi += (int)(int8_t)wb[2 + j] * (int)(int8_t)xb[2 + j];
-        if (sumi == 0) return __uint_as_float(kX86NaN);
-        const float p = sumi < 0 ? -delta : delta;
-        if (__builtin_isinf(acc) && acc != p) return __uint_as_float(kX86NaN);  // Inf - Inf
-        acc = p;
-    }
-    return acc;
-}
-
 constexpr int kGT = 128;  // tile rows = tile tokens
 constexpr int kGB = 4;    // blocks per LDS stage
 
@@ -1399,6 +1347,7 @@ void launch_q8_0_gemm_S_multi(const uint8_t* const* W, float* const* out, const 
                               int m_tokens, int K, int nan_mode, hipStream_t s) {
     bool aligned = K % 128 == 0 && (reinterpret_cast<uintptr_t>(Xq) & 3) == 0;
     for (int i = 0; i < n; i++) aligned = aligned && (reinterpret_cast<uintptr_t>(W[i]) & 3) == 0;
+    if (launch_q8_0_gemm_S_few(W, out, M, n, Xq, m_tokens, K, aligned, nan_mode, s)) return;
     if (K / 32 == 0 || !aligned) {
         for (int i = 0; i < n; i++) {
             if (K / 32 == 0) {  // the kernel indexes block nb-1

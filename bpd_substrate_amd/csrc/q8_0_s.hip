@@ -1,0 +1,325 @@
+// q8_0_s.hip — Q8_0 x Q8_0 for few activation rows in the scalar order S
+// (bench/bpd_gemm_q8_0_cpu.c:102-131, bench/bpd_cpu.c:4263-4280), on int8 MFMA.
+#include <mutex>
+
+#include "bpdq_device.h"
+#include "bpdq_launch.h"
+#include "bpdq_q8_0.h"
+
+namespace bpdq {
+
+// ----------------------------------------------------------------------------
+// k_q8_0_gemm_SQ.  Per cell  acc = RN(acc + RN(float(S_b) * RN(Ad_b * Bd_b)))  over the
+// blocks in order, S_b the exact dot of the cell's two blocks.  k_q8_0_gemm_SH stages 128
+// tokens for any token count and waits for one half-stage of 4 blocks at a time, so a few
+// tokens cost what 128 do and every 4 blocks a memory round trip: 14336x8, K = 4096, 46 us
+// there, 18 here (62 MB at 3.5 TB/s; a wave alone on its SIMD issues an instruction every 5
+// cycles, 34 VALU and MFMA of them per 4 blocks, and that bounds it).  Here the workgroup puts
+// its C activation rows into LDS once; after that barrier each wave runs by itself over its
+// 16 rows: chunks of 16 blocks as 16-byte pieces, two chunks in flight in registers, through
+// its own LDS slot (a wave's LDS operations execute in order, so the next chunk is written
+// behind the last reads of this one without a wait).  One v_mfma_i32_16x16x32_i8 is one
+// block of 16 rows x 16 tokens; the scale products of four blocks come from one
+// v_mfma_f32_16x16x4_4b_f16 (scales at inner index 0, zeros elsewhere: exact), so a tile and
+// block costs the 12 VALU operations of the order (convert, multiply, add for 4 cells per
+// lane) and one realignment.  Any K and any alignment (the pieces
+// are 16-byte loads at any address), as long as the activation fits in LDS.
+// LDS: a weight row's chunk at an odd multiple of 8 dwords (16 rows x 4 eight-byte groups of
+// a block meet each bank twice, the least for 512 bytes); the quants of C tokens of a block
+// are contiguous.
+// ----------------------------------------------------------------------------
+typedef _Float16 sh16x4 __attribute__((ext_vector_type(4)));
+typedef float sf32x16 __attribute__((ext_vector_type(16)));
+typedef int si32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t su32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t su32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
+
+constexpr int kSqPieces = 34;             // 16-byte pieces of a row's chunk of 16 blocks
+constexpr int kSqPitch = 16 * kSqPieces;  // 544 bytes: 136 dwords, 8 mod 64
+constexpr int kSqSlot = 16 * kSqPitch;    // a wave's 16 rows
+constexpr int kSqPer = (16 * kSqPieces + 63) / 64;
+constexpr int kSqMaxLds = 160 * 1024;
+
+// blocks of the activation in LDS: whole groups of 4, zeros past the end (a zero block adds
+// +0 to a sum that is never -0)
+__host__ __device__ constexpr int sq_blocks(int nb) { return (nb + 3) / 4 * 4; }
+// bytes of LDS: quants [blocks][C][32], f16 scales [blocks][C], the waves' slots
+__host__ __device__ constexpr size_t sq_lds(int C, int nw, int nb) {
+    return (size_t)sq_blocks(nb) * C * 34 + (size_t)nw * kSqSlot;
+}
+
+// The operands of blocks 4t .. 4t+3 of a chunk.
+struct SqOps {
+    uint32_t a[4][3];  // even blocks: 3 dwords from 2 bytes before the quants; odd ones: 2
+    uint32_t da, db;   // the scales of block 4t + lane / 16: this lane's row, this lane's token
+    uint2 b[4];
+};
+
+template <int C>
+__device__ __forceinline__ void sq_read(SqOps& o, const uint8_t* wq, const uint8_t* wd, const uint8_t* xq,
+                                        const uint16_t* xd, int t) {
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int off = 34 * (4 * t + u);
+        if (u & 1) {
+            o.a[u][0] = *reinterpret_cast<const uint32_t*>(wq + off + 2);
+            o.a[u][1] = *reinterpret_cast<const uint32_t*>(wq + off + 6);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 3; i++) o.a[u][i] = *reinterpret_cast<const uint32_t*>(wq + off + 4 * i);
+        }
+        o.b[u] = *reinterpret_cast<const uint2*>(xq + (4 * t + u) * C * 32);
+    }
+    o.da = *reinterpret_cast<const uint16_t*>(wd + 136 * t);
+    o.db = xd[4 * t * C];
+}
+
+__device__ __forceinline__ void sq_group(const SqOps& o, float (&acc)[4]) {
+    const sf32x16 fzero = {0.0f};
+    const si32x4 zero = {0, 0, 0, 0};
+    const sf32x16 delta =
+        __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(sh16x4, make_uint2(o.da, 0u)),
+                                             __builtin_bit_cast(sh16x4, make_uint2(o.db, 0u)), fzero, 0, 0, 0);
+    si32x4 s[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const uint2 w = u & 1 ? make_uint2(o.a[u][0], o.a[u][1])
+                              : make_uint2(__builtin_amdgcn_alignbit(o.a[u][1], o.a[u][0], 16),
+                                           __builtin_amdgcn_alignbit(o.a[u][2], o.a[u][1], 16));
+        s[u] = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, w), __builtin_bit_cast(long, o.b[u]), zero,
+                                                     0, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[r] = acc[r] + (float)s[u][r] * delta[4 * u + r];
+    // the group's arithmetic ends here (the compiler would move every group's to the end of
+    // the unrolled chunk and spill)
+    asm volatile("" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+}
+
+template <int C, int NW>
+__global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_SQ(GemmW gw, const uint8_t* __restrict__ X, int m_tokens, int nb,
+                                                          int nan_mode) {
+    constexpr int R = 16 * NW, NT = 64 * NW;
+    extern __shared__ __align__(16) uint8_t sqlds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int bx, by;
+    sh_tile(blockIdx.x, gw.first[kGemmMulti], (m_tokens + C - 1) / C, bx, by);
+    const int mi = (bx >= gw.first[1]) + (bx >= gw.first[2]);
+    const uint8_t* __restrict__ W = gw.w[mi];
+    float* __restrict__ out = gw.out[mi];
+    const int m_weight = gw.m[mi];
+    const int row0 = (bx - gw.first[mi]) * R + wave * 16, n0 = by * C;
+    const int64_t bpr = (int64_t)nb * kQ80Bytes;
+    const int nch = (nb + 15) / 16, nbp = sq_blocks(nb);
+    const int last = (int)bpr - 16;  // where a row's last 16 bytes start
+
+    // weights: rows past the end repeat the last one; a piece past a row's end is its last
+    // 16 bytes, moved into place (zeros behind) by wfix
+    const int base = min(row0, m_weight - 1);
+    const uint8_t* wbase = W + (int64_t)base * bpr;
+    uint32_t off[kSqPer], dst[kSqPer];
+    int pc[kSqPer];
+#pragma unroll
+    for (int k = 0; k < kSqPer; k++) {
+        const int f = min(lane + 64 * k, 16 * kSqPieces - 1), r = f / kSqPieces;
+        pc[k] = f % kSqPieces;
+        off[k] = (uint32_t)((min(row0 + r, m_weight - 1) - base) * bpr);
+        dst[k] = (uint32_t)(r * kSqPitch + 16 * pc[k]);
+    }
+    uint8_t* xs = sqlds;
+    uint16_t* xsc = reinterpret_cast<uint16_t*>(sqlds + (size_t)nbp * C * 32);
+    uint8_t* slot = sqlds + (size_t)nbp * C * 34 + wave * kSqSlot;
+    const auto wload = [&](su32x4 (&v)[kSqPer], int c) {
+        const int at = min(c, nch - 1) * kSqPitch;
+#pragma unroll
+        for (int k = 0; k < kSqPer; k++)
+            v[k] = *reinterpret_cast<const su32x4_a1*>(wbase + (off[k] + (uint32_t)min(at + 16 * pc[k], last)));
+    };
+    const auto wfix = [&](su32x4 (&v)[kSqPer]) {  // chunk nch - 1
+#pragma unroll
+        for (int k = 0; k < kSqPer; k++) {
+            const int past = (nch - 1) * kSqPitch + 16 * pc[k] - last;
+            if (past <= 0) continue;
+            const unsigned __int128 x = __builtin_bit_cast(unsigned __int128, v[k]);
+            v[k] = __builtin_bit_cast(su32x4, past >= 16 ? (unsigned __int128)0 : x >> (8 * past));
+        }
+    };
+    const auto wstore = [&](const su32x4 (&v)[kSqPer]) {
+        asm volatile("" ::: "memory");  // behind the reads of the previous chunk
+#pragma unroll
+        for (int k = 0; k < kSqPer; k++)
+            if (k < kSqPer - 1 || lane + 64 * k < 16 * kSqPieces) *reinterpret_cast<su32x4*>(slot + dst[k]) = v[k];
+        asm volatile("" ::: "memory");
+    };
+
+    // the activation: unit i is token i % C, half (i / C) & 1 of block i / (2 C); the first
+    // batch is loaded before the weights (loads return in order)
+    constexpr int XU = 4;
+    su32x4 xv[XU];
+    uint32_t xh[XU];
+    const int nu = 2 * C * nb, nup = 2 * C * nbp;
+    const auto xload = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < XU; u++) {
+            const int i = min(i0 + u * NT, nu - 1);
+            const uint8_t* s = X + (int64_t)min(n0 + i % C, m_tokens - 1) * bpr + (i / (2 * C)) * kQ80Bytes;
+            xv[u] = *reinterpret_cast<const su32x4_a1*>(s + 2 + 16 * ((i / C) & 1));
+            xh[u] = ld_u16(s);
+        }
+    };
+    const auto xstore = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < XU; u++) {
+            const int i = i0 + u * NT, t = i % C, h = (i / C) & 1, b = i / (2 * C);
+            if (i >= nup) continue;
+            *reinterpret_cast<su32x4*>(xs + ((size_t)b * C + t) * 32 + 16 * h) = i < nu ? xv[u] : su32x4{0, 0, 0, 0};
+            if (h == 0) xsc[b * C + t] = i < nu ? (uint16_t)xh[u] : (uint16_t)0;
+        }
+    };
+    su32x4 wv[2][kSqPer];
+    xload(tid);
+    __builtin_amdgcn_sched_barrier(0);
+    wload(wv[0], 0);
+    wload(wv[1], 1);
+    __builtin_amdgcn_sched_barrier(0);
+    xstore(tid);
+    for (int i0 = tid + XU * NT; i0 < nup; i0 += XU * NT) {
+        xload(i0);
+        xstore(i0);
+    }
+    lds_barrier();
+
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int j = lane & 15, k = lane >> 4;
+    const uint8_t* wq = slot + j * kSqPitch + 8 * k;   // this lane's row, eight quants from 8 k
+    const uint8_t* wd = slot + j * kSqPitch + 34 * k;  // the scale of block k of a group of four
+    const uint8_t* xq = xs + (j % C) * 32 + 8 * k;     // columns past C repeat tokens (not stored)
+    const uint16_t* xd = xsc + k * C + j % C;
+    SqOps o[2];
+    if (nch == 1) wfix(wv[0]);
+    wstore(wv[0]);
+    wload(wv[0], 2);
+    sq_read<C>(o[0], wq, wd, xq, xd, 0);
+    // a whole chunk of 4 groups; the next chunk goes into the slot behind the last group's reads
+    const auto step = [&](su32x4 (&next)[kSqPer], int c) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            if (t < 3) {
+                sq_read<C>(o[(t + 1) & 1], wq, wd, xq, xd, t + 1);
+            } else {
+                xq += 16 * C * 32;
+                xd += 16 * C;
+                if (c + 2 == nch) wfix(next);
+                wstore(next);
+                wload(next, c + 3);
+                sq_read<C>(o[0], wq, wd, xq, xd, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            sq_group(o[t & 1], acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    int c = 0;
+    for (; c + 2 < nch; c += 2) {
+        step(wv[1], c);
+        step(wv[0], c + 1);
+    }
+    if (c + 1 < nch) {
+        step(wv[1], c);
+        c++;
+    }
+    // the last chunk: 1 to 4 groups, the first already read
+    const int ng = (nb - 16 * c + 3) / 4;
+#pragma unroll 1
+    for (int t = 0; t < ng; t += 2) {
+        sq_read<C>(o[1], wq, wd, xq, xd, min(t + 1, ng - 1));
+        sq_group(o[0], acc);
+        if (t + 1 == ng) break;
+        sq_read<C>(o[0], wq, wd, xq, xd, min(t + 2, ng - 1));
+        sq_group(o[1], acc);
+    }
+
+    // register r of lane l: row 4 (l / 16) + r of the wave's 16, token l % 16
+    const int tok = n0 + j, r0 = row0 + 4 * k;
+    if (j >= C || tok >= m_tokens) return;
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        if (__builtin_isnan(acc[r]) && r0 + r < m_weight)
+            acc[r] = s_order_nan_bits(W + (r0 + r) * bpr, X + tok * bpr, nb, nan_mode);
+    float* o_ = out + (int64_t)tok * m_weight + r0;
+    if ((reinterpret_cast<uintptr_t>(o_) & 15) == 0 && r0 + 4 <= m_weight) {
+        *reinterpret_cast<float4*>(o_) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+            if (r0 + r < m_weight) o_[r] = acc[r];
+    }
+}
+
+template <int C, int NW>
+static bool launch_sq(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq, int m_tokens,
+                      int nb, int nan_mode, hipStream_t s) {
+    const size_t lds = sq_lds(C, NW, nb);
+    if (lds > kSqMaxLds) return false;
+    if (lds > 64 * 1024) {  // asked for once per process
+        static std::once_flag once;
+        static bool ok = false;
+        std::call_once(once, [] {
+            ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_q8_0_gemm_SQ<C, NW>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, kSqMaxLds) == hipSuccess;
+            (void)hipGetLastError();
+        });
+        if (!ok) return false;
+    }
+    const GemmW g = gemm_args<16 * NW>(W, out, M, n);
+    hipLaunchKernelGGL((k_q8_0_gemm_SQ<C, NW>), dim3(g.first[kGemmMulti] * ((m_tokens + C - 1) / C)), dim3(64 * NW), lds, s,
+                       g, Xq, m_tokens, nb, nan_mode);
+    return true;
+}
+
+// Which form, or none (the caller then takes k_q8_0_gemm_SH or, where that does not run,
+// k_q8_0_gemm_S).  A workgroup costs about the same however many of its tokens are real
+// and whatever the row count, so the time of a launch is its workgroups per CU times one
+// workgroup's cost; in units of 0.01 us per block: 8, 9, 15 and 24 for 4, 8, 16 tokens x 64
+// rows and 16 x 128; k_q8_0_gemm_SH costs 30 and k_q8_0_gemm_S 110, and 1 more for every 8
+// workgroups of 128 rows.  The cheapest form that fits in LDS is taken if it is cheaper than
+// that.  Measured, us per call, weights beyond the MALL, the other kernel in brackets:
+//   K = 4096   14336x1 15.6 (48), x8 18.8 (46), x16 22-25 (47), x32 31.6 (49; x48 58 against
+//              49: not taken); 4096x1 12.0 (39), x16 13.5 (41), x32 15.3 (41), x64 21.2 (43),
+//              x128 29.5 (44); 28672x8 30 (66); 128256x1 101 (241); 1024x512 29.5 (44)
+//   K = 14336  4096x1 32 (129), 4096x64 90 (143; x100 165 against 150: not taken)
+//   K = 28672  8192x16 137 (281)
+//   K = 1440   5413x3 9.4 (52), 5413x40 12.5 (55), 14336x64 30.4 (57)
+//   K = 3776   325x233 14.3 (134);  K = 8320  1097x17 21.9 (76)
+bool launch_q8_0_gemm_S_few(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq,
+                            int m_tokens, int K, bool staged, int nan_mode, hipStream_t s) {
+    const int nb = K / 32;
+    if (nb == 0) return false;
+    const auto wgs = [&](int rows, int tokens) {
+        int64_t b = 0;
+        for (int i = 0; i < n; i++) b += (M[i] + rows - 1) / rows;
+        return b * ((m_tokens + tokens - 1) / tokens);
+    };
+    struct Form {
+        int rows, tokens, cost;
+        bool (*launch)(const uint8_t* const*, float* const*, const int*, int, const uint8_t*, int, int, int, hipStream_t);
+    };
+    static constexpr Form forms[] = {{64, 4, 8, launch_sq<4, 4>},
+                                     {64, 8, 9, launch_sq<8, 4>},
+                                     {64, 16, 15, launch_sq<16, 4>},
+                                     {128, 16, 24, launch_sq<16, 8>}};
+    int64_t least = (staged ? 30 : 110) + wgs(128, 128) / 8;
+    const Form* form = nullptr;
+    for (const Form& f : forms) {
+        const int64_t cost = (wgs(f.rows, f.tokens) + 255) / 256 * f.cost;
+        if (cost >= least || sq_lds(f.tokens, f.rows / 16, nb) > kSqMaxLds) continue;
+        least = cost;
+        form = &f;
+    }
+    return form != nullptr && form->launch(W, out, M, n, Xq, m_tokens, nb, nan_mode, s);
+}
+
+}  // namespace bpdq

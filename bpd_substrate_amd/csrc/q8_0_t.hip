@@ -494,22 +494,6 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
     }
 }
 
-template <int R>
-static GemmW gemm_args(const uint8_t* const* W, float* const* out, const int* M, int n) {
-    GemmW g{};
-    int blocks = 0;
-    for (int i = 0; i < kGemmMulti; i++) {
-        const int q = i < n ? i : 0;
-        g.first[i] = blocks;
-        g.w[i] = W[q];
-        g.out[i] = out[q];
-        g.m[i] = M[q];
-        if (i < n) blocks += (M[i] + R - 1) / R;
-    }
-    g.first[kGemmMulti] = blocks;
-    return g;
-}
-
 template <int WRN, int WCN, int CT, int PF>
 static void launch_tm(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq, int m_tokens,
                       int nb, bool aligned, hipStream_t s) {
