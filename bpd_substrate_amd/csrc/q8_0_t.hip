@@ -260,7 +260,9 @@ __global__ __launch_bounds__(64 * WRN * WCN) void k_q8_0_gemm_TM(GemmW gw, const
 // 4 NQ registers.  Each wave streams its own rows in chunks of CB blocks through
 // registers (two chunks in flight) and its own LDS slot as 16-byte pieces; the
 // workgroup shares only the activation chunk (f16, two slots), so there is one
-// barrier per CB blocks.  Needs nb % 8 == 0 and W 16-byte aligned.
+// barrier per CB blocks.  Any K and alignment: the pieces are 16-byte loads at any address,
+// and zero blocks fill the last chunk.  (4096x8 at K = 4128: 34.5 us in per-token GEMVs,
+// 15.8 here; at K = 4096 the alignment is worth less than the runs differ.)
 // LDS: rows at an odd multiple of 8 dwords (8 rows x 8 quant dwords of a block touch
 // 64 different banks); the quants of 4 tokens of a block are 256 contiguous bytes.
 // ----------------------------------------------------------------------------
@@ -351,9 +353,11 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
     const int m_weight = gw.m[mi];
     const int row0 = (bx - gw.first[mi]) * G::R + wave * 8, n0 = by * G::C;
     const int64_t bpr = (int64_t)nb * kQ80Bytes;
-    const int nch = (nb + CB - 1) / CB, npc = nb * 17 / 8;  // chunks, 16-byte pieces of a row
+    const int nch = (nb + CB - 1) / CB;
+    const int last = (int)bpr - 16;  // where a row's last 16 bytes start
 
-    // weights: piece k of this lane is piece f % PIECES of row f / PIECES of the chunk
+    // weights: piece k of this lane is piece f % PIECES of row f / PIECES of the chunk; a
+    // piece past the row's end is its last 16 bytes, moved into place (zeros behind) by wfix
     const uint8_t* wbase = W + (int64_t)min(row0, m_weight - 1) * bpr;
     uint32_t off[G::PER], dst[G::PER];
     int pc[G::PER];
@@ -366,10 +370,18 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
     }
     uint8_t* slot = lds + 2 * G::XSLOT + wave * 8 * G::PITCH;
     const auto wload = [&](tu32x4 (&v)[G::PER], int c) {
+        const int at = min(c, nch - 1) * 16 * G::PIECES;
+#pragma unroll
+        for (int k = 0; k < G::PER; k++)
+            v[k] = *reinterpret_cast<const tu32x4_a1*>(wbase + (off[k] + (uint32_t)min(at + 16 * pc[k], last)));
+    };
+    const auto wfix = [&](tu32x4 (&v)[G::PER]) {  // chunk nch - 1
 #pragma unroll
         for (int k = 0; k < G::PER; k++) {
-            const uint8_t* s = wbase + off[k] + 16 * min(c * G::PIECES + pc[k], npc - 1);
-            v[k] = *reinterpret_cast<const tu32x4*>(s);
+            const int past = (nch - 1) * 16 * G::PIECES + 16 * pc[k] - last;
+            if (past <= 0) continue;
+            const unsigned __int128 x = __builtin_bit_cast(unsigned __int128, v[k]);
+            v[k] = __builtin_bit_cast(tu32x4, past >= 16 ? (unsigned __int128)0 : x >> (8 * past));
         }
     };
     // activations: unit i is half i & 1 of block (i / 2) % CB of token i / (2 CB)
@@ -384,12 +396,13 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
         }
     };
     uint32_t bad[G::XP] = {};
-    const auto xstore = [&](int xs) {
+    const auto xstore = [&](int xs, int c) {
         uint8_t* x = lds + xs * G::XSLOT;
 #pragma unroll
         for (int u = 0; u < G::XP; u++) {
             const int i = tid + u * G::NT, t = i / (2 * CB), b = (i >> 1) % CB;
             if (G::UX % G::NT != 0 && i >= G::UX) continue;
+            if (c * CB + b >= nb) xr[u] = TqX{{0, 0, 0, 0}, 0};  // a zero block adds +0
             const uint2 q0 = tm_f16(xr[u].q[0]), q1 = tm_f16(xr[u].q[1]), q2 = tm_f16(xr[u].q[2]), q3 = tm_f16(xr[u].q[3]);
             uint4* d = reinterpret_cast<uint4*>(x + b * G::PLANE + t * 64 + 32 * (i & 1));
             d[0] = make_uint4(q0.x, q0.y, q1.x, q1.y);
@@ -405,7 +418,7 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
     wload(wv[0], 0);
     wload(wv[1], 1);
     for (int i = tid; i < G::C; i += G::NT) m128[i] = 0u;
-    xstore(0);
+    xstore(0, 0);
     lds_barrier();
 
     float acc[NQ][4];
@@ -418,6 +431,7 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
     const uint8_t* wd = slot + (4 * rg + j) * G::PITCH;
 
     const auto step = [&](tu32x4 (&v)[G::PER], int xs, int c) {
+        if (c == nch - 1) wfix(v);
 #pragma unroll
         for (int k = 0; k < G::PER; k++)
             if (k < G::PER - 1 || G::WP % 64 == 0 || lane + 64 * k < G::WP) *reinterpret_cast<tu32x4*>(slot + dst[k]) = v[k];
@@ -430,7 +444,7 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
         // pairs of blocks, the next pair's operands read before this one's arithmetic
         TqOps<NQ> o[2];
         tq_read<NQ, G::C, G::PLANE>(o[0], wq, wd, xq, xd, 0);
-        if (CB == 8 || (c + 1) * CB <= nb) {
+        if ((c + 1) * CB <= nb) {
 #pragma unroll
             for (int t = 0; t < CB / 2; t++) {
                 if (t + 1 < CB / 2) tq_read<NQ, G::C, G::PLANE>(o[(t + 1) & 1], wq, wd, xq, xd, t + 1);
@@ -439,14 +453,14 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
                 __builtin_amdgcn_sched_barrier(0);
             }
         } else {
-            const int npair = (nb - c * CB) / 2;
+            const int npair = (nb - c * CB + 1) / 2;
 #pragma unroll 1
             for (int t = 0; t < npair; t++) {
                 tq_read<NQ, G::C, G::PLANE>(o[0], wq, wd, xq, xd, t);
                 tq_pair<NQ>(o[0], acc);
             }
         }
-        xstore(xs ^ 1);  // last read before the previous barrier
+        xstore(xs ^ 1, c + 1);  // last read before the previous barrier
         lds_barrier();
     };
     int c0 = 0;
@@ -520,7 +534,9 @@ static void launch_tq(const uint8_t* const* W, float* const* out, const int* M, 
 // per call, the per-token GEMVs they replace in brackets:
 //   TQ   14336x2 18.9 (22.3), 14336x4 19.0 (39.7), 14336x8 26 (73), 4096x4 13.5
 //        (14.1), 4096x8 13.8 (22.7), 4096x16 17.8 (41), 4096x32 25.9 (75);
-//        1024x8 12.6 (7.5: the GEMVs stay below 16,384 cells);
+//        1024x8 12.6 (7.5: the GEMVs stay below 16,384 cells); K = 4128: 14336x2 23.5
+//        (36), 4096x4 15.4 (20), 4096x2 15.5 (15.7); K = 1440: 5413x3 8.4 (9.7), 1024x4
+//        8.2 (5.4);
 //   TM   32 rows x 64 tokens: 4096x64 45.6 (TQ 48), 4096x128 46.7 (TQ 89), 1024x512
 //        50 (304); 64 x 64: 14336x32 67 (TQ 80), 14336x64 69 (650), 4096x512 137
 //        (1,360), 14336x512 434 (4,890: 84 % of the 382 us that 16 VALU operations
@@ -530,20 +546,15 @@ static void launch_tq(const uint8_t* const* W, float* const* out, const int* M, 
 bool launch_q8_0_gemm_T_multi(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq,
                               int m_tokens, int K, hipStream_t s) {
     const int nb = K / 32;
-    bool al4 = nb % 2 == 0 && (reinterpret_cast<uintptr_t>(Xq) & 3) == 0, al16 = nb % 8 == 0;
+    bool al4 = nb % 2 == 0 && (reinterpret_cast<uintptr_t>(Xq) & 3) == 0;
     int64_t rows = 0;
     for (int i = 0; i < n; i++) {
         rows += M[i];
         al4 = al4 && (reinterpret_cast<uintptr_t>(W[i]) & 3) == 0;
-        al16 = al16 && (reinterpret_cast<uintptr_t>(W[i]) & 15) == 0;
     }
-    if (nb == 0 || m_tokens < 2) return false;
-    if (al16 && rows * m_tokens < 16384) return false;
-    // without 16-byte rows the few-token kernel does not apply, and the GEMVs take the
-    // dword form: 18 us per token at 14336x4096 against 46 for the smallest TM launch
-    if (!al16 && rows * m_tokens < 40960) return false;
+    if (nb == 0 || m_tokens < 2 || rows * m_tokens < 16384) return false;
     const int64_t w8 = (rows + 7) / 8 * ((m_tokens + 7) / 8);  // waves of 8 rows x 8 tokens
-    if (al16 && w8 <= 4096) {
+    if (w8 <= 4096) {
         if (w8 < 1024)
             launch_tq<1, 4, 16>(W, out, M, n, Xq, m_tokens, nb, s);
         else

@@ -14,11 +14,15 @@ pytestmark = pytest.mark.gpu
 CASES = [(4099, 4, 256, 0),      # 4 tokens per wave, a half chunk
          (2050, 9, 768, 0),      # 4 tokens per wave, a whole and a half chunk, 3 token groups
          (4100, 13, 1280, 0),    # 8 tokens per wave
+         (703, 65, 224, 0),      # 4 tokens per wave, an odd number of blocks
+         (4100, 14, 544, 0),     # 8 tokens per wave, a last chunk of one block
+         (8200, 2, 32, 2),       # one block, W off the 4-byte grid
+         (703, 65, 960, 1),      # 30 blocks, W at an odd address
          (1030, 290, 512, 0),    # 32 x 64 tiles
-         (703, 65, 192, 0),      # ... K % 256 != 0
-         (703, 65, 224, 0),      # ... an odd number of blocks
-         (703, 65, 256, 2),      # ... W off the 4-byte grid
-         (703, 65, 256, 1),      # ... W at an odd address
+         (1030, 290, 192, 0),    # ... K % 256 != 0
+         (1030, 290, 224, 0),    # ... an odd number of blocks
+         (1030, 290, 256, 2),    # ... W off the 4-byte grid
+         (1030, 290, 256, 1),    # ... W at an odd address
          (4100, 300, 128, 0),    # 64 x 64 tiles
          (4100, 300, 96, 0)]
 
