@@ -1,7 +1,8 @@
 // q6k.hip — Q6_K super-block kernels for gfx950.
 //
 //   k_dequant_q6k<ORDER>        Q6_K -> fp32
-//   k_q6k_q8k_gemv<ORDER>       Q6_K x Q8_K GEMV, exact integer group sums + fixed fp32 tree
+//   k_q6k_q8k_gemv<ORDER>       Q6_K x Q8_K GEMV, exact integer group sums + fixed fp32 tree; _span, _span_long
+//                               and _stream forms for K = 4096, K = 14336 and other long rows
 //
 // Q6_K block, 210 B per 256 elements: ql[128] (low 4 bits), qh[64] (high 2 bits),
 // sc[16] (int8, element e uses sc[e/16]), d (f16 at byte 208); q = low | high<<4, minus 32.
@@ -512,6 +513,123 @@ __global__ __launch_bounds__(64 * WPB) void k_q6k_q8k_gemv_span_long(const uint8
     if (lane == 0 && has) y[row] = (p01 + p23) + (p45 + p67);
 }
 
+// Any K from 9 super-blocks, W at any 2-byte address: passes of 8 super-blocks as 16-byte loads at
+// any address, kQ6Ahead passes in flight in registers over the wave's R rows, one after the
+// other through the wave's LDS buffer; x as the lanes' records in LDS, staged once per
+// workgroup (k_q6k_q8k_gemv_span_long).  The last pass of a row is the row's last 1,680
+// bytes, of which only the pieces with blocks not yet seen are read, so every load stays
+// inside its row.  Integer sums, c_b and the fp32 order are k_q6k_q8k_gemv's.
+// k_q6k_q8k_gemv waits for memory once per 8 super-blocks and builds the six-bit values of
+// the reference map bit by bit (3.0 TB/s at 25296x3072); here the LDS pipe bounds a long
+// launch, about 8 bytes through it for each weight byte (3.9 TB/s).
+constexpr int kQ6Rec = 20;    // dwords of an x record: xs[16], bs0, bs1, dy, pad
+constexpr int kQ6Ahead = 4;
+constexpr int kQ6PassPieces = kQ6Pass / 16;  // 105
+
+__host__ __device__ constexpr size_t q6_stream_lds(int nb, int wpb) {
+    return (size_t)nb * 8 * kQ6Rec * 4 + (size_t)wpb * kQ6Buf;
+}
+
+template <int ORDER, int WPB>
+__global__ __launch_bounds__(64 * WPB) void k_q6k_q8k_gemv_stream(const uint8_t* __restrict__ w,
+                                                                 const uint8_t* __restrict__ xq,
+                                                                 float* __restrict__ y, int M, int nb, int R) {
+    extern __shared__ __align__(16) uint8_t q6lds[];
+    uint32_t* xrec = reinterpret_cast<uint32_t*>(q6lds);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int q = lane >> 3, c = lane & 7;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    uint8_t* buf = q6lds + (size_t)nb * 8 * kQ6Rec * 4 + wave * kQ6Buf;
+    const int row0 = (xcd_major(blockIdx.x, gridDim.x) * WPB + wave) * R;
+    const int64_t row_bytes = (int64_t)nb * kQ6KBytes;
+    const int np = (nb + 7) >> 3, tail = nb - 8 * (np - 1);  // passes; super-blocks of the last
+    const int lead = kQ6Pass - tail * kQ6KBytes;             // bytes of it that the one before held
+    const int total = max(min(R, M - row0), 0) * np;
+    // x: thread tid the records tid, tid + 64 WPB, ...; the first batch before the weights
+    const int nrec = nb * 8;
+    const auto xread = [&](int i) {
+        const int k = min(i, nrec - 1);
+        return q6x_load_raw<ORDER>(xq + (int64_t)(k >> 3) * kQ8KBytes, k & 7);
+    };
+    const auto xwrite = [&](const Q6XRaw& r, int i) {
+        if (i >= nrec) return;
+        const Q6X<ORDER> xo = q6x_regroup<ORDER>(r);
+        uint32_t* rec = xrec + i * kQ6Rec;
+#pragma unroll
+        for (int k = 0; k < (ORDER == 0 ? 16 : 8); k++) rec[k] = xo.xs[k];
+        rec[16] = (uint32_t)xo.bs0;
+        rec[17] = (uint32_t)xo.bs1;
+        rec[18] = __float_as_uint(xo.dy);
+    };
+    // the next pass to load: its row's address, its index in the row
+    const uint8_t* lrow = w + (int64_t)min(row0, M - 1) * row_bytes;
+    int lt = 0, li = 0;
+    q6u32x4 v[kQ6Ahead][2];
+    const auto load = [&](q6u32x4 (&d)[2]) {
+        const bool end = lt == np - 1;
+        // past the last pass: one 16-byte read that every lane shares
+        const int lo = end ? lead >> 4 : 0, hi = li < total ? kQ6PassPieces - 1 : lo;
+        const uint8_t* base = lrow + ((int64_t)lt * kQ6Pass - (end ? lead : 0));
+        typedef q6u32x4 q6u32x4_a1 __attribute__((aligned(1)));
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            d[u] = __builtin_nontemporal_load(
+                reinterpret_cast<const q6u32x4_a1*>(base + 16 * min(max(lane + 64 * u, lo), hi)));
+        li++;
+        if (li < total) {
+            lt = end ? 0 : lt + 1;
+            if (end) lrow += row_bytes;
+        }
+    };
+    const Q6XRaw xr = xread(tid);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int a = 0; a < kQ6Ahead; a++) load(v[a]);
+    __builtin_amdgcn_sched_barrier(0);
+    xwrite(xr, tid);
+    for (int i = tid + 64 * WPB; i < nrec; i += 64 * WPB) xwrite(xread(i), i);
+    __syncthreads();
+    float s = 0.0f;
+    int t = 0, row = row0;
+    for (int i0 = 0; i0 < total; i0 += kQ6Ahead) {
+#pragma unroll
+        for (int a = 0; a < kQ6Ahead; a++) {
+            if (i0 + a >= total) break;
+#pragma unroll
+            for (int u = 0; u < 2; u++)  // pieces past the pass go to the spare slot behind it
+                *reinterpret_cast<q6u32x4*>(buf + 16 * min(lane + 64 * u, kQ6PassPieces)) = v[a][u];
+            load(v[a]);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            const bool end = t == np - 1;
+            const int qq = end ? min(q, tail - 1) : q;
+            Q6X<ORDER> x;
+            const uint32_t* rec = xrec + ((8 * t + qq) * 8 + c) * kQ6Rec;
+#pragma unroll
+            for (int k = 0; k < (ORDER == 0 ? 16 : 8); k++) x.xs[k] = rec[k];
+            x.bs0 = (int)rec[16];
+            x.bs1 = (int)rec[17];
+            x.dy = __uint_as_float(rec[18]);
+            const uint8_t* blk = buf + (end ? lead : 0) + qq * kQ6KBytes;
+            int isum = q6k_lane_isum_lds<ORDER>(blk, x, c);
+            isum = sum8_i(isum);
+            uint16_t dh;
+            __builtin_memcpy(&dh, blk + 208, 2);
+            const float sum = s + (f16_ieee(dh) * x.dy) * (float)isum;
+            s = qq == q ? sum : s;
+            asm volatile("" : "+v"(s) : : "memory");  // as in k_q6k_q8k_gemv_span
+            t = end ? 0 : t + 1;
+            if (end) {
+                s = s + dpp_f<0x140>(s);
+                const float p01 = readlane_f(s, 0), p23 = readlane_f(s, 16);
+                const float p45 = readlane_f(s, 32), p67 = readlane_f(s, 48);
+                if (lane == 0) y[row] = (p01 + p23) + (p45 + p67);
+                s = 0.0f;
+                row++;
+            }
+        }
+    }
+}
+
 void launch_qmatmul_q6k_q8k(const uint8_t* w, const uint8_t* xq, float* y, int M, int K, int order, hipStream_t s) {
     if (K == 14336 && (reinterpret_cast<uintptr_t>(w) & 15) == 0) {
         constexpr int WPB = 8;
@@ -532,8 +650,26 @@ void launch_qmatmul_q6k_q8k(const uint8_t* w, const uint8_t* xq, float* y, int M
             hipLaunchKernelGGL((k_q6k_q8k_gemv_span<1, WPB>), grid, dim3(64 * WPB), 0, s, w, xq, y, M);
         return;
     }
-    constexpr int R = 2, WPB = 4;
+    constexpr int WPB = 4;
     const int nb = K / 256;
+    // More than one pass a row and x records that fit in 64 KB of LDS (K <= 23,296): the
+    // stream, two rows per wave where that leaves 4 waves per SIMD.  us, k_q6k_q8k_gemv in
+    // brackets (reference / GGUF map): 25296x3072 16.4 (22.1 / 20.8), 10720x2560 8.9 (12.5 /
+    // 10.5), 3072x9216 8.1 (17.9 / 13.2), 5120x13824 15.6 (26.6 / 20.9), 32000x5120 28.2
+    // (37.2 / 38.5), 33x2304 3.0 (4.2 / 3.0), 33x11008 4.8 (9.8 / 6.0); one row against two:
+    // 3072x9216 8.1 (9.1), 25296x3072 19.6 (16.4).  One pass a row: 8192x2048 6.1 (5.2), so
+    // k_q6k_q8k_gemv keeps K = 2048 and below.
+    if (nb > 8 && q6_stream_lds(nb, WPB) <= 64 * 1024) {
+        const int rpw = M >= 8192 ? 2 : 1, rows = rpw * WPB;
+        const dim3 grid((M + rows - 1) / rows);
+        const size_t lds = q6_stream_lds(nb, WPB);
+        if (order == 0)
+            hipLaunchKernelGGL((k_q6k_q8k_gemv_stream<0, WPB>), grid, dim3(64 * WPB), lds, s, w, xq, y, M, nb, rpw);
+        else
+            hipLaunchKernelGGL((k_q6k_q8k_gemv_stream<1, WPB>), grid, dim3(64 * WPB), lds, s, w, xq, y, M, nb, rpw);
+        return;
+    }
+    constexpr int R = 2;
     const int waves = (M + R - 1) / R;
     const dim3 grid((waves + WPB - 1) / WPB);
     if (order == 0)

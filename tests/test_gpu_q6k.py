@@ -60,3 +60,23 @@ def test_q6k_empty_and_k0(dev):
     gpu.qmatmul_q6k_q8k(_d(np.zeros(2, np.uint8), dev), _d(np.zeros(4, np.uint8), dev), 3, 0, out=y)
     torch.cuda.synchronize()
     assert np.array_equal(to_np(y), np.zeros(3, np.float32))
+
+
+@pytest.mark.parametrize("order,o", ORDERS)
+@pytest.mark.parametrize("M,K,off", [(5, 2304, 0),      # a second pass of one super-block
+                                     (9, 3840, 6),      # ... of 7, W off the 4-byte grid
+                                     (7, 4096, 2),      # whole passes, W off the 16-byte grid
+                                     (8195, 2560, 0),   # two rows per wave, the last wave with one
+                                     (1030, 4352, 4),   # three passes
+                                     (3, 23296, 0),     # the longest x that stays in LDS
+                                     (3, 23552, 0)])    # the first that does not
+def test_qmatmul_q6k_q8k_stream(dev, order, o, M, K, off):
+    """The general-K kernel at the edges of its passes, rows and LDS."""
+    import torch
+
+    w = q6k_blocks(M * K // 256, M + K)
+    buf = torch.zeros(w.size + 16, dtype=torch.uint8, device=dev)
+    buf[off:off + w.size] = _d(w, dev)
+    xq = gpu.quant_q8_k(_d(synth.normal_f32(K, synth.key(70, K)), dev))
+    y = to_np(gpu.qmatmul_q6k_q8k(buf[off:off + w.size], xq, M, K, order))
+    assert_bits_equal(y, O.qmatmul_q6k_q8k(w, to_np(xq), M, K, o, nthreads=8), f"q6k gemv order {o} {M}x{K} +{off}")
