@@ -756,37 +756,8 @@ __device__ __forceinline__ void gemv4_rows(const uint8_t* __restrict__ w, const 
     }
 }
 
-// KIND 0: gemv_rows (8 lanes per super-block), KIND 1: gemv4_rows.
-template <int KIND, int R, int G>
-struct PassW;
-template <int R, int G>
-struct PassW<0, R, G> { using type = WideW<R, G>; };
-template <int R, int G>
-struct PassW<1, R, G> { using type = FourW<R>; };
-
-template <int KIND, int R, int G>
-__device__ __forceinline__ void load_first(typename PassW<KIND, R, G>::type& W, const uint8_t* __restrict__ w, int M,
-                                           int nb, int row0) {
-    if constexpr (KIND == 0) {
-#pragma unroll
-        for (int g = 0; g < G; g++) wide_load_g<R, G>(W, g, w, M, nb, row0, 0);
-    } else {
-        four_load<R>(W, w, M, nb, row0, 0);
-    }
-}
-
-template <int KIND, int ORDER, int R, int G, bool LX = false, bool PRE = false>
-__device__ __forceinline__ void rows(const uint8_t* __restrict__ w, const uint8_t* __restrict__ xsrc,
-                                     float* __restrict__ y, int M, int nb, int row0,
-                                     const typename PassW<KIND, R, G>::type& pre) {
-    if constexpr (KIND == 0)
-        gemv_rows<ORDER, R, G, LX, PRE>(w, xsrc, y, M, nb, row0, pre);
-    else
-        gemv4_rows<ORDER, R, LX, PRE>(w, xsrc, y, M, nb, row0, pre);
-}
-
 // R rows per wave, WPB waves per workgroup.
-template <int KIND, int ORDER, int R, int G, int WPB>
+template <int ORDER, int R, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_gemv(const uint8_t* __restrict__ w,
                                                            const uint8_t* __restrict__ xq, float* __restrict__ y,
                                                            int M, int nb) {
@@ -794,8 +765,8 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_gemv(const uint8_t* __rest
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int row0 = (xcd_major(blockIdx.x, gridDim.x) * WPB + wave) * R;
     if (row0 >= M) return;
-    typename PassW<KIND, R, G>::type unused;
-    rows<KIND, ORDER, R, G>(w, xq, y, M, nb, row0, unused);
+    FourW<R> unused;
+    gemv4_rows<ORDER, R, false, false>(w, xq, y, M, nb, row0, unused);
 }
 
 // ----------------------------------------------------------------------------
@@ -812,8 +783,7 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_gemv(const uint8_t* __rest
 // decode and the fp32 combine are shared by 4 lanes.  Passes run row by row,
 // each as soon as the loads holding it are in.  Operands, integer sums, the
 // valid-block rule and the fp32 order are gemv4_rows's (and so gemv_rows's):
-// the bits are the same.  Weights must be 16-byte aligned (rows are then too:
-// 144*NB is a multiple of 16 for even NB).
+// the bits are the same.  Weights must be 16-byte aligned (rows are then too).
 // Measured at 14336x4096 (graph of back-to-back launches over weights beyond
 // the MALL): 6.73 us against 7.36 for gemv_rows with per-lane chunk loads; the
 // same span in gemv_rows's 8-lane mapping 6.98.
@@ -867,22 +837,24 @@ __device__ __forceinline__ void span_issue(u32x4v (&v)[S::kLoads], const uint8_t
 // before the span loads: the first pass then waits for no weight bytes it does
 // not use).
 template <int ORDER, int NB>
-__device__ __forceinline__ void span_load_x(XOps (&xr)[(NB + 15) / 16][2], const uint8_t* __restrict__ xq) {
+__device__ __forceinline__ void span_load_x(XOps (&xr)[(NB + 15) / 16][2], const uint8_t* __restrict__ xq,
+                                            int nb = NB) {
     const int lane = threadIdx.x & 63, bl = lane >> 2, c4 = lane & 3;
 #pragma unroll
     for (int t = 0; t < (NB + 15) / 16; t++) {
-        const uint8_t* xb = xq + (int64_t)min(16 * t + bl, NB - 1) * kQ8KBytes;
+        const uint8_t* xb = xq + (int64_t)min(16 * t + bl, nb - 1) * kQ8KBytes;
         xr[t][0] = load_x<ORDER>(xb, c4);
         xr[t][1] = load_x<ORDER>(xb, c4 + 4);
     }
 }
 
 // The R row results (wave-uniform) from the staged loads; x from xr (LX false)
-// or from the workgroup's LDS copy xl (LX true).
+// or from the workgroup's LDS copy xl (LX true).  nb < NB super-blocks a row: each row a
+// segment of its own (not JOINT) with 9 nb pieces.
 template <int ORDER, int NB, int R, bool JOINT, bool LX, bool PB = false>
 __device__ __forceinline__ void span_rows(const u32x4v (&v)[Span<NB, R, JOINT, PB>::kLoads],
                                           uint8_t* __restrict__ slot, const uint8_t* __restrict__ xl,
-                                          const XOps (&xr)[(NB + 15) / 16][2], float (&out)[R]) {
+                                          const XOps (&xr)[(NB + 15) / 16][2], float (&out)[R], int nb = NB) {
     using S = Span<NB, R, JOINT, PB>;
     const int lane = threadIdx.x & 63, bl = lane >> 2, c4 = lane & 3;
     float s[R];
@@ -893,7 +865,8 @@ __device__ __forceinline__ void span_rows(const u32x4v (&v)[Span<NB, R, JOINT, P
     for (int r = 0; r < R; r++) {
 #pragma unroll
         for (int t = 0; t < S::kNT; t++) {
-            const int b = 16 * t + bl, bb = min(b, NB - 1);
+            if (16 * t >= nb) break;
+            const int b = 16 * t + bl, bb = min(b, nb - 1);
             const uint8_t* blk;
             if constexpr (PB) {
                 // the pass's pieces, in order, from the loads of its segment that hold
@@ -930,8 +903,8 @@ __device__ __forceinline__ void span_rows(const u32x4v (&v)[Span<NB, R, JOINT, P
             uint32_t c_lo = __float_as_uint(c), c_hi = c_lo;
             swap32(c_lo, c_hi);  // lanes 0-31: c_hi = contribution of block b+8
             float acc = s[r];
-            if (b < NB) acc = acc + c;
-            if (b + 8 < NB) acc = acc + __uint_as_float(c_hi);
+            if (b < nb) acc = acc + c;
+            if (b + 8 < nb) acc = acc + __uint_as_float(c_hi);
             // this pass's arithmetic is done before the next pass's LDS writes, which
             // wait for their loads: without this the compiler hoists those writes
             // (and their vmcnt waits) above it, and every pass waits for every load
@@ -950,25 +923,43 @@ __device__ __forceinline__ void span_rows(const u32x4v (&v)[Span<NB, R, JOINT, P
     }
 }
 
-// Single matrix, R consecutive rows per wave, x as Q8_K in global memory.
-template <int ORDER, int NB, int R, int WPB>
+// The segments of R rows from row0 of a matrix of M (rows past the end repeat the last
+// piece or row; their results are not stored).
+template <int NB, int R, bool JOINT>
+__device__ __forceinline__ void span_segs(const uint8_t* (&seg)[JOINT ? 1 : R], int (&np)[JOINT ? 1 : R],
+                                          const uint8_t* w, int row0, int M, int nb) {
+    if constexpr (JOINT) {
+        seg[0] = w + (int64_t)row0 * (NB * kQ4KBytes);
+        np[0] = min(R, M - row0) * NB * 9;
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            seg[r] = w + (int64_t)min(row0 + r, M - 1) * (nb * kQ4KBytes);
+            np[r] = nb * 9;
+        }
+    }
+}
+
+// Single matrix, R consecutive rows per wave, x as Q8_K in global memory.  JOINT: nb == NB.
+template <int ORDER, int NB, int R, bool JOINT, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_gemv_span(const uint8_t* __restrict__ w,
                                                                 const uint8_t* __restrict__ xq,
-                                                                float* __restrict__ y, int M) {
-    using S = Span<NB, R, true>;
+                                                                float* __restrict__ y, int M, int nbr) {
+    using S = Span<NB, R, JOINT>;
+    const int nb = JOINT ? NB : nbr;
     __shared__ __align__(16) uint8_t slots[WPB][S::kSlot];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int row0 = (xcd_major(blockIdx.x, gridDim.x) * WPB + wave) * R;
     if (row0 >= M) return;
     XOps xr[S::kNT][2];
-    span_load_x<ORDER, NB>(xr, xq);
-    // rows past M repeat the last piece of row M-1 (their results are not stored)
-    const uint8_t* seg[1] = {w + (int64_t)row0 * (NB * kQ4KBytes)};
-    const int np[1] = {min(R, M - row0) * NB * 9};
+    span_load_x<ORDER, NB>(xr, xq, nb);
+    const uint8_t* seg[S::kSegs];
+    int np[S::kSegs];
+    span_segs<NB, R, JOINT>(seg, np, w, row0, M, nb);
     u32x4v v[S::kLoads];
     span_issue<S>(v, seg, np);
     float out[R];
-    span_rows<ORDER, NB, R, true, false>(v, slots[wave], nullptr, xr, out);
+    span_rows<ORDER, NB, R, JOINT, false>(v, slots[wave], nullptr, xr, out, nb);
 #pragma unroll
     for (int r = 0; r < R; r++)
         if ((threadIdx.x & 63) == 0 && row0 + r < M) y[row0 + r] = out[r];
@@ -988,7 +979,7 @@ struct MultiArgs {
     int rows;  // total rows
 };
 
-template <int KIND, int ORDER, int R, int G, int WPB>
+template <int ORDER, int R, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_gemv_multi(MultiArgs a, const uint8_t* __restrict__ xq, int nb) {
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int gw = xcd_major(blockIdx.x, gridDim.x) * WPB + wave;
@@ -999,59 +990,49 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_gemv_multi(MultiArgs a, co
     if (gw >= a.first[kMulti]) return;
     const int row0 = (gw - a.first[i]) * R;
     if (row0 >= a.M[i]) return;
-    typename PassW<KIND, R, G>::type unused;
-    rows<KIND, ORDER, R, G>(a.w[i], xq, a.y[i], a.M[i], nb, row0, unused);
+    FourW<R> unused;
+    gemv4_rows<ORDER, R, false, false>(a.w[i], xq, a.y[i], a.M[i], nb, row0, unused);
 }
 
-// Launch shapes, measured on MI355X (one graph of back-to-back launches over
-// weights that do not fit the MALL):
-//   kWide  8 lanes/block, 2 rows x 2 block-groups per wave, 4 waves: best for
-//          many short rows (14336x4096: 7.37 us vs 7.75 for k4Row2)
-//   k4Row1 4 lanes/block, 1 row per wave, 8 waves: best up to ~8K rows of
-//          K <= 4096 (4096x4096: 3.87 us vs 4.00; 1024x4096: 2.85 vs 3.05)
-//   k4Row2 4 lanes/block, 2 rows per wave, 4 waves: best for long rows
-//          (4096x14336: 8.13 us vs 8.57)
-enum GemvShape { kWide, k4Row1, k4Row2 };
-
-static GemvShape choose_shape(int rows, int nb) {
-    if (nb > 16) return k4Row2;
-    return rows <= 8192 ? k4Row1 : kWide;
-}
-
-static int shape_rows_per_wave(GemvShape sh) { return sh == k4Row1 ? 1 : 2; }
-
-template <int KIND, int ORDER, int R, int G, int WPB>
+// K > 4096 (and the empty row): 4 lanes per block, 2 rows per wave, 4 waves (4096x14336:
+// 8.13 us against 8.57 with one row per wave and 8 waves).
+template <int ORDER>
 static void launch_gemv(const uint8_t* w, const uint8_t* xq, float* y, int M, int nb, hipStream_t s) {
+    constexpr int R = 2, WPB = 4;
     const int waves = (M + R - 1) / R;
-    hipLaunchKernelGGL((k_q4k_q8k_gemv<KIND, ORDER, R, G, WPB>), dim3((waves + WPB - 1) / WPB), dim3(64 * WPB), 0,
-                       s, w, xq, y, M, nb);
+    hipLaunchKernelGGL((k_q4k_q8k_gemv<ORDER, R, WPB>), dim3((waves + WPB - 1) / WPB), dim3(64 * WPB), 0, s, w, xq, y, M,
+                       nb);
 }
 
-// Span kernels where they apply (K = 4096, 16-byte aligned weights): two rows
-// per wave, one up to 2048 rows (measured: 4096x4096 3.54 us against 3.85 for
-// k4Row1, 1024x4096 2.40 against 2.86), 4 waves per workgroup.
-static bool span16(int nb, const void* w) { return nb == 16 && (reinterpret_cast<uintptr_t>(w) & 15) == 0; }
+// Span kernels where they apply (K <= 4096, 16-byte aligned weights): two rows
+// per wave, one up to 2048 rows (measured: 4096x4096 3.54 us against 3.85 without
+// spans, 1024x4096 2.40 against 2.86), 4 waves per workgroup.  Below K = 4096 every row is
+// a segment of its own, so the lanes' pieces need no division by the row length, and the
+// loads past a row's pieces repeat its last one: 32000x2048 9.6 us (12.5 without spans),
+// 15456x2560 5.9 (7.5), 25296x3072 8.8 (10.6), 8192x3584 4.4 (4.9), 1001x1024 2.3 (2.3).
+static bool span_fits(int nb) { return nb >= 1 && nb <= 16; }
 static int span_rows_per_wave(int rows) { return rows <= 2048 ? 1 : 2; }
 
 template <int ORDER, int R>
-static void launch_span(const uint8_t* w, const uint8_t* xq, float* y, int M, hipStream_t s) {
+static void launch_span(const uint8_t* w, const uint8_t* xq, float* y, int M, int nb, hipStream_t s) {
     constexpr int WPB = 4;
-    const int waves = (M + R - 1) / R;
-    hipLaunchKernelGGL((k_q4k_q8k_gemv_span<ORDER, 16, R, WPB>), dim3((waves + WPB - 1) / WPB), dim3(64 * WPB), 0, s,
-                       w, xq, y, M);
+    const dim3 grid(((M + R - 1) / R + WPB - 1) / WPB);
+    if (nb == 16)
+        hipLaunchKernelGGL((k_q4k_q8k_gemv_span<ORDER, 16, R, true, WPB>), grid, dim3(64 * WPB), 0, s, w, xq, y, M, nb);
+    else
+        hipLaunchKernelGGL((k_q4k_q8k_gemv_span<ORDER, 16, R, false, WPB>), grid, dim3(64 * WPB), 0, s, w, xq, y, M, nb);
 }
 
 template <int ORDER>
 static void launch_gemv_order(const uint8_t* w, const uint8_t* xq, float* y, int M, int nb, hipStream_t s) {
-    if (span16(nb, w)) {
-        if (span_rows_per_wave(M) == 1) launch_span<ORDER, 1>(w, xq, y, M, s); else launch_span<ORDER, 2>(w, xq, y, M, s);
+    if (span_fits(nb)) {
+        if (span_rows_per_wave(M) == 1)
+            launch_span<ORDER, 1>(w, xq, y, M, nb, s);
+        else
+            launch_span<ORDER, 2>(w, xq, y, M, nb, s);
         return;
     }
-    switch (choose_shape(M, nb)) {
-        case kWide: launch_gemv<0, ORDER, 2, 2, 4>(w, xq, y, M, nb, s); break;
-        case k4Row1: launch_gemv<1, ORDER, 1, 1, 8>(w, xq, y, M, nb, s); break;
-        case k4Row2: launch_gemv<1, ORDER, 2, 1, 4>(w, xq, y, M, nb, s); break;
-    }
+    launch_gemv<ORDER>(w, xq, y, M, nb, s);
 }
 
 void launch_qmatmul_q4k_q8k(const uint8_t* w, const uint8_t* xq, float* y, int M, int K, int order, hipStream_t s) {
@@ -1062,20 +1043,12 @@ void launch_qmatmul_q4k_q8k(const uint8_t* w, const uint8_t* xq, float* y, int M
         launch_gemv_order<1>(w, xq, y, M, nb, s);
 }
 
-template <int KIND, int ORDER, int R, int G, int WPB>
-static void launch_multi(const MultiArgs& a, const uint8_t* xq, int nb, hipStream_t s) {
-    const int waves = a.first[kMulti];
-    hipLaunchKernelGGL((k_q4k_q8k_gemv_multi<KIND, ORDER, R, G, WPB>), dim3((waves + WPB - 1) / WPB),
-                       dim3(64 * WPB), 0, s, a, xq, nb);
-}
-
 template <int ORDER>
-static void launch_multi_order(const MultiArgs& a, GemvShape sh, const uint8_t* xq, int nb, hipStream_t s) {
-    switch (sh) {
-        case kWide: launch_multi<0, ORDER, 2, 2, 4>(a, xq, nb, s); break;
-        case k4Row1: launch_multi<1, ORDER, 1, 1, 8>(a, xq, nb, s); break;
-        case k4Row2: launch_multi<1, ORDER, 2, 1, 4>(a, xq, nb, s); break;
-    }
+static void launch_multi(const MultiArgs& a, const uint8_t* xq, int nb, hipStream_t s) {
+    constexpr int R = 2, WPB = 4;
+    const int waves = a.first[kMulti];
+    hipLaunchKernelGGL((k_q4k_q8k_gemv_multi<ORDER, R, WPB>), dim3((waves + WPB - 1) / WPB), dim3(64 * WPB), 0, s, a, xq,
+                       nb);
 }
 
 static int total_rows(const int* M, int n) {
@@ -1194,7 +1167,7 @@ __device__ __forceinline__ bool wave_rows(const MultiArgs& a, int gw, int R, int
     return has;
 }
 
-template <int KIND, int ORDER, int R, int G, int WPB, int IT>
+template <int ORDER, int R, int WPB, int IT>
 __global__ __launch_bounds__(64 * WPB) void k_q4k_fused_gemv(MultiArgs a, const float* __restrict__ x, int nb) {
     extern __shared__ __align__(16) uint8_t xl[];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -1202,19 +1175,19 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_fused_gemv(MultiArgs a, const 
     const bool has = wave_rows(a, xcd_major(blockIdx.x, gridDim.x) * WPB + wave, R, i, row0);
     XPre<IT> P;
     x32_load<WPB, IT>(P, x, nb);
-    typename PassW<KIND, R, G>::type pre;
-    load_first<KIND, R, G>(pre, a.w[i], a.M[i], nb, row0);
+    FourW<R> pre;
+    four_load<R>(pre, a.w[i], a.M[i], nb, row0, 0);
     __builtin_amdgcn_sched_barrier(0);
     x32_quantize<WPB, IT>(P, xl, nb);
     __syncthreads();
     if (!has) return;
-    rows<KIND, ORDER, R, G, true, true>(a.w[i], xl, a.y[i], a.M[i], nb, row0, pre);
+    gemv4_rows<ORDER, R, true, true>(a.w[i], xl, a.y[i], a.M[i], nb, row0, pre);
 }
 
-template <int KIND, int ORDER, int R, int G, int WPB, int IT>
+template <int ORDER, int R, int WPB, int IT>
 static void launch_fused(const MultiArgs& a, const float* x, int nb, hipStream_t s) {
     const int waves = a.first[kMulti];
-    hipLaunchKernelGGL((k_q4k_fused_gemv<KIND, ORDER, R, G, WPB, IT>), dim3((waves + WPB - 1) / WPB),
+    hipLaunchKernelGGL((k_q4k_fused_gemv<ORDER, R, WPB, IT>), dim3((waves + WPB - 1) / WPB),
                        dim3(64 * WPB), (size_t)nb * kXS, s, a, x, nb);
 }
 
@@ -1223,65 +1196,57 @@ static void launch_fused(const MultiArgs& a, const float* x, int nb, hipStream_t
 // fp32 x, quantized to Q8_K in LDS as in k_q4k_fused_gemv, and stores
 // y[w] = silu(gate_w) * up_w.  gate_w and up_w are the bits the plain GEMV
 // gives, so y equals the GEMVs followed by bpd_swiglu_fuse_cpu's arithmetic.
-// QX: x is already Q8_K (xq), read from global memory, with no quantization pass.
-template <int ORDER, int G, int WPB, bool QX = false>
+template <int ORDER, int G, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_q4k_fused_swiglu(const uint8_t* __restrict__ wg,
                                                               const uint8_t* __restrict__ wu, float* __restrict__ y,
-                                                              int M, const float* __restrict__ x,
-                                                              const uint8_t* __restrict__ xq, int nb) {
+                                                              int M, const float* __restrict__ x, int nb) {
     extern __shared__ __align__(16) uint8_t xl[];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int row = xcd_major(blockIdx.x, gridDim.x) * WPB + wave;
     const bool has = row < M;
     const int row0 = has ? row : 0;
-    if constexpr (QX) {
-        if (!has) return;
-        WideW<2, G> pre;
+    XPre<1> P;
+    x32_load<WPB, 1>(P, x, nb);
+    WideW<2, G> pre;
 #pragma unroll
-        for (int g = 0; g < G; g++) wide_load_g<2, G, true>(pre, g, wg, M, nb, row0, 0, wu);
-        gemv_rows<ORDER, 2, G, false, true, true>(wg, xq, y, M, nb, row0, pre, wu);
-    } else {
-        XPre<1> P;
-        x32_load<WPB, 1>(P, x, nb);
-        WideW<2, G> pre;
-#pragma unroll
-        for (int g = 0; g < G; g++) wide_load_g<2, G, true>(pre, g, wg, M, nb, row0, 0, wu);
-        __builtin_amdgcn_sched_barrier(0);
-        x32_quantize<WPB, 1>(P, xl, nb);
-        __syncthreads();
-        if (!has) return;
-        gemv_rows<ORDER, 2, G, true, true, true>(wg, xl, y, M, nb, row0, pre, wu);
-    }
+    for (int g = 0; g < G; g++) wide_load_g<2, G, true>(pre, g, wg, M, nb, row0, 0, wu);
+    __builtin_amdgcn_sched_barrier(0);
+    x32_quantize<WPB, 1>(P, xl, nb);
+    __syncthreads();
+    if (!has) return;
+    gemv_rows<ORDER, 2, G, true, true, true>(wg, xl, y, M, nb, row0, pre, wu);
 }
 
 template <int ORDER, int WPB>
 static void launch_swiglu(const uint8_t* wg, const uint8_t* wu, float* y, int M, const float* x, int nb,
                           hipStream_t s) {
     hipLaunchKernelGGL((k_q4k_fused_swiglu<ORDER, 2, WPB>), dim3((M + WPB - 1) / WPB), dim3(64 * WPB),
-                       (size_t)nb * kXS, s, wg, wu, y, M, x, nullptr, nb);
+                       (size_t)nb * kXS, s, wg, wu, y, M, x, nb);
 }
 
 // ----------------------------------------------------------------------------
 // Span forms (see span_rows) of the multi-matrix, fused-quantization and
-// Q8_K gate/up SwiGLU launches, for K = 4096 and 16-byte aligned weights.
+// Q8_K gate/up SwiGLU launches, for K <= 4096 (JOINT: K = 4096) and 16-byte aligned weights.
 // Waves, rows and outputs are numbered as in the kernels above, and so are the
 // bits.
 // ----------------------------------------------------------------------------
-template <int ORDER, int NB, int R, int WPB>
-__global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_multi_span(MultiArgs a, const uint8_t* __restrict__ xq) {
-    using S = Span<NB, R, true>;
+template <int ORDER, int NB, int R, bool JOINT, int WPB>
+__global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_multi_span(MultiArgs a, const uint8_t* __restrict__ xq, int nbr) {
+    using S = Span<NB, R, JOINT>;
+    const int nb = JOINT ? NB : nbr;
     __shared__ __align__(16) uint8_t slots[WPB][S::kSlot];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     int i, row0;
     if (!wave_rows(a, xcd_major(blockIdx.x, gridDim.x) * WPB + wave, R, i, row0)) return;
     XOps xr[S::kNT][2];
-    span_load_x<ORDER, NB>(xr, xq);
-    const uint8_t* seg[1] = {a.w[i] + (int64_t)row0 * (NB * kQ4KBytes)};
-    const int np[1] = {min(R, a.M[i] - row0) * NB * 9};
+    span_load_x<ORDER, NB>(xr, xq, nb);
+    const uint8_t* seg[S::kSegs];
+    int np[S::kSegs];
+    span_segs<NB, R, JOINT>(seg, np, a.w[i], row0, a.M[i], nb);
     u32x4v v[S::kLoads];
     span_issue<S>(v, seg, np);
     float out[R];
-    span_rows<ORDER, NB, R, true, false>(v, slots[wave], nullptr, xr, out);
+    span_rows<ORDER, NB, R, JOINT, false>(v, slots[wave], nullptr, xr, out, nb);
 #pragma unroll
     for (int r = 0; r < R; r++)
         if ((threadIdx.x & 63) == 0 && row0 + r < a.M[i]) a.y[i][row0 + r] = out[r];
@@ -1290,9 +1255,10 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_multi_span(MultiArgs a, co
 // Fused quantization: the workgroup quantizes x into LDS (x32_load /
 // x32_quantize, issued before and run after the span loads), then every wave
 // runs its rows with x from LDS.
-template <int ORDER, int NB, int R, int WPB, bool PB = false>
-__global__ __launch_bounds__(64 * WPB) void k_q4k_fused_span(MultiArgs a, const float* __restrict__ x) {
-    using S = Span<NB, R, true, PB>;
+template <int ORDER, int NB, int R, bool JOINT, int WPB, bool PB = false>
+__global__ __launch_bounds__(64 * WPB) void k_q4k_fused_span(MultiArgs a, const float* __restrict__ x, int nbr) {
+    using S = Span<NB, R, JOINT, PB>;
+    const int nb = JOINT ? NB : nbr;
     constexpr int IT = (NB + 4 * WPB - 1) / (4 * WPB);
     __shared__ __align__(16) uint8_t slots[WPB][S::kSlot];
     __shared__ __align__(16) uint8_t xl[NB * kXS];
@@ -1300,126 +1266,111 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_fused_span(MultiArgs a, const 
     int i, row0;
     const bool has = wave_rows(a, xcd_major(blockIdx.x, gridDim.x) * WPB + wave, R, i, row0);
     XPre<IT> P;
-    x32_load<WPB, IT>(P, x, NB);
-    const uint8_t* seg[1] = {a.w[i] + (int64_t)row0 * (NB * kQ4KBytes)};
-    const int np[1] = {min(R, a.M[i] - row0) * NB * 9};
+    x32_load<WPB, IT>(P, x, nb);
+    const uint8_t* seg[S::kSegs];
+    int np[S::kSegs];
+    span_segs<NB, R, JOINT>(seg, np, a.w[i], row0, a.M[i], nb);
     u32x4v v[S::kLoads];
     span_issue<S>(v, seg, np);
     __builtin_amdgcn_sched_barrier(0);
-    x32_quantize<WPB, IT>(P, xl, NB);
+    x32_quantize<WPB, IT>(P, xl, nb);
     __syncthreads();
     if (!has) return;
     XOps unused[S::kNT][2];
     float out[R];
-    span_rows<ORDER, NB, R, true, true, PB>(v, slots[wave], xl, unused, out);
+    span_rows<ORDER, NB, R, JOINT, true, PB>(v, slots[wave], xl, unused, out, nb);
 #pragma unroll
     for (int r = 0; r < R; r++)
         if ((threadIdx.x & 63) == 0 && row0 + r < a.M[i]) a.y[i][row0 + r] = out[r];
 }
 
 // Gate row r and up row r per wave (two spans) from the Q8_K activation xq,
-// y[r] = silu(gate_r) * up_r (k_q4k_fused_swiglu<..., QX = true>'s bits).
+// y[r] = silu(gate_r) * up_r (k_q4k_fused_swiglu's bits); 2x9216x3072 10.4 us, 11.8 with per-lane chunk loads.
 template <int ORDER, int NB, int WPB>
 __global__ __launch_bounds__(64 * WPB) void k_q4k_swiglu_span(const uint8_t* __restrict__ wg,
                                                              const uint8_t* __restrict__ wu, float* __restrict__ y,
-                                                             int M, const uint8_t* __restrict__ xq) {
+                                                             int M, const uint8_t* __restrict__ xq, int nb) {
     using S = Span<NB, 2, false>;
     __shared__ __align__(16) uint8_t slots[WPB][S::kSlot];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int row = xcd_major(blockIdx.x, gridDim.x) * WPB + wave;
     if (row >= M) return;
     XOps xr[S::kNT][2];
-    span_load_x<ORDER, NB>(xr, xq);
-    const int64_t off = (int64_t)row * (NB * kQ4KBytes);
+    span_load_x<ORDER, NB>(xr, xq, nb);
+    const int64_t off = (int64_t)row * (nb * kQ4KBytes);
     const uint8_t* seg[2] = {wg + off, wu + off};
-    const int np[2] = {NB * 9, NB * 9};
+    const int np[2] = {nb * 9, nb * 9};
     u32x4v v[S::kLoads];
     span_issue<S>(v, seg, np);
     float out[2];
-    span_rows<ORDER, NB, 2, false, false>(v, slots[wave], nullptr, xr, out);
+    span_rows<ORDER, NB, 2, false, false>(v, slots[wave], nullptr, xr, out, nb);
     if ((threadIdx.x & 63) == 0) y[row] = silu_mul(out[0], out[1]);
 }
 
-static bool all_aligned16(const uint8_t* const* w, int n) {
-    for (int i = 0; i < n; i++)
-        if (reinterpret_cast<uintptr_t>(w[i]) & 15) return false;
-    return true;
-}
-
 template <int ORDER, int R>
-static void launch_multi_span(const MultiArgs& a, const uint8_t* xq, hipStream_t s) {
+static void launch_multi_span(const MultiArgs& a, const uint8_t* xq, int nb, hipStream_t s) {
     constexpr int WPB = 4;
-    const int waves = a.first[kMulti];
-    hipLaunchKernelGGL((k_q4k_q8k_multi_span<ORDER, 16, R, WPB>), dim3((waves + WPB - 1) / WPB), dim3(64 * WPB), 0,
-                       s, a, xq);
+    const dim3 grid((a.first[kMulti] + WPB - 1) / WPB);
+    if (nb == 16)
+        hipLaunchKernelGGL((k_q4k_q8k_multi_span<ORDER, 16, R, true, WPB>), grid, dim3(64 * WPB), 0, s, a, xq, nb);
+    else
+        hipLaunchKernelGGL((k_q4k_q8k_multi_span<ORDER, 16, R, false, WPB>), grid, dim3(64 * WPB), 0, s, a, xq, nb);
 }
 
 void launch_qmatmul_q4k_q8k_multi(const uint8_t* const* w, float* const* y, const int* M, int n, const uint8_t* xq,
                                   int K, int order, hipStream_t s) {
     const int nb = K / 256;
-    if (nb == 16 && all_aligned16(w, n)) {
+    if (span_fits(nb)) {
         const int R = span_rows_per_wave(total_rows(M, n));
         const MultiArgs a = make_multi_args(w, y, M, n, R);
         if (a.first[kMulti] == 0) return;
         if (order == 0)
-            R == 1 ? launch_multi_span<0, 1>(a, xq, s) : launch_multi_span<0, 2>(a, xq, s);
+            R == 1 ? launch_multi_span<0, 1>(a, xq, nb, s) : launch_multi_span<0, 2>(a, xq, nb, s);
         else
-            R == 1 ? launch_multi_span<1, 1>(a, xq, s) : launch_multi_span<1, 2>(a, xq, s);
+            R == 1 ? launch_multi_span<1, 1>(a, xq, nb, s) : launch_multi_span<1, 2>(a, xq, nb, s);
         return;
     }
-    const GemvShape sh = choose_shape(total_rows(M, n), nb);
-    const MultiArgs a = make_multi_args(w, y, M, n, shape_rows_per_wave(sh));
+    const MultiArgs a = make_multi_args(w, y, M, n, 2);
     if (a.first[kMulti] == 0) return;
     if (order == 0)
-        launch_multi_order<0>(a, sh, xq, nb, s);
+        launch_multi<0>(a, xq, nb, s);
     else
-        launch_multi_order<1>(a, sh, xq, nb, s);
+        launch_multi<1>(a, xq, nb, s);
 }
 
 // Gate and up from a Q8_K activation (K <= 4096), as launch_qmatmul_q4k_fused_swiglu
 // computes them after quantizing.
 template <int ORDER>
-static void launch_swiglu_span(const uint8_t* wg, const uint8_t* wu, float* y, int M, const uint8_t* xq,
+static void launch_swiglu_span(const uint8_t* wg, const uint8_t* wu, float* y, int M, const uint8_t* xq, int nb,
                                hipStream_t s) {
     constexpr int WPB = 4;
     hipLaunchKernelGGL((k_q4k_swiglu_span<ORDER, 16, WPB>), dim3((M + WPB - 1) / WPB), dim3(64 * WPB), 0, s, wg, wu, y,
-                       M, xq);
+                       M, xq, nb);
 }
 
 void launch_qmatmul_q4k_swiglu_q8k(const uint8_t* wg, const uint8_t* wu, float* y, int M, const uint8_t* xq, int K,
                                    int order, hipStream_t s) {
     const int nb = K / 256;
-    const uint8_t* wgu[2] = {wg, wu};
-    if (nb == 16 && all_aligned16(wgu, 2)) {
-        if (order == 0) launch_swiglu_span<0>(wg, wu, y, M, xq, s); else launch_swiglu_span<1>(wg, wu, y, M, xq, s);
-        return;
-    }
     if (order == 0)
-        hipLaunchKernelGGL((k_q4k_fused_swiglu<0, 2, 4, true>), dim3((M + 3) / 4), dim3(256), 0, s, wg, wu, y, M,
-                           nullptr, xq, nb);
+        launch_swiglu_span<0>(wg, wu, y, M, xq, nb, s);
     else
-        hipLaunchKernelGGL((k_q4k_fused_swiglu<1, 2, 4, true>), dim3((M + 3) / 4), dim3(256), 0, s, wg, wu, y, M,
-                           nullptr, xq, nb);
+        launch_swiglu_span<1>(wg, wu, y, M, xq, nb, s);
 }
 
-// One quantization pass covers 4*WPB blocks: 4 waves up to K = 4096, 16 up to
-// fused_max_k().
+// K > 4096 (a shorter row comes as Q8_K).  One quantization pass covers 4*WPB blocks: 16
+// waves up to fused_max_k().
 void launch_qmatmul_q4k_fused_swiglu(const uint8_t* wg, const uint8_t* wu, float* y, int M, const float* x, int K,
                                      int order, hipStream_t s) {
     const int nb = K / 256;
-    if (nb <= 16) {
-        if (order == 0) launch_swiglu<0, 4>(wg, wu, y, M, x, nb, s); else launch_swiglu<1, 4>(wg, wu, y, M, x, nb, s);
-    } else {
-        if (order == 0) launch_swiglu<0, 16>(wg, wu, y, M, x, nb, s); else launch_swiglu<1, 16>(wg, wu, y, M, x, nb, s);
-    }
+    if (order == 0)
+        launch_swiglu<0, 16>(wg, wu, y, M, x, nb, s);
+    else
+        launch_swiglu<1, 16>(wg, wu, y, M, x, nb, s);
 }
 
-// Fused shapes, measured on MI355X for the decode-chain GEMVs (one graph of
-// back-to-back launches, weights beyond the MALL): K <= 4096 takes the 8-lane
-// kernel with 4 waves (QKV 6144x4096: 5.14 us vs 5.44 for k4Row1; O 4096x4096:
-// 4.36 vs 4.40; gate+up 2x14336x4096: 14.24), longer rows the 4-lane kernel
-// with one row per wave and 16 waves (4096x14336: 9.20 us vs 9.50 for 2 rows x
-// 8 waves).  IT = 1: 4*WPB Q8_K blocks per quantization pass cover nb.
+// K > 4096 outside the span forms: the 4-lane kernel with one row per wave and 16 waves
+// (4096x14336: 9.20 us vs 9.50 for 2 rows x 8 waves).  IT = 1: 4*WPB Q8_K blocks per
+// quantization pass cover nb.
 int fused_max_k() { return 64 * 256; }
 
 // K = 4096: 4 waves per workgroup; from 16,384 rows (gate + up) 8 waves with the
@@ -1427,53 +1378,71 @@ int fused_max_k() { return 64 * 256; }
 // gate+up 2x14336 12.98 us against 13.35; Q/K/V and O 4.9 and 4.1 us against 5.4
 // and 4.3 with 8 waves).
 template <int ORDER, int R>
-static void launch_fused_span(const MultiArgs& a, const float* x, hipStream_t s) {
+static void launch_fused_span(const MultiArgs& a, const float* x, int nb, hipStream_t s) {
     const int waves = a.first[kMulti];
-    if (R == 2 && a.rows >= 16384) {
-        constexpr int WPB = 8;
-        hipLaunchKernelGGL((k_q4k_fused_span<ORDER, 16, 2, WPB, true>), dim3((waves + WPB - 1) / WPB), dim3(64 * WPB),
-                           0, s, a, x);
-        return;
-    }
     constexpr int WPB = 4;
-    hipLaunchKernelGGL((k_q4k_fused_span<ORDER, 16, R, WPB>), dim3((waves + WPB - 1) / WPB), dim3(64 * WPB), 0, s, a,
-                       x);
+    const dim3 grid((waves + WPB - 1) / WPB);
+    if (nb != 16) {
+        hipLaunchKernelGGL((k_q4k_fused_span<ORDER, 16, R, false, WPB>), grid, dim3(64 * WPB), 0, s, a, x, nb);
+    } else if (R == 2 && a.rows >= 16384) {
+        constexpr int W8 = 8;
+        hipLaunchKernelGGL((k_q4k_fused_span<ORDER, 16, 2, true, W8, true>), dim3((waves + W8 - 1) / W8), dim3(64 * W8), 0,
+                           s, a, x, nb);
+    } else {
+        hipLaunchKernelGGL((k_q4k_fused_span<ORDER, 16, R, true, WPB>), grid, dim3(64 * WPB), 0, s, a, x, nb);
+    }
+}
+
+// Longer rows up to K = 14336: one row per wave through a pass buffer, in workgroups of 8
+// waves.  From 257 to 511 of those some CUs run two and others one, and the 16-wave general
+// kernel is the faster one; us, that kernel in brackets: 1001x4352 4.2 (5.1), 2048x5632 4.2
+// (5.4), 33x8192 3.7 (4.8); 2560x8704 7.7 (6.4), 3072x9216 8.0 (7.0); 8192x8192 9.8 (10.4),
+// 5120x13824 13.2 (14.8).  (16 waves here as well: 2048x5632 5.3, 5120x13824 16.0.)
+static bool fused_span_long_fits(int rows, int nb) {
+    return nb > 16 && nb <= 56 && (rows <= 2048 || rows >= 4096 || nb == 56);
+}
+
+template <int ORDER>
+static void launch_fused_span_long(const MultiArgs& a, const float* x, int nb, hipStream_t s) {
+    constexpr int WPB = 8;
+    const dim3 grid((a.first[kMulti] + WPB - 1) / WPB);
+    if (nb == 56)
+        hipLaunchKernelGGL((k_q4k_fused_span<ORDER, 56, 1, true, WPB, true>), grid, dim3(64 * WPB), 0, s, a, x, nb);
+    else if (nb > 32)
+        hipLaunchKernelGGL((k_q4k_fused_span<ORDER, 56, 1, false, WPB, true>), grid, dim3(64 * WPB), 0, s, a, x, nb);
+    else
+        hipLaunchKernelGGL((k_q4k_fused_span<ORDER, 32, 1, false, WPB, true>), grid, dim3(64 * WPB), 0, s, a, x, nb);
 }
 
 void launch_qmatmul_q4k_fused_multi(const uint8_t* const* w, float* const* y, const int* M, int n, const float* x,
                                     int K, int order, hipStream_t s) {
     const int nb = K / 256;
-    if (nb == 16 && all_aligned16(w, n)) {
+    if (span_fits(nb)) {
         const int R = span_rows_per_wave(total_rows(M, n));
         const MultiArgs a = make_multi_args(w, y, M, n, R);
         if (a.first[kMulti] == 0) return;
         if (order == 0)
-            R == 1 ? launch_fused_span<0, 1>(a, x, s) : launch_fused_span<0, 2>(a, x, s);
+            R == 1 ? launch_fused_span<0, 1>(a, x, nb, s) : launch_fused_span<0, 2>(a, x, nb, s);
         else
-            R == 1 ? launch_fused_span<1, 1>(a, x, s) : launch_fused_span<1, 2>(a, x, s);
+            R == 1 ? launch_fused_span<1, 1>(a, x, nb, s) : launch_fused_span<1, 2>(a, x, nb, s);
         return;
     }
-    if (nb == 56 && all_aligned16(w, n)) {  // K = 14336: one row per wave through a pass buffer
-        constexpr int WPB = 8;
+    if (fused_span_long_fits(total_rows(M, n), nb)) {
         const MultiArgs a = make_multi_args(w, y, M, n, 1);
         if (a.first[kMulti] == 0) return;
-        const dim3 grid((a.first[kMulti] + WPB - 1) / WPB);
         if (order == 0)
-            hipLaunchKernelGGL((k_q4k_fused_span<0, 56, 1, WPB, true>), grid, dim3(64 * WPB), 0, s, a, x);
+            launch_fused_span_long<0>(a, x, nb, s);
         else
-            hipLaunchKernelGGL((k_q4k_fused_span<1, 56, 1, WPB, true>), grid, dim3(64 * WPB), 0, s, a, x);
+            launch_fused_span_long<1>(a, x, nb, s);
         return;
     }
-    const bool wide = nb <= 16;
-    const MultiArgs a = make_multi_args(w, y, M, n, wide ? 2 : 1);
+    const MultiArgs a = make_multi_args(w, y, M, n, 1);
     if (a.first[kMulti] == 0) return;
-    if (order == 0) {
-        if (wide) launch_fused<0, 0, 2, 2, 4, 1>(a, x, nb, s); else launch_fused<1, 0, 1, 1, 16, 1>(a, x, nb, s);
-    } else {
-        if (wide) launch_fused<0, 1, 2, 2, 4, 1>(a, x, nb, s); else launch_fused<1, 1, 1, 1, 16, 1>(a, x, nb, s);
-    }
+    if (order == 0)
+        launch_fused<0, 1, 16, 1>(a, x, nb, s);
+    else
+        launch_fused<1, 1, 16, 1>(a, x, nb, s);
 }
-
 
 // ----------------------------------------------------------------------------
 // RMSNorm folded into the decode step's GEMVs (n_embd = 4096).  The reference

@@ -224,3 +224,28 @@ def test_qmm_q4k_nan_bits(dev):
     want = O.qmm_q4k(A, B, M, N, K)
     assert np.isnan(want).any()
     assert_bits_equal(to_np(C), want, "bpd_qmm_q4k NaN bits")
+
+
+@pytest.mark.parametrize("Ms,K", [([5], 256),                   # one super-block a row
+                                  ([2049, 3, 0], 512),          # two rows per wave, odd counts, an empty matrix
+                                  ([1001, 7], 3840),            # one row per wave, 15 super-blocks
+                                  ([9], 4352),                  # 17: the long rows' first, a last pass of one
+                                  ([2048], 8192),               # the last of one workgroup per CU
+                                  ([2049], 8448),               # the rows between, on the general kernel
+                                  ([4096, 1], 8448),            # 33 super-blocks on 56 pieces' loads
+                                  ([3, 2], 14080)])             # 55
+def test_span_any_length(dev, Ms, K):
+    """Rows that are not 4096 or 14336 long through the span kernels: the Q8_K and the
+    quantizing product, several matrices in a launch."""
+    import torch
+
+    x = synth.normal_f32(K, synth.key(48, K))
+    xq = O.quant_q8_k(x)
+    W = [synth.q4k(M, K, synth.key(48, i)) if M else np.zeros(16, np.uint8) for i, M in enumerate(Ms)]
+    want = [O.qmatmul_q4k_q8k(w, xq, M, K, formats.ORDER_BPD) if M else np.zeros(0, np.float32) for w, M in zip(W, Ms)]
+    ws = [_dev_u8(w, dev) for w in W]
+    for name, got in (("multi", gpu.qmatmul_q4k_q8k_multi(ws, _dev_u8(xq, dev), Ms, K)),
+                      ("fused", gpu.qmatmul_q4k_q8k_fused_multi(ws, torch.from_numpy(x).to(dev), Ms, K))):
+        for g, w, M in zip(got, want, Ms):
+            if M:
+                assert_bits_equal(to_np(g), w, f"{name} {M}x{K}")
