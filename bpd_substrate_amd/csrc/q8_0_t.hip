@@ -543,6 +543,9 @@ static void launch_tq(const uint8_t* const* W, float* const* out, const int* M, 
 //        per cell and block take).
 // 4 tokens per wave (NQ 1) while 8 would leave SIMDs without a wave: 4096x8 13.8
 // against 17.5, 14336x8 31 against 26.
+// 4 waves of 16-block chunks per workgroup; with 2 waves, 8 waves, 8-block chunks (whole
+// calls, us): 14336x8 30.5 against 32.5, 29.8, 32.5; 8192x8 20.6 against 26.1, 26.5, 22.9;
+// 4096x16 19.7 against 25.5, 26.1, 22.6; 14336x16 53.3 against 55.5, 53.1, 53.0.
 bool launch_q8_0_gemm_T_multi(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq,
                               int m_tokens, int K, hipStream_t s) {
     const int nb = K / 32;
