@@ -29,6 +29,7 @@ HIP_LIB = os.path.join(PKG, "libbpdq_hip.so")
 SYNTH_LIB = os.path.join(PKG, "libbpdq_synth.so")
 
 ARCH = os.environ.get("BPDQ_OFFLOAD_ARCH", "gfx950")
+CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
 
 # -ffp-contract=off: the parity kernels must execute the fp32 operations as
@@ -61,7 +62,8 @@ def hip_sources():
     return sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith(".hip"))
 
 
-def build_hip(verbose=False):
+def compile_hip(verbose=False):
+    """One object per csrc/*.hip in _obj/; their paths."""
     os.makedirs(OBJ, exist_ok=True)
     srcs = hip_sources()
     objs = [os.path.join(OBJ, os.path.basename(s)[:-4] + ".o") for s in srcs]
@@ -72,6 +74,11 @@ def build_hip(verbose=False):
             out = f.result()
             if verbose and out.strip():
                 print(out)
+    return objs
+
+
+def build_hip(verbose=False):
+    objs = compile_hip(verbose)
     tmp = HIP_LIB + ".tmp"
     _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs])
     os.replace(tmp, HIP_LIB)

@@ -1,5 +1,7 @@
 // q8_0_t.hip — Q8_0 x Q8_0 for several activation rows in the AVX1 tile order T
 // (bench/bpd_gemm_q8_0_cpu.c:32-86), on f16 MFMA.
+#include <algorithm>
+
 #include "bpdq_device.h"
 #include "bpdq_launch.h"
 #include "bpdq_q8_0.h"
@@ -508,16 +510,13 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
     }
 }
 
-template <int WRN, int WCN, int CT, int PF>
+template <int WRN, int WCN, int CT, int PF, bool AL>
 static void launch_tm(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq, int m_tokens,
-                      int nb, bool aligned, hipStream_t s) {
+                      int nb, hipStream_t s) {
     using G = TmGeo<WRN, WCN, CT>;
     const GemmW g = gemm_args<G::R>(W, out, M, n);
-    const dim3 grid(g.first[kGemmMulti] * ((m_tokens + G::C - 1) / G::C));
-    if (aligned)
-        hipLaunchKernelGGL((k_q8_0_gemm_TM<WRN, WCN, CT, PF, true>), grid, dim3(G::NT), 0, s, g, Xq, m_tokens, nb);
-    else
-        hipLaunchKernelGGL((k_q8_0_gemm_TM<WRN, WCN, CT, PF, false>), grid, dim3(G::NT), 0, s, g, Xq, m_tokens, nb);
+    hipLaunchKernelGGL((k_q8_0_gemm_TM<WRN, WCN, CT, PF, AL>), dim3(g.first[kGemmMulti] * ((m_tokens + G::C - 1) / G::C)),
+                       dim3(G::NT), 0, s, g, Xq, m_tokens, nb);
 }
 
 template <int NQ, int NW, int CB>
@@ -529,20 +528,29 @@ static void launch_tq(const uint8_t* const* W, float* const* out, const int* M, 
                        dim3(G::NT), 0, s, g, Xq, m_tokens, nb);
 }
 
-// Which kernel, by the cells M * m_tokens (every one costs about the same per block,
-// so K does not enter).  Measured on MI355X at K = 4096, weights beyond the MALL, us
-// per call, the per-token GEMVs they replace in brackets:
-//   TQ   14336x2 18.9 (22.3), 14336x4 19.0 (39.7), 14336x8 26 (73), 4096x4 13.5
-//        (14.1), 4096x8 13.8 (22.7), 4096x16 17.8 (41), 4096x32 25.9 (75);
-//        1024x8 12.6 (7.5: the GEMVs stay below 16,384 cells); K = 4128: 14336x2 23.5
-//        (36), 4096x4 15.4 (20), 4096x2 15.5 (15.7); K = 1440: 5413x3 8.4 (9.7), 1024x4
-//        8.2 (5.4);
-//   TM   32 rows x 64 tokens: 4096x64 45.6 (TQ 48), 4096x128 46.7 (TQ 89), 1024x512
-//        50 (304); 64 x 64: 14336x32 67 (TQ 80), 14336x64 69 (650), 4096x512 137
-//        (1,360), 14336x512 434 (4,890: 84 % of the 382 us that 16 VALU operations
-//        per cell and block take).
-// 4 tokens per wave (NQ 1) while 8 would leave SIMDs without a wave: 4096x8 13.8
-// against 17.5, 14336x8 31 against 26.
+// Which kernel: the least of the estimated times (ns) of the per-token GEMVs and the four
+// forms here.  A launch's workgroups run in n = ceil(workgroups / 256) per CU, whether their
+// rows and tokens are real or padding, and its time is close to fixed + step * n + K * g(n),
+// g the ns per element of K:
+//   TQ<1> 32 rows x 4 tokens    g = max(1.22 + 1.38 n, 1.85 n)
+//   TQ<2> 32 rows x 8 tokens    g = max(1.5 + 1.95 n, 3.3 n - 1.9)
+//   TM    32 rows x 64 tokens   g = 2 + 9 n
+//   TM    64 rows x 64 tokens   g = 16.6 n - 2; not without 4-byte alignment, where 23 n - 2 is
+//                               more than twice the n of 32 rows cost
+// (a first wave per SIMD waits for memory, so the small forms cost more at n = 1 than their
+// share).  The GEMVs (launch_wide) take time by cells: rows * tokens * (0.04 + 1.6e-4 K), less
+// where the rows stay in the L2s between tokens, more where launch_wide does not run.  Fitted
+// to 1,200 shapes on MI355X, weights beyond the MALL (512 to 128256 rows, 2 to 256 tokens,
+// K 1024 to 14336, 1440, 4128 and 8032): the choice is on the average 0.4 % and at most 16 %
+// over the best form, and no shape is slower than the GEMVs.  us, K = 4096, the GEMVs / TQ<1>
+// / TQ<2> / TM 32 / TM 64:
+//   4096x2 8.7 / 14.3 / 17.8; 4096x4 14.1 / 14.5 / 17.9; 4096x8 22.4 / 14.6 / 18.0
+//   8192x2 14.8 / 15.2 / 18.7; 11008x2 18.7 / 20.6 / 26.6; 14336x2 22.3 / 20.6 / 26.9
+//   14336x8 74 / 34 / 30; 32000x2 44 / 37 / 55; 32000x9 184 / 85 / 97 / - / 157
+//   128256x2 175 / 132 / 224 / - / 579; 4096x33 77 / - / 44 / 54 / 61; 14336x33 286 / - / 119 / 86 / 70
+//   4096x512 1,360 / - / - / - / 125;  14336x512 4,890 / - / - / - / 434 (88 % of it the 382 us that 16
+//   VALU operations per cell and block take)
+// Below 16,384 cells the GEMVs stay: 1024x8 7.8 against 14.2.
 // 4 waves of 16-block chunks per workgroup; with 2 waves, 8 waves, 8-block chunks (whole
 // calls, us): 14336x8 30.5 against 32.5, 29.8, 32.5; 8192x8 20.6 against 26.1, 26.5, 22.9;
 // 4096x16 19.7 against 25.5, 26.1, 22.6; 14336x16 53.3 against 55.5, 53.1, 53.0.
@@ -550,23 +558,40 @@ bool launch_q8_0_gemm_T_multi(const uint8_t* const* W, float* const* out, const 
                               int m_tokens, int K, hipStream_t s) {
     const int nb = K / 32;
     bool al4 = nb % 2 == 0 && (reinterpret_cast<uintptr_t>(Xq) & 3) == 0;
+    bool wide = nb % 32 == 0;  // launch_wide takes every matrix
     int64_t rows = 0;
     for (int i = 0; i < n; i++) {
         rows += M[i];
         al4 = al4 && (reinterpret_cast<uintptr_t>(W[i]) & 3) == 0;
+        wide = wide && (reinterpret_cast<uintptr_t>(W[i]) & 15) == 0;
     }
-    if (nb == 0 || m_tokens < 2 || rows * m_tokens < 16384) return false;
-    const int64_t w8 = (rows + 7) / 8 * ((m_tokens + 7) / 8);  // waves of 8 rows x 8 tokens
-    if (w8 <= 4096) {
-        if (w8 < 1024)
-            launch_tq<1, 4, 16>(W, out, M, n, Xq, m_tokens, nb, s);
-        else
-            launch_tq<2, 4, 16>(W, out, M, n, Xq, m_tokens, nb, s);
-    } else if ((rows + 31) / 32 * ((m_tokens + 63) / 64) <= 256) {
-        launch_tm<2, 4, 1, 4>(W, out, M, n, Xq, m_tokens, nb, al4, s);
-    } else {
-        launch_tm<4, 4, 1, 4>(W, out, M, n, Xq, m_tokens, nb, al4, s);
-    }
+    const int64_t cells = rows * m_tokens;
+    if (nb == 0 || m_tokens < 2 || cells < 16384) return false;
+    // workgroups of R rows x C tokens per CU
+    const auto per_cu = [&](int R, int C) {
+        int64_t b = 0;
+        for (int i = 0; i < n; i++) b += (M[i] + R - 1) / R;
+        return (double)((b * ((m_tokens + C - 1) / C) + 255) / 256);
+    };
+    const double k = K, n1 = per_cu(32, 4), n2 = per_cu(32, 8), n3 = per_cu(32, 64), n4 = per_cu(64, 64);
+    const double gemv = 2600.0 * n + (double)cells * (!wide ? 2.6e-4 * k : rows <= 2048 ? 0.03 + 1.35e-4 * k : 0.04 + 1.6e-4 * k);
+    const double tq1 = 3300 + 600 * n1 + k * std::max(1.22 + 1.38 * n1, 1.85 * n1);
+    const double tq2 = 3500 + 600 * n2 + k * std::max(1.5 + 1.95 * n2, 3.3 * n2 - 1.9);
+    const double tm32 = 3000 + 300 * n3 + k * (2 + 9 * n3);
+    const double tm64 = 3000 + 300 * n4 + k * (16.6 * n4 - 2);
+    double least = std::min(std::min(tq1, tq2), tm32);
+    if (al4) least = std::min(least, tm64);
+    if (gemv <= least) return false;
+    if (least == tq1)
+        launch_tq<1, 4, 16>(W, out, M, n, Xq, m_tokens, nb, s);
+    else if (least == tq2)
+        launch_tq<2, 4, 16>(W, out, M, n, Xq, m_tokens, nb, s);
+    else if (least == tm32 && al4)
+        launch_tm<2, 4, 1, 4, true>(W, out, M, n, Xq, m_tokens, nb, s);
+    else if (least == tm32)
+        launch_tm<2, 4, 1, 4, false>(W, out, M, n, Xq, m_tokens, nb, s);
+    else
+        launch_tm<4, 4, 1, 4, true>(W, out, M, n, Xq, m_tokens, nb, s);
     return true;
 }
 

@@ -11,12 +11,12 @@ from test_gpu_q8_0 import _d, _q8_full_range, _q8_nan_heavy
 
 pytestmark = pytest.mark.gpu
 
-CASES = [(4099, 4, 256, 0),      # 4 tokens per wave, a half chunk
+CASES = [(4099, 4, 256, 0),      # the per-token GEMVs still
          (2050, 9, 768, 0),      # 4 tokens per wave, a whole and a half chunk, 3 token groups
          (4100, 13, 1280, 0),    # 8 tokens per wave
-         (703, 65, 224, 0),      # 4 tokens per wave, an odd number of blocks
+         (703, 65, 224, 0),      # 8 tokens per wave, an odd number of blocks
          (4100, 14, 544, 0),     # 8 tokens per wave, a last chunk of one block
-         (8200, 2, 32, 2),       # one block, W off the 4-byte grid
+         (8200, 2, 32, 2),       # the per-token GEMVs, W off the 4-byte grid
          (703, 65, 960, 1),      # 30 blocks, W at an odd address
          (1030, 290, 512, 0),    # 32 x 64 tiles
          (1030, 290, 192, 0),    # ... K % 256 != 0
@@ -24,7 +24,11 @@ CASES = [(4099, 4, 256, 0),      # 4 tokens per wave, a half chunk
          (1030, 290, 256, 2),    # ... W off the 4-byte grid
          (1030, 290, 256, 1),    # ... W at an odd address
          (4100, 300, 128, 0),    # 64 x 64 tiles
-         (4100, 300, 96, 0)]
+         (4100, 300, 96, 0),
+         (2000, 16, 480, 0),     # 4 tokens per wave, one chunk that ends early
+         (1100, 20, 544, 1),     # ... a last chunk of one block, W at an odd address
+         (33000, 3, 768, 0),     # ... several workgroups per CU, a ragged last one
+         (703, 256, 32, 2)]      # 32 x 64 tiles, one block
 
 
 @pytest.mark.parametrize("mw,mt,K,off", CASES)

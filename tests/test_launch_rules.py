@@ -1,0 +1,76 @@
+"""Which kernel the launchers choose, against the times measured for each form.
+
+`launches` records what an entry point launches; the tables hold the microseconds per call of
+every form on MI355X (graphs of back-to-back launches, weights beyond the MALL).  No GPU.
+"""
+import pytest
+
+from launches import Recorder
+
+W, X, OUT = 0x100000, 0x200000, 0x300000  # never read: aligned as a torch tensor is
+
+
+@pytest.fixture(scope="module")
+def launched(tmp_path_factory):
+    return Recorder(str(tmp_path_factory.mktemp("launches")))
+
+
+def one_of(shapes, forms):
+    """The time of the form that a launch belongs to (None: not measured at this shape)."""
+    def f(launch):
+        for form, t in zip(forms, shapes):
+            if form(launch):
+                return t
+        raise AssertionError(f"{launch} is none of the forms")
+    return f
+
+
+# ---------------------------------------------------------------- Q8_0, order T, several rows of X
+
+T_FORMS = [lambda l: l.kernel == "k_q8_0_gemm_TQ" and l.args[0] == 1,
+           lambda l: l.kernel == "k_q8_0_gemm_TQ" and l.args[0] == 2,
+           lambda l: l.kernel == "k_q8_0_gemm_TM" and l.args[0] == 2,
+           lambda l: l.kernel == "k_q8_0_gemm_TM" and l.args[0] == 4,
+           lambda l: l.kernel.startswith("k_q8_0_gemv_")]
+# M, tokens, K, then us of TQ with 4 and 8 tokens, TM with 32 and 64 rows, the per-token GEMVs
+T_US = [
+    (1024, 16, 4096, 14.0, 17.7, None, None, 12.5), (1024, 16, 14336, 39.8, 51.7, None, None, 33.9),
+    (2048, 8, 1024, 6.4, 7.4, None, None, 5.8), (2048, 8, 4096, 14.1, 17.7, None, None, 13.0),
+    (2048, 8, 14336, 40.2, 52.1, None, None, 37.7), (2048, 33, 4096, None, 25.9, 44.8, 57.5, 38.6),
+    (3000, 8, 1024, 6.7, 7.5, None, None, 8.3), (4096, 4, 1024, 6.4, 7.3, None, None, 5.9),
+    (4096, 4, 4096, 14.5, 17.9, None, None, 14.1), (4096, 4, 14336, 40.6, 53.2, None, None, 40.4),
+    (4096, 5, 4096, 14.6, 18.0, None, None, 16.2), (4096, 16, 4096, 19.5, 18.5, None, None, 39.8),
+    (4096, 33, 4096, None, 44.4, 54.3, 60.9, 76.8), (4096, 65, 4096, None, 58.9, 47.6, 60.0, None),
+    (5632, 3, 4096, 14.8, 18.2, None, None, 14.7), (5632, 3, 14336, 40.6, 53.3, None, None, 44.6),
+    (5632, 12, 4096, 23.6, 26.2, None, None, 42.7), (8192, 2, 1024, 7.0, 7.8, None, None, 6.2),
+    (8192, 2, 4096, 15.2, 18.7, None, None, 14.8), (8192, 2, 14336, 43.6, 57.0, None, None, 41.9),
+    (8192, 3, 4096, 15.3, 19.0, None, None, 19.4), (8192, 8, 4096, 20.0, 19.7, None, None, 43.4),
+    (8192, 33, 8032, None, 118.6, 97.7, 167.9, 399.2), (11008, 2, 1024, 9.0, 10.2, None, None, 7.2),
+    (11008, 2, 4096, 20.6, 26.6, None, None, 18.7), (11008, 2, 14336, 60.7, 82.2, None, None, 54.8),
+    (11008, 3, 4096, 20.8, 26.6, None, None, 25.5), (11008, 5, 4096, 25.8, 27.6, None, None, 39.3),
+    (11008, 24, 14336, None, 266.0, 256.3, 215.4, 603.0), (14336, 2, 4096, 20.6, 26.9, None, None, 22.3),
+    (14336, 4, 4096, 20.7, 27.0, None, None, 39.5), (14336, 8, 4096, 34.3, 30.2, None, None, 73.8),
+    (14336, 9, 4096, 46.9, 53.5, None, None, 82.5), (14336, 16, 4096, 66.2, 55.6, None, None, 143.7),
+    (14336, 33, 4096, None, 119.0, 86.3, 69.8, 285.6), (14336, 65, 4128, None, 189.2, 140.5, 171.9, None),
+    (20000, 65, 1440, None, 109.5, 67.2, 88.6, None), (20000, 96, 1440, None, 146.5, 68.2, 89.5, None),
+    (32000, 2, 1024, 14.6, 18.4, None, None, 16.1), (32000, 2, 4096, 37.2, 54.6, None, None, 44.0),
+    (32000, 4, 14336, 119.4, 179.7, None, None, 290.9), (32000, 9, 4096, 84.6, 97.1, None, None, 183.6),
+    (32000, 17, 4096, None, 169.0, 166.2, 140.9, 349.0), (32000, 64, 1440, None, 156.6, 59.0, 70.4, None),
+    (65536, 2, 1440, 33.7, 45.5, None, None, 53.4), (65536, 4, 4096, 67.3, 104.5, None, None, 170.4),
+    (65536, 5, 8032, 236.8, 195.8, None, None, 664.4), (128256, 2, 1024, 39.6, 61.2, None, None, 54.1),
+    (128256, 2, 4096, 132.0, 224.2, None, None, 174.7), (128256, 4, 4096, 133.4, 211.0, None, None, 336.1),
+    (128256, 5, 4096, 267.3, 200.9, None, None, 424.0), (128256, 17, 1440, None, 236.1, 214.2, 262.4, 703.9),
+    (128256, 9, 1024, 107.9, 127.2, None, None, 247.7),
+]
+
+
+@pytest.mark.parametrize("M,T,K,tq1,tq2,tm32,tm64,gemv", T_US)
+def test_order_t_takes_a_measured_fast_form(launched, M, T, K, tq1, tq2, tm32, tm64, gemv):
+    """Within a sixth of the best form measured, and never slower than the per-token GEMVs
+    that take every shape."""
+    l, = launched("bpd_qmatmul_q8_0_dispatch_gpu", W, X, OUT, M, T, K)
+    times = (tq1, tq2, tm32, tm64, gemv)
+    t = one_of(times, T_FORMS)(l)
+    assert t is not None, f"{l}: a form so far off that it was not measured"
+    assert t <= 1.17 * min(x for x in times if x is not None), l
+    assert gemv is None or t <= 1.02 * gemv, l
