@@ -1,5 +1,6 @@
 // q8_0_s.hip — Q8_0 x Q8_0 for few activation rows in the scalar order S
 // (bench/bpd_gemm_q8_0_cpu.c:102-131, bench/bpd_cpu.c:4263-4280), on int8 MFMA.
+#include <algorithm>
 #include <mutex>
 
 #include "bpdq_device.h"
@@ -280,46 +281,75 @@ static bool launch_sq(const uint8_t* const* W, float* const* out, const int* M, 
     return true;
 }
 
-// Which form, or none (the caller then takes k_q8_0_gemm_SH or, where that does not run,
-// k_q8_0_gemm_S).  A workgroup costs about the same however many of its tokens are real
-// and whatever the row count, so the time of a launch is its workgroups per CU times one
-// workgroup's cost; in units of 0.01 us per block: 8, 9, 15 and 24 for 4, 8, 16 tokens x 64
-// rows and 16 x 128; k_q8_0_gemm_SH costs 30 and k_q8_0_gemm_S 110, and 1 more for every 8
-// workgroups of 128 rows.  The cheapest form that fits in LDS is taken if it is cheaper than
-// that.  Measured, us per call, weights beyond the MALL, the other kernel in brackets:
-//   K = 4096   14336x1 15.6 (48), x8 18.8 (46), x16 22-25 (47), x32 31.6 (49; x48 58 against
-//              49: not taken); 4096x1 12.0 (39), x16 13.5 (41), x32 15.3 (41), x64 21.2 (43),
-//              x128 29.5 (44); 28672x8 30 (66); 128256x1 101 (241); 1024x512 29.5 (44)
-//   K = 14336  4096x1 32 (129), 4096x64 90 (143; x100 165 against 150: not taken)
-//   K = 28672  8192x16 137 (281)
-//   K = 1440   5413x3 9.4 (52), 5413x40 12.5 (55), 14336x64 30.4 (57)
-//   K = 3776   325x233 14.3 (134);  K = 8320  1097x17 21.9 (76)
+// Estimated times (ns) of a launch over the rows and tokens of n matrices.  Its workgroups run
+// in `per` = ceil(workgroups / 256) per CU however many of their rows and tokens are real, so
+// it is fixed + step * per + K * g(per), g the ns per element of K: g1 for one workgroup per CU,
+// else gs[o - 1] per workgroup where LDS lets o of them run at once (2.25 against 1.85 for 4
+// tokens, 4.3 against 2.85 for 16, where one has the CU to itself).  An odd number of blocks
+// leaves the rows off the 4-byte grid: `odd` times that.  Fitted to 950 shapes on MI355X, weights
+// beyond the MALL (512 to 128256 rows, 1 to 512 tokens, K 1024 to 28672): the choice is on the
+// average 0.2 % and at most 16 % over the best form, and no shape is more than 4 % slower than
+// k_q8_0_gemm_SH and k_q8_0_gemm_S.  us, 4 / 8 / 16 tokens x 64 rows / 16 x 128 / those two:
+//   K = 1024   32000x8 21 / 13 / 15 / 15 / 20; 32000x17 39 / 28 / 22 / 26 / 20
+//   K = 1440   14336x64 74 / 43 / 32 / 32 / 57
+//   K = 4096   14336x1 17 / 18 / 20 / 27 / 47; 14336x16 40 / 27 / 23 / 32 / 47; 14336x48 95 / 65 / 60 / 60 / 49
+//              4096x64 40 / 27 / 22 / 30 / 43; 128256x1 103 / 108 / 140 / 123 / 230
+//   K = 8192   8192x64 130 / 100 / - / - / 83; 32000x17 207 / 167 / - / - / 128
+struct SqForm {
+    int rows, tokens;
+    double step, g1, gs[3], odd;
+    bool (*launch)(const uint8_t* const*, float* const*, const int*, int, const uint8_t*, int, int, int, hipStream_t);
+};
+static constexpr SqForm kSqForms[] = {{64, 4, 800, 1.85, {2.25, 2.15, 1.85}, 1.55, launch_sq<4, 4>},
+                                      {64, 8, 800, 2.1, {2.85, 2.15, 2.15}, 1.5, launch_sq<8, 4>},
+                                      {64, 16, 800, 2.85, {4.3, 3.4, 2.85}, 1.25, launch_sq<16, 4>},
+                                      {128, 16, 1600, 5.2, {6.5, 6.5, 6.5}, 1.35, launch_sq<16, 8>}};
+
+static int64_t tiles(const int* M, int n, int m_tokens, int rows, int tokens) {
+    int64_t b = 0;
+    for (int i = 0; i < n; i++) b += (M[i] + rows - 1) / rows;
+    return b * ((m_tokens + tokens - 1) / tokens);
+}
+
+static const SqForm* sq_best(const int* M, int n, int m_tokens, int K, double* ns) {
+    const int nb = K / 32;
+    const SqForm* best = nullptr;
+    *ns = 0;
+    for (const SqForm& f : kSqForms) {
+        const size_t lds = sq_lds(f.tokens, f.rows / 16, nb);
+        if (lds > kSqMaxLds) continue;
+        const int at_once = std::min<int>((int)(kSqMaxLds / lds), 3);
+        const double per = (double)((tiles(M, n, m_tokens, f.rows, f.tokens) + 255) / 256);
+        const double g = (per == 1 ? f.g1 : f.gs[at_once - 1] * per) * (nb % 2 != 0 ? f.odd : 1.0);
+        const double t = 4000 + f.step * per + K * g;
+        if (best != nullptr && t >= *ns) continue;
+        best = &f;
+        *ns = t;
+    }
+    return best;
+}
+
+// k_q8_0_gemm_SH (staged) by its three forms, k_q8_0_gemm_S otherwise.
+static double sh_ns(const int* M, int n, int m_tokens, int K, bool staged) {
+    const auto wgs = [&](int rows) { return tiles(M, n, m_tokens, rows, 128); };
+    if (!staged) {
+        const double fixed = m_tokens <= 64 ? 4600 : 8600, g = m_tokens <= 64 ? 32.5 : 36.5;
+        return fixed + K * std::max(g, 0.096 * (double)wgs(128));
+    }
+    const double g = wgs(128) >= 256 ? (wgs(128) <= 512 ? 27.0 : 28.0 * (double)((wgs(128) + 511) / 512))
+                     : wgs(64) >= 256 ? 15.0
+                     : wgs(32) > 256  ? 11.3
+                                      : 9.4;
+    return 3000 + K * g;
+}
+
 bool launch_q8_0_gemm_S_few(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq,
                             int m_tokens, int K, bool staged, int nan_mode, hipStream_t s) {
-    const int nb = K / 32;
-    if (nb == 0) return false;
-    const auto wgs = [&](int rows, int tokens) {
-        int64_t b = 0;
-        for (int i = 0; i < n; i++) b += (M[i] + rows - 1) / rows;
-        return b * ((m_tokens + tokens - 1) / tokens);
-    };
-    struct Form {
-        int rows, tokens, cost;
-        bool (*launch)(const uint8_t* const*, float* const*, const int*, int, const uint8_t*, int, int, int, hipStream_t);
-    };
-    static constexpr Form forms[] = {{64, 4, 8, launch_sq<4, 4>},
-                                     {64, 8, 9, launch_sq<8, 4>},
-                                     {64, 16, 15, launch_sq<16, 4>},
-                                     {128, 16, 24, launch_sq<16, 8>}};
-    int64_t least = (staged ? 30 : 110) + wgs(128, 128) / 8;
-    const Form* form = nullptr;
-    for (const Form& f : forms) {
-        const int64_t cost = (wgs(f.rows, f.tokens) + 255) / 256 * f.cost;
-        if (cost >= least || sq_lds(f.tokens, f.rows / 16, nb) > kSqMaxLds) continue;
-        least = cost;
-        form = &f;
-    }
-    return form != nullptr && form->launch(W, out, M, n, Xq, m_tokens, nb, nan_mode, s);
+    if (K / 32 == 0) return false;
+    double ns;
+    const SqForm* form = sq_best(M, n, m_tokens, K, &ns);
+    if (form == nullptr || ns >= 0.97 * sh_ns(M, n, m_tokens, K, staged)) return false;
+    return form->launch(W, out, M, n, Xq, m_tokens, K / 32, nan_mode, s);
 }
 
 }  // namespace bpdq

@@ -10,10 +10,13 @@ from test_gpu_q8_0 import _d, _q8_full_range, _q8_nan_heavy
 
 pytestmark = pytest.mark.gpu
 
-CASES = [(70, 1, 256, 0, 0),        # 4 tokens per workgroup, half a chunk
+CASES = [(70, 1, 256, 0, 0),        # the kernel for any number of tokens still
+         (70, 1, 480, 0, 0),        # 4 tokens per workgroup, a chunk that ends early
          (130, 3, 512, 0, 1),       # ... one whole chunk, X at an odd address
          (4099, 18, 768, 0, 2),     # 8 tokens, a ragged last tile of rows and of tokens
-         (4100, 50, 1280, 0, 0),    # 16 tokens x 64 rows
+         (4100, 50, 1280, 0, 0),    # ... with several workgroups per CU
+         (8201, 9, 256, 0, 0),      # 16 tokens x 64 rows, half a chunk, a ragged last tile of rows and of tokens
+         (4100, 64, 1440, 2, 1),    # 16 tokens x 128 rows, 45 blocks, W off the 4-byte grid, X at an odd address
          (14340, 17, 1024, 0, 2),   # 16 tokens x 128 rows
          (66, 5, 14336, 0, 0),      # a long K: more than 64 KiB of LDS
          (130, 9, 28672, 0, 0),     # ... that only 4 tokens fit

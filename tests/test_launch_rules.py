@@ -74,3 +74,50 @@ def test_order_t_takes_a_measured_fast_form(launched, M, T, K, tq1, tq2, tm32, t
     assert t is not None, f"{l}: a form so far off that it was not measured"
     assert t <= 1.17 * min(x for x in times if x is not None), l
     assert gemv is None or t <= 1.02 * gemv, l
+
+
+# ---------------------------------------------------------------- Q8_0, order S, few rows of X
+
+def _sq(tokens, waves):
+    return lambda l: l.kernel == "k_q8_0_gemm_SQ" and l.args == [tokens, waves]
+
+
+S_FORMS = [_sq(4, 4), _sq(8, 4), _sq(16, 4), _sq(16, 8), lambda l: l.kernel in ("k_q8_0_gemm_SH", "k_q8_0_gemm_S")]
+# M, tokens, K, then us of SQ with 4, 8 and 16 tokens x 64 rows and 16 x 128 (None: does not fit in
+# LDS), of the kernels for any number of tokens
+S_US = [
+    (32000, 1, 32, 7.8, 7.8, 8.1, 7.8, 6.3), (8192, 200, 64, 44.7, 25.3, 16.5, 19.3, 12.6),
+    (2048, 200, 64, 14.8, 9.3, 6.0, 6.1, 11.9), (70, 1, 256, 4.7, 4.8, 4.9, 5.9, 4.9),
+    (2048, 4, 512, 5.7, 5.6, 5.9, 7.8, 7.8), (512, 16, 1024, 6.8, 6.6, 7.4, 10.5, 12.1),
+    (8192, 17, 1024, 13.1, 9.8, 8.0, 10.6, 12.7), (14336, 24, 1024, 20.6, 14.1, 11.7, 11.4, 14.5),
+    (32000, 8, 1024, 20.8, 13.4, 14.8, 15.0, 19.6), (32000, 17, 1024, 39.3, 28.2, 22.2, 25.7, 19.9),
+    (32000, 32, 1024, 59.2, 35.1, 23.4, 26.2, 21.0), (128256, 16, 1024, 108.2, 64.4, 41.3, 52.4, 63.7),
+    (20000, 32, 1024, 40.5, 25.5, 17.9, 22.8, 19.6), (20000, 128, 1440, 209.5, 116.9, 76.3, 79.7, 64.8),
+    (14336, 64, 1440, 73.8, 42.7, 32.3, 31.6, 57.0), (32000, 64, 1440, 170.0, 96.2, 64.2, 66.9, 62.2),
+    (65536, 48, 1440, 252.1, 143.0, 93.1, 97.8, 85.2), (128256, 32, 1440, 337.6, 194.3, 129.3, 138.5, 153.4),
+    (4096, 200, 1440, 68.3, 41.8, 31.6, 31.0, 62.6), (2932, 197, 1248, 46.6, 28.9, 23.0, 28.1, 52.8),
+    (10304, 152, 1600, 119.1, 69.5, 52.5, 64.3, 67.6), (32000, 16, 2048, 53.7, 33.2, 24.5, 23.8, 36.0),
+    (32000, 24, 2048, 75.5, 46.0, 39.1, 39.7, 36.4), (32000, 32, 2048, 94.9, 58.0, 40.8, 41.0, 37.0),
+    (25856, 96, 2336, 274.0, 163.4, 109.3, 109.4, 95.4), (4096, 1, 4096, 13.6, 14.7, 17.6, 26.4, 40.5),
+    (4096, 64, 4096, 39.6, 26.8, 22.2, 30.3, 42.6), (14336, 1, 4096, 16.8, 17.7, 19.5, 27.3, 46.5),
+    (14336, 16, 4096, 39.7, 27.2, 23.3, 31.5, 47.0), (14336, 48, 4096, 95.0, 64.8, 59.9, 60.0, 48.5),
+    (8192, 96, 4096, 100.1, 62.9, 58.1, 57.1, 45.3), (32000, 17, 4096, 110.1, 76.7, 76.5, 63.4, 66.1),
+    (128256, 1, 4096, 102.8, 108.3, 139.6, 123.5, 229.8), (13928, 25, 7296, 117.1, 95.2, 63.0, None, 85.3),
+    (4096, 96, 8192, 97.9, 74.1, None, None, 84.7), (8192, 48, 8192, 101.0, 77.1, None, None, 79.9),
+    (8192, 64, 8192, 130.2, 100.2, None, None, 83.2), (14336, 32, 8192, 115.0, 100.8, None, None, 89.6),
+    (20000, 32, 8192, 199.9, 142.9, None, None, 123.5), (28672, 24, 8192, 175.8, 150.2, None, None, 123.1),
+    (32000, 16, 8192, 169.1, 122.9, None, None, 126.0), (32000, 17, 8192, 206.7, 167.1, None, None, 128.1),
+    (65536, 9, 8192, 200.3, 203.5, None, None, 226.1), (4096, 48, 14336, 106.9, 85.7, None, None, 135.4),
+    (11584, 9, 16256, 125.9, None, None, None, 176.9), (2048, 16, 28672, 67.9, None, None, None, 261.0),
+    (8192, 9, 28672, 127.8, None, None, None, 262.3),
+]
+
+
+@pytest.mark.parametrize("M,T,K,c4,c8,c16,c16w8,any_", S_US)
+def test_order_s_takes_a_measured_fast_form(launched, M, T, K, c4, c8, c16, c16w8, any_):
+    l, = launched("bpd_qmatmul_q8_0_dispatch_s_gpu", W, X, OUT, M, T, K)
+    times = (c4, c8, c16, c16w8, any_)
+    t = one_of(times, S_FORMS)(l)
+    assert t is not None, l
+    assert t <= 1.14 * min(x for x in times if x is not None), l
+    assert t <= 1.05 * any_, l
