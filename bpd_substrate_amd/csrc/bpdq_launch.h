@@ -109,7 +109,10 @@ void launch_q8_0_gemm_S(const uint8_t* Wq, const uint8_t* Xq, float* out, int m_
 // Up to 3 matrices of M[i] >= 1 rows sharing the activation rows Xq, one launch.
 void launch_q8_0_gemm_S_multi(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq,
                               int m_tokens, int K, int nan_mode, hipStream_t s);
-// The same by the kernel for few activation rows; false (nothing launched) where its rule
+// Whether gate and up of F rows each are faster as two products and k_swiglu than by
+// launch_q8_0_gemm_S_swiglu.
+bool q8_0_swiglu_S_apart(int F, int m_tokens, int K);
+// launch_q8_0_gemm_S_multi by the kernel for few activation rows; false (nothing launched) where its rule
 // asks for another.  staged: k_q8_0_gemm_SH can run instead.
 bool launch_q8_0_gemm_S_few(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq,
                             int m_tokens, int K, bool staged, int nan_mode, hipStream_t s);

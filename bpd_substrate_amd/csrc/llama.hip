@@ -2074,11 +2074,6 @@ void mt_gemm3(const MtCtx& c, std::initializer_list<const uint8_t*> W, std::init
     for (int i = 0; i < n; i++) mt_gemm(c, w[i], o[i], m[i], K);
 }
 
-// Tokens up to which order S takes gate, up and SwiGLU in two launches: at E = 4096, F =
-// 14336 the epilogue form is 81 us for 1 to 128 tokens, the two launches 37 + 5 at 16
-// tokens and 63 + 5 at 32; above that k_q8_0_gemm_SH runs both ways.
-constexpr int kMtFewTokens = 32;
-
 // Attention of the batch: out[T][H*D] and its Q8_0 rows in c.xq.  The tile
 // kernels (k_mt_scores_tile, k_mt_softmax, k_mt_pv) when the scores tile fits in
 // LDS (G * head_dim <= 2,048 at head_dim <= 256: every llama shape), otherwise
@@ -2153,10 +2148,11 @@ void mt_layer(const MtCtx& c, float* x, const bpd_llama_layer_weights& w, CT* kc
     mt_gemm(c, w.w_o, s2, g.E, qd);
     launch_norm(x, s2, x, w.ffn_norm_w, nullptr, c.xq, g.E, g.eps, c.s, nullptr, T);
     // order S: SwiGLU and its Q8_0 rows in the gate/up GEMM's epilogue (into c.yq;
-    // s2 and s3 then keep no gate, up or SwiGLU rows); otherwise, and for the few rows
-    // whose kernel beats the epilogue's 128-token tile, k_swiglu
+    // s2 and s3 then keep no gate, up or SwiGLU rows); otherwise, and where two
+    // products and it are faster, k_swiglu
     const uint8_t* fq = nullptr;
-    if (c.order_s && T > kMtFewTokens && launch_q8_0_gemm_S_swiglu(w.w_gate, w.w_up, g.F, c.xq, T, g.E, 1, c.yq, c.s)) {
+    if (c.order_s && !q8_0_swiglu_S_apart(g.F, T, g.E) &&
+        launch_q8_0_gemm_S_swiglu(w.w_gate, w.w_up, g.F, c.xq, T, g.E, 1, c.yq, c.s)) {
         fq = c.yq;
     } else {
         mt_gemm3(c, {w.w_gate, w.w_up, w.w_up}, {s2, s3, s3}, {g.F, g.F, g.F}, 2, g.E);

@@ -352,4 +352,20 @@ bool launch_q8_0_gemm_S_few(const uint8_t* const* W, float* const* out, const in
     return form->launch(W, out, M, n, Xq, m_tokens, K / 32, nan_mode, s);
 }
 
+// The epilogue form takes 64 rows of gate and of up x 128 tokens per workgroup, so a few tokens
+// cost what 128 do: about 16.5 ns per element of K for up to 256 workgroups, 25.7 for each 512
+// beyond; k_swiglu costs 2.5 us and 4.5 us per million values.  us, epilogue / apart, K = 4096:
+// 4096x16 73 / 20, 14336x16 75 / 39, 14336x32 76 / 65, 14336x96 77 / 80, 28672x24 115 / 122;
+// K = 1024: 14336x17 25 / 23, 28672x32 37 / 40; K = 8192: 4096x64 140 / 107, 14336x32 144 / 129.
+bool q8_0_swiglu_S_apart(int F, int m_tokens, int K) {
+    const int M[2] = {F, F};
+    double ns;
+    const bool few = K / 32 > 0 && sq_best(M, 2, m_tokens, K, &ns) != nullptr;
+    const double sh = sh_ns(M, 2, m_tokens, K, true);
+    const double apart = (few ? std::min(ns, sh) : sh) + 2500 + 4.5e-3 * (double)F * m_tokens;
+    const int64_t wgs = tiles(M, 1, m_tokens, 64, 128);
+    const double joint = wgs <= 256 ? 5200 + 0.2 * F + 16.5 * K : 10000 + 25.7 * K * (double)((wgs + 511) / 512);
+    return apart < 0.95 * joint;
+}
+
 }  // namespace bpdq

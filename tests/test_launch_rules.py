@@ -3,8 +3,11 @@
 `launches` records what an entry point launches; the tables hold the microseconds per call of
 every form on MI355X (graphs of back-to-back launches, weights beyond the MALL).  No GPU.
 """
+import ctypes
+
 import pytest
 
+from bpd_substrate_amd import llama
 from launches import Recorder
 
 W, X, OUT = 0x100000, 0x200000, 0x300000  # never read: aligned as a torch tensor is
@@ -121,3 +124,32 @@ def test_order_s_takes_a_measured_fast_form(launched, M, T, K, c4, c8, c16, c16w
     assert t is not None, l
     assert t <= 1.14 * min(x for x in times if x is not None), l
     assert t <= 1.05 * any_, l
+
+
+# ---------------------------------------------------------------- gate and up of a layer, order S
+
+# ffn_dim, tokens, embed_dim, then us of the products with SwiGLU in the epilogue, and of two
+# products and k_swiglu
+GLU_US = [
+    (1408, 16, 1024, 22.4, 9.8), (2816, 200, 1024, 24.4, 20.9), (8192, 32, 1024, 23.4, 15.5),
+    (14336, 17, 1024, 25.3, 22.6), (14336, 64, 1024, 25.9, 27.2), (28672, 16, 1024, 37.2, 27.7),
+    (28672, 32, 1024, 38.5, 41.2), (4096, 8, 2048, 37.6, 12.6), (14336, 32, 2048, 41.8, 38.5),
+    (28672, 32, 2048, 63.3, 66.6), (15488, 90, 2048, 47.5, 50.9), (4096, 1, 4096, 72.8, 17.3),
+    (4096, 64, 4096, 74.6, 35.8), (14336, 8, 4096, 75.2, 34.4), (14336, 32, 4096, 76.4, 64.6),
+    (14336, 96, 4096, 78.5, 81.3), (11008, 128, 4096, 77.0, 84.9), (28672, 16, 4096, 116.2, 72.8),
+    (28672, 24, 4096, 114.9, 122.3), (28672, 32, 4096, 116.1, 123.5), (28672, 24, 5120, 141.7, 148.3),
+    (4096, 48, 8192, 139.5, 82.4), (14336, 16, 8192, 141.6, 105.1), (28672, 24, 8192, 216.8, 226.7),
+]
+
+
+@pytest.mark.parametrize("F,T,E,joint,apart", GLU_US)
+def test_block_takes_the_faster_gate_and_up(launched, F, T, E, joint, apart):
+    import numpy as np
+
+    cfg = llama.BpdLlamaConfig(1, E // 64, 1, 64, E, F, 1000, T, 1e-5, 1e4, 64, 0)
+    lw = llama.BpdLlamaLayerWeights(*[ctypes.cast(W, t) for _, t in llama.BpdLlamaLayerWeights._fields_])
+    pos = np.arange(T, dtype=np.int32)
+    ls = launched("bpd_llama_block_s_gpu", X, ctypes.addressof(lw), ctypes.addressof(cfg), pos.ctypes.data, T, 0,
+                  *[0x400000 + 0x100000 * i for i in range(5)], None)
+    t = apart if any(l.kernel == "k_swiglu" for l in ls) else joint
+    assert t <= 1.06 * min(joint, apart), ls
