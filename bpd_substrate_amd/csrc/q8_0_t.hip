@@ -574,7 +574,7 @@ bool launch_q8_0_gemm_T_multi(const uint8_t* const* W, float* const* out, const 
         return (double)((b * ((m_tokens + C - 1) / C) + 255) / 256);
     };
     const double k = K, n1 = per_cu(32, 4), n2 = per_cu(32, 8), n3 = per_cu(32, 64), n4 = per_cu(64, 64);
-    const double gemv = 2600.0 * n + (double)cells * (!wide ? 2.6e-4 * k : rows <= 2048 ? 0.03 + 1.35e-4 * k : 0.04 + 1.6e-4 * k);
+    const double gemv = 2600.0 * n + (double)cells * (!wide ? 0.08 + 2.5e-4 * k : rows <= 2048 ? 0.03 + 1.35e-4 * k : 0.04 + 1.6e-4 * k);
     const double tq1 = 3300 + 600 * n1 + k * std::max(1.22 + 1.38 * n1, 1.85 * n1);
     const double tq2 = 3500 + 600 * n2 + k * std::max(1.5 + 1.95 * n2, 3.3 * n2 - 1.9);
     const double tm32 = 3000 + 300 * n3 + k * (2 + 9 * n3);

@@ -11,7 +11,7 @@ from test_gpu_q8_0 import _d, _q8_full_range, _q8_nan_heavy
 
 pytestmark = pytest.mark.gpu
 
-CASES = [(4099, 4, 256, 0),      # the per-token GEMVs still
+CASES = [(4099, 4, 256, 0),      # 4 tokens per wave, a half chunk
          (2050, 9, 768, 0),      # 4 tokens per wave, a whole and a half chunk, 3 token groups
          (4100, 13, 1280, 0),    # 8 tokens per wave
          (703, 65, 224, 0),      # 8 tokens per wave, an odd number of blocks

@@ -37,6 +37,10 @@ T_FORMS = [lambda l: l.kernel == "k_q8_0_gemm_TQ" and l.args[0] == 1,
            lambda l: l.kernel.startswith("k_q8_0_gemv_")]
 # M, tokens, K, then us of TQ with 4 and 8 tokens, TM with 32 and 64 rows, the per-token GEMVs
 T_US = [
+    (2048, 16, 64, 4.3, 4.5, 4.1, 4.7, 6.1), (8192, 8, 32, 5.4, 4.8, 4.1, 5.2, 8.6),
+    (8192, 8, 64, 5.0, 4.6, 4.1, 4.7, 8.8), (32000, 4, 64, 7.2, 8.5, 8.1, 8.2, 13.8),
+    (32000, 2, 256, 8.3, 10.4, 14.3, 14.4, 13.4), (512, 200, 32, 7.5, 5.9, 4.5, 5.8, 11.8),
+    (32000, 8, 512, 12.9, 11.8, 21.9, 21.3, 29.1),
     (1024, 16, 4096, 14.0, 17.7, None, None, 12.5), (1024, 16, 14336, 39.8, 51.7, None, None, 33.9),
     (2048, 8, 1024, 6.4, 7.4, None, None, 5.8), (2048, 8, 4096, 14.1, 17.7, None, None, 13.0),
     (2048, 8, 14336, 40.2, 52.1, None, None, 37.7), (2048, 33, 4096, None, 25.9, 44.8, 57.5, 38.6),
