@@ -382,12 +382,15 @@ __device__ __forceinline__ void tp_gemv(const uint8_t* __restrict__ W, const uin
     }
 }
 
+// LAYOUT 0: 34-byte rows; 1: the padded layout.
+template <int LAYOUT>
 __global__ __launch_bounds__(320) void k_q8_0_gemv_TP(const uint8_t* __restrict__ W, const uint8_t* __restrict__ Xq,
                                                       float* __restrict__ out, int m_weight, int nb) {
-    tp_gemv<0>(W, Xq, out, m_weight, nb, blockIdx.x);
+    tp_gemv<LAYOUT>(W, Xq, out, m_weight, nb, blockIdx.x);
 }
 
-// The padded layout; up to 3 matrices that share the activation (a decode step's Q, K and V).
+// The padded layout, up to 3 matrices that share the activation (a decode step's Q, K and V).
+// Not for one: reading the matrix from the argument block costs 0.4 us (1024x4096 6.0 against 6.4).
 __global__ __launch_bounds__(320) void k_q8_pad64_gemv_TP(GemmW gw, const uint8_t* __restrict__ Xq, int nb) {
     const int bx = blockIdx.x, mi = (bx >= gw.first[1]) + (bx >= gw.first[2]);
     tp_gemv<1>(gw.w[mi], Xq, gw.out[mi], gw.m[mi], nb, bx - gw.first[mi]);
@@ -731,7 +734,7 @@ void launch_q8_0_dispatch_T(const uint8_t* Wq, const uint8_t* Xq, float* out, in
         hipLaunchKernelGGL((k_q8_0_gemv_T<16, 4>), dim3((waves + 3) / 4, m_tokens), dim3(256), lds, s, Wq, Xq, out,
                            m_weight, nb);
     else if (lds + sizeof(float) * 2 * 64 * kTpLd <= 64 * 1024)
-        hipLaunchKernelGGL(k_q8_0_gemv_TP, dim3((m_weight + 7) / 8, m_tokens), dim3(320), lds, s, Wq, Xq, out, m_weight,
+        hipLaunchKernelGGL(k_q8_0_gemv_TP<0>, dim3((m_weight + 7) / 8, m_tokens), dim3(320), lds, s, Wq, Xq, out, m_weight,
                            nb);
     else
         hipLaunchKernelGGL((k_q8_0_gemv_T<32, 2>), dim3((waves + 1) / 2, m_tokens), dim3(128), lds, s, Wq, Xq, out,
@@ -739,27 +742,22 @@ void launch_q8_0_dispatch_T(const uint8_t* Wq, const uint8_t* Xq, float* out, in
 }
 
 // The padded layout: m_tokens rows of Xq, or (m_tokens == 1) up to 3 matrices in one launch.
-// Few rows take the producer/consumer kernel while its ring and the activation fit in 64 KB of
-// LDS, the rest launch_pad_gemv; k_q8_0_gemm_T where the activation does not fit in LDS at all.
+// The producer/consumer kernel where its ring and the activation fit in 64 KB of LDS and
+// launch_pad_gemv leaves the shape to it, launch_pad_gemv otherwise; k_q8_0_gemm_T where the
+// activation does not fit in LDS at all.
 static void pad64_T(const uint8_t* const* W, float* const* out, const int* N, int n, const uint8_t* Xq, int m_tokens,
                     int K, hipStream_t s) {
     const int nb = K / 32;
     const size_t lds = (size_t)nb * 36;
     const bool ring = lds + sizeof(float) * 2 * 64 * kTpLd <= 64 * 1024;
     if (nb > 0 && launch_pad_gemv(W, out, N, n, Xq, m_tokens, K, ring, s)) return;
+    if (nb > 0 && ring && n == 1) {
+        hipLaunchKernelGGL(k_q8_0_gemv_TP<1>, dim3((N[0] + 7) / 8, m_tokens), dim3(320), lds, s, W[0], Xq, out[0], N[0], nb);
+        return;
+    }
     if (nb > 0 && ring) {
-        GemmW g{};
-        int blocks = 0;
-        for (int i = 0; i < kGemmMulti; i++) {
-            const int q = i < n ? i : 0;
-            g.w[i] = W[q];
-            g.out[i] = out[q];
-            g.m[i] = N[q];
-            g.first[i] = blocks;
-            if (i < n) blocks += (N[i] + 7) / 8;
-        }
-        g.first[kGemmMulti] = blocks;
-        hipLaunchKernelGGL(k_q8_pad64_gemv_TP, dim3(blocks, m_tokens), dim3(320), lds, s, g, Xq, nb);
+        const GemmW g = gemm_args<8>(W, out, N, n);
+        hipLaunchKernelGGL(k_q8_pad64_gemv_TP, dim3(g.first[kGemmMulti], m_tokens), dim3(320), lds, s, g, Xq, nb);
         return;
     }
     for (int i = 0; i < n; i++) {

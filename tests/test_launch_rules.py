@@ -157,3 +157,11 @@ def test_block_takes_the_faster_gate_and_up(launched, F, T, E, joint, apart):
                   *[0x400000 + 0x100000 * i for i in range(5)], None)
     t = apart if any(l.kernel == "k_swiglu" for l in ls) else joint
     assert t <= 1.06 * min(joint, apart), ls
+
+
+# ---------------------------------------------------------------- the padded layout
+
+def test_one_padded_matrix_is_not_read_from_an_argument_block(launched):
+    """The kernel for up to 3 matrices costs one matrix 0.4 us (1024x4096: 6.4 against 6.0)."""
+    l, = launched("bpd_qmatmul_q8_pad64_gpu", W, X, OUT, 1024, 1, 4096)
+    assert (l.kernel, l.args, l.grid) == ("k_q8_0_gemv_TP", [1], (128, 1, 1))
