@@ -92,7 +92,7 @@ void launch_q8_pad64_dispatch_T(const uint8_t* Wp, const uint8_t* Xq, float* out
 
 // The padded layout (q8_pad.hip): up to 3 matrices of N[i] >= 1 rows sharing the activation
 // rows Xq; false (nothing launched) where the activation does not fit in LDS, or where
-// k_q8_pad64_gemv_TP is faster and ring_fits says that it can run.
+// k_q8_0_gemv_TP is faster and ring_fits says that it can run.
 bool launch_pad_gemv(const uint8_t* const* W, float* const* y, const int* N, int n, const uint8_t* Xq, int m_tokens,
                      int K, bool ring_fits, hipStream_t s);
 // Up to 3 matrices sharing one activation row: y[i][N[i]].

@@ -1,7 +1,9 @@
 // q8_pad.hip — the padded Q8 layout [K/32][N][64] (records {f16 d, 0, 0, int8 q[32],
 // 28 zero bytes}): the order-T product of one activation row, and of a gate/up pair with
 // SwiGLU.
+#include <algorithm>
 #include <mutex>
+#include <numeric>
 
 #include "bpdq_device.h"
 #include "bpdq_launch.h"
@@ -179,18 +181,20 @@ __global__ __launch_bounds__(64 * (NW + NH)) void k_pad_gemv(PadW pw, const uint
     }
 }
 
-constexpr int kPadMaxNb = 2540;  // blocks whose activation fits in the 160 KB of LDS
+constexpr int kPadMaxLds = 160 * 1024;
+constexpr int kPadMaxNb = 2540;  // blocks whose activation fits in it
+constexpr size_t pad_lds(int nb) { return (size_t)(nb + kPadG) * 64; }
 
 template <int NW, int NH, int U, bool SWG>
 static bool launch_pad(const PadW& g, int blocks, int m_tokens, const uint8_t* Xq, int nb, hipStream_t s) {
-    const size_t lds = (size_t)(nb + kPadG) * 64;
+    const size_t lds = pad_lds(nb);
     if (nb > kPadMaxNb) return false;
     if (lds > 64 * 1024 - 512) {  // asked for once per process
         static std::once_flag once;
         static bool ok = false;
         std::call_once(once, [] {
             ok = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_pad_gemv<NW, NH, U, SWG>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (kPadMaxNb + kPadG) * 64) == hipSuccess;
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)pad_lds(kPadMaxNb)) == hipSuccess;
             (void)hipGetLastError();
         });
         if (!ok) return false;
@@ -214,26 +218,42 @@ static PadW pad_args(const uint8_t* const* W, float* const* y, const int* N, int
     return g;
 }
 
-// n <= 3 matrices of N[i] >= 1 rows.  Measured on MI355X (K = 4096, weights beyond the
-// MALL; us, the kernels replaced in brackets): 4 waves per workgroup 28672 rows 40
-// (2 x 23), 14336 20.3 (23.1), 32000 44 (47); with fewer rows a workgroup per wave, three
-// waves helping to stage the activation: 6144 10.8 (17), 4096 8.8 (10.6), 4096x14336
-// 24.7 (25.8).  Below 3,072 rows false where that kernel's LDS ring fits: there the chains of the few waves set the time
-// and k_q8_0_gemv_TP, which splits the products from them, is faster (2048x2048 4.5
-// against 5.7, 1024x4096 5.5 against 8.3).
+// n <= 3 matrices of N[i] >= 1 rows: 64 rows per workgroup (4 waves), or 16 rows and three waves
+// that help to stage the activation, or false for k_q8_0_gemv_TP, which splits the products
+// from the chains of its 8 rows.  us on MI355X, weights beyond the MALL, TP / 16 rows / 64 rows:
+//   few cells (rows * tokens), the chains set the time:
+//     K = 1024   1024x1 4.0 / 4.9 / 4.9, 4096x1 4.8 / 5.0 / 5.0, 5120x1 7.0 / 5.7 / 5.2
+//     K = 4096   1024x1 6.0 / 8.9 / 9.6, 1024x4 7.3 / 9.0 / 9.6, 2048x2 7.8 / 9.3 / 10.0,
+//                3584x1 9.4 / 9.9 / 14.5, 4096x1 10.2 / 9.9 / 14.3, 3072x2 13.8 / 10.7 / 14.0
+//     K = 14336  1024x4 17.8 / 23.4 / 35.8, 3072x1 22.6 / 24.1 / 38.9, 4096x1 26.1 / 24.7 / 40.0
+//     K = 512    2048x1 4.0 / 4.3 / 4.4, 4096x1 4.6 / 4.4 / 4.3; K = 128 1024x1 3.8 / 3.2 / 3.1
+//   many: K = 4096 12288x1 - / 18.8 / 18.3, 28672x1 - / 41 / 40; 4096x14336 one row 24.7
+//   16-row workgroups that do not run at once, long rows: K = 28672 3072x3 85 / 86 / 74,
+//     K = 40960 3072x2 85 / 119 / 108, 2048x4 111 / 119 / 104
+//   several tokens read a matrix once where its workgroups meet on an XCD again (a count that 8
+//   divides): 7296x4 K = 1856 (456 / 114 workgroups) 13.3 / 18.0, 9689x2 K = 2880 (606 / 152)
+//     23.2 / 14.0, 5568x3 K = 11552 (348 / 87) 49 / 66.
 bool launch_pad_gemv(const uint8_t* const* W, float* const* y, const int* N, int n, const uint8_t* Xq, int m_tokens,
                      int K, bool ring_fits, hipStream_t s) {
-    int64_t rows = 0;
-    for (int i = 0; i < n; i++) rows += N[i];
-    rows *= m_tokens;
-    if (rows < 3072 && ring_fits) return false;
-    int blocks;
-    if (rows >= 12288) {
-        const PadW g = pad_args(W, y, N, n, 64, &blocks);
-        return launch_pad<4, 0, 8, false>(g, blocks, m_tokens, Xq, K / 32, s);
+    const int nb = K / 32;
+    int64_t cells = 0;
+    for (int i = 0; i < n; i++) cells += N[i];
+    cells *= m_tokens;
+    int b16, b64;
+    const PadW g16 = pad_args(W, y, N, n, 16, &b16), g64 = pad_args(W, y, N, n, 64, &b64);
+    // 16-row workgroups per CU: 4 waves of 52 VGPRs, the activation in LDS
+    const int64_t at_once = std::min<int64_t>(8, kPadMaxLds / pad_lds(nb));
+    const bool fits = (int64_t)b16 * m_tokens <= 256 * at_once;
+    const int64_t few = !fits && at_once == 1 ? 6144 : K < 768 ? 3071 : m_tokens > 1 || K < 4096 ? 4096 : 3840;
+    if (ring_fits && K >= 512 && cells <= few) return false;
+    bool wide = cells >= 12288;
+    if (m_tokens > 1) {
+        const int x16 = std::gcd(b16, 8), x64 = std::gcd(b64, 8);
+        if (x16 > x64) wide = cells >= 32768;
+        if (x64 > x16) wide = cells >= 8192;
     }
-    const PadW g = pad_args(W, y, N, n, 16, &blocks);
-    return launch_pad<1, 3, 16, false>(g, blocks, m_tokens, Xq, K / 32, s);
+    if (wide || !fits) return launch_pad<4, 0, 8, false>(g64, b64, m_tokens, Xq, nb, s);
+    return launch_pad<1, 3, 16, false>(g16, b16, m_tokens, Xq, nb, s);
 }
 
 // Gate and up (F rows each, F % 32 == 0) of one activation row: y = silu(gate) * up and its

@@ -165,3 +165,40 @@ def test_one_padded_matrix_is_not_read_from_an_argument_block(launched):
     """The kernel for up to 3 matrices costs one matrix 0.4 us (1024x4096: 6.4 against 6.0)."""
     l, = launched("bpd_qmatmul_q8_pad64_gpu", W, X, OUT, 1024, 1, 4096)
     assert (l.kernel, l.args, l.grid) == ("k_q8_0_gemv_TP", [1], (128, 1, 1))
+
+
+PAD_FORMS = [lambda l: l.kernel == "k_q8_0_gemv_TP" and l.args == [1],
+             lambda l: l.kernel == "k_pad_gemv" and l.args[0] == 1,
+             lambda l: l.kernel == "k_pad_gemv" and l.args[0] == 4 and not l.args[3]]
+# M, tokens, K, then us of the producer/consumer kernel (None: its ring does not fit in LDS), of
+# 16 and of 64 rows per workgroup, and of the kernel that took the shape before k_pad_gemv was there
+PAD_US = [
+    (1024, 1, 128, 3.8, 3.2, 3.1, 3.8), (5120, 1, 128, 6.3, 4.1, 3.7, 6.3), (2048, 1, 512, 4.0, 4.3, 4.1, 4.0),
+    (4096, 1, 512, 4.6, 4.4, 4.2, 4.6), (1024, 2, 1024, 4.1, 4.9, 4.9, 4.1), (3072, 1, 1024, 4.7, 5.0, 5.0, 4.7),
+    (4096, 1, 1024, 4.8, 5.0, 5.0, 4.8), (5120, 1, 1024, 7.0, 5.7, 5.2, 7.0), (2048, 2, 2048, 5.5, 6.3, 6.6, 5.5),
+    (4096, 1, 2048, 6.2, 6.6, 7.0, 6.2), (6144, 1, 2048, 10.1, 8.0, 9.6, 10.1),
+    (28672, 1, 2048, 38.9, 21.8, 21.4, 24.0), (1024, 4, 4096, 7.3, 9.0, 9.6, 7.3),
+    (2048, 2, 4096, 7.8, 9.3, 10.0, 7.8), (3072, 1, 4096, 9.0, 9.7, 14.3, 9.0),
+    (4096, 1, 4096, 10.2, 9.9, 14.3, 10.2), (3072, 2, 4096, 13.8, 10.7, 14.0, 13.8),
+    (8192, 1, 4096, 22.4, 13.8, 16.0, 16.8), (16384, 1, 4096, 36.9, 23.6, 22.9, 25.1),
+    (28672, 1, 4096, 58.8, 41.0, 40.2, 46.9), (2048, 2, 8192, 13.4, 15.2, 23.7, 13.4),
+    (6144, 1, 8192, 23.2, 18.9, 26.6, 23.2), (1024, 4, 14336, 17.8, 23.4, 35.8, 17.8),
+    (3072, 1, 14336, 22.6, 24.1, 38.9, 22.6), (4096, 1, 14336, 26.1, 24.7, 40.0, 26.1),
+    (3072, 3, 28672, 87.9, 86.1, 74.0, 85.4), (2048, 2, 36864, 41.4, 55.7, 95.1, 41.4),
+    (3072, 1, 36864, 47.2, 57.5, 100.1, 47.2), (3584, 3, 36864, 143.9, 115.4, 97.6, 110.6),
+    (3072, 2, 40960, 84.8, 119.5, 107.7, 84.8), (2048, 4, 40960, 108.3, 118.8, 103.9, 110.6),
+    (3072, 3, 45056, None, 194.9, 117.0, 132.8), (2048, 8, 45056, None, 257.1, 111.3, 136.8),
+    (2048, 4, 57344, None, 166.1, 144.0, 152.8), (1024, 8, 65536, None, 188.4, 147.0, 843.4),
+    (2800, 4, 22784, 94.1, 75.3, 57.9, 69.9), (5757, 3, 2336, 25.4, 12.6, 16.7, 15.5),
+    (7296, 4, 1856, 33.2, 13.3, 18.0, 16.1), (9689, 2, 2880, 33.4, 23.2, 14.0, 26.1),
+]
+
+
+@pytest.mark.parametrize("M,T,K,tp,rows16,rows64,before", PAD_US)
+def test_padded_product_takes_a_measured_fast_form(launched, M, T, K, tp, rows16, rows64, before):
+    l, = launched("bpd_qmatmul_q8_pad64_gpu", W, X, OUT, M, T, K)
+    times = (tp, rows16, rows64)
+    t = one_of(times, PAD_FORMS)(l)
+    assert t is not None, l
+    assert t <= 1.17 * min(x for x in times if x is not None), l
+    assert t <= 1.04 * before, l
