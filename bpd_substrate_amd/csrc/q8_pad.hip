@@ -257,9 +257,13 @@ bool launch_pad_gemv(const uint8_t* const* W, float* const* y, const int* N, int
 }
 
 // Gate and up (F rows each, F % 32 == 0) of one activation row: y = silu(gate) * up and its
-// Q8_0 blocks; false (nothing launched) where the activation does not fit in LDS.
+// Q8_0 blocks; false (nothing launched) where the activation does not fit in LDS, and for few
+// rows of a long K, where two products and k_swiglu are faster: us, apart in brackets, 1024 rows
+// K = 2048 7.3 (7.9), K = 4096 10.7 (10.1), K = 8192 25.4 (14.3), K = 14336 37.8 (19.5); 4096 rows
+// K = 4096 17.0 (16.3), K = 14336 46.2 (42.5); 5632 rows K = 8192 31.7 (34.3).
 bool launch_pad_swiglu(const uint8_t* Wg, const uint8_t* Wu, float* y, uint8_t* yq, int F, const uint8_t* Xq, int K,
                        hipStream_t s) {
+    if (F <= 4096 && K >= 4096) return false;
     PadW g{};
     for (int i = 0; i < kPadMulti; i++) {
         g.w[i] = i == 1 ? Wu : Wg;

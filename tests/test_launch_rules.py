@@ -6,6 +6,7 @@ every form on MI355X (graphs of back-to-back launches, weights beyond the MALL).
 import ctypes
 
 import pytest
+import torch
 
 from bpd_substrate_amd import llama
 from launches import Recorder
@@ -202,3 +203,24 @@ def test_padded_product_takes_a_measured_fast_form(launched, M, T, K, tp, rows16
     assert t is not None, l
     assert t <= 1.17 * min(x for x in times if x is not None), l
     assert t <= 1.04 * before, l
+
+
+# ff_dim, n_embd, then us of gate, up and SwiGLU in one launch, and of the two products in one launch
+# and k_swiglu
+PAD_GLU_US = [
+    (1024, 1024, 5.7, 7.1), (1024, 2048, 7.3, 7.8), (4096, 2048, 12.0, 11.2), (1024, 4096, 10.7, 10.1),
+    (2816, 4096, 17.4, 14.2), (4096, 4096, 17.0, 16.3), (5632, 4096, 19.6, 20.4), (14336, 4096, 42.2, 42.1),
+    (1024, 8192, 25.4, 14.3), (4096, 8192, 27.3, 26.7), (5632, 8192, 31.7, 34.2), (512, 14336, 38.4, 17.4),
+    (2048, 14336, 40.9, 26.9), (4096, 14336, 46.2, 42.5),
+]
+
+
+@pytest.mark.parametrize("F,E,joint,apart", PAD_GLU_US)
+def test_padded_step_takes_the_faster_gate_and_up(launched, F, E, joint, apart):
+    w = torch.zeros(64, dtype=torch.uint8)  # its address is all that is used
+    cfg = dict(n_layers=1, n_embd=E, n_head=E // 64, n_head_kv=1, head_dim=64, ff_dim=F, vocab_size=1000, max_seq=64,
+               eps=1e-5, rope_theta=1e4)
+    m = llama.DecodeModel(cfg, [{k: w for k in llama.MATRICES + ("attn_norm", "ffn_norm")}], w, lm_head=w)
+    ls = launched("bpd_llama_step_gpu", llama.W_Q8_PAD64, *m._args(w, 0))
+    t = apart if any(l.kernel == "k_swiglu" for l in ls) else joint
+    assert t <= 1.1 * min(joint, apart), ls
