@@ -1269,7 +1269,12 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_fused_span(MultiArgs a, const 
     x32_load<WPB, IT>(P, x, nb);
     const uint8_t* seg[S::kSegs];
     int np[S::kSegs];
-    span_segs<NB, R, JOINT>(seg, np, a.w[i], row0, a.M[i], nb);
+    if constexpr (JOINT && NB > 16) {  // by span_segs the scalar loads come behind x's: 512x14336 5.84 us, here 5.63
+        seg[0] = a.w[i] + (int64_t)row0 * (NB * kQ4KBytes);
+        np[0] = min(R, a.M[i] - row0) * NB * 9;
+    } else {
+        span_segs<NB, R, JOINT>(seg, np, a.w[i], row0, a.M[i], nb);
+    }
     u32x4v v[S::kLoads];
     span_issue<S>(v, seg, np);
     __builtin_amdgcn_sched_barrier(0);
