@@ -1009,14 +1009,22 @@ static void launch_gemv(const uint8_t* w, const uint8_t* xq, float* y, int M, in
 // spans, 1024x4096 2.40 against 2.86), 4 waves per workgroup.  Below K = 4096 every row is
 // a segment of its own, so the lanes' pieces need no division by the row length, and the
 // loads past a row's pieces repeat its last one: 32000x2048 9.6 us (12.5 without spans),
-// 15456x2560 5.9 (7.5), 25296x3072 8.8 (10.6), 8192x3584 4.4 (4.9), 1001x1024 2.3 (2.3).
+// 15456x2560 5.9 (7.5), 25296x3072 8.8 (10.6).  Rows that short take one per wave up to 12288
+// (cold weights, us, two rows per wave / without spans: 3000x2048 2.87 / 3.47 / 3.08,
+// 4096x3072 3.32 / 3.85 / 3.38, 6144x1024 3.60 / 3.82 / 3.63, 9000x3072 4.93 / 5.64 / 5.28),
+// in a grid that 8 divides, whose workgroups xcd_major puts in row order: 4 outputs each of a
+// 128-byte line (1001x1024 2.10, 2.17 in a grid of 251; 700x512 1.98, 2.14).
 static bool span_fits(int nb) { return nb >= 1 && nb <= 16; }
-static int span_rows_per_wave(int rows) { return rows <= 2048 ? 1 : 2; }
+static int span_rows_per_wave(int rows, int nb) { return rows <= (nb < 16 ? 12288 : 2048) ? 1 : 2; }
+static dim3 span_grid(int waves, int R, int wpb, int nb) {
+    const int wgs = (waves + wpb - 1) / wpb;
+    return dim3(R == 1 && nb < 16 ? (wgs + 7) / 8 * 8 : wgs);
+}
 
 template <int ORDER, int R>
 static void launch_span(const uint8_t* w, const uint8_t* xq, float* y, int M, int nb, hipStream_t s) {
     constexpr int WPB = 4;
-    const dim3 grid(((M + R - 1) / R + WPB - 1) / WPB);
+    const dim3 grid = span_grid((M + R - 1) / R, R, WPB, nb);
     if (nb == 16)
         hipLaunchKernelGGL((k_q4k_q8k_gemv_span<ORDER, 16, R, true, WPB>), grid, dim3(64 * WPB), 0, s, w, xq, y, M, nb);
     else
@@ -1026,7 +1034,7 @@ static void launch_span(const uint8_t* w, const uint8_t* xq, float* y, int M, in
 template <int ORDER>
 static void launch_gemv_order(const uint8_t* w, const uint8_t* xq, float* y, int M, int nb, hipStream_t s) {
     if (span_fits(nb)) {
-        if (span_rows_per_wave(M) == 1)
+        if (span_rows_per_wave(M, nb) == 1)
             launch_span<ORDER, 1>(w, xq, y, M, nb, s);
         else
             launch_span<ORDER, 2>(w, xq, y, M, nb, s);
@@ -1315,7 +1323,7 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_swiglu_span(const uint8_t* __r
 template <int ORDER, int R>
 static void launch_multi_span(const MultiArgs& a, const uint8_t* xq, int nb, hipStream_t s) {
     constexpr int WPB = 4;
-    const dim3 grid((a.first[kMulti] + WPB - 1) / WPB);
+    const dim3 grid = span_grid(a.first[kMulti], R, WPB, nb);
     if (nb == 16)
         hipLaunchKernelGGL((k_q4k_q8k_multi_span<ORDER, 16, R, true, WPB>), grid, dim3(64 * WPB), 0, s, a, xq, nb);
     else
@@ -1326,7 +1334,7 @@ void launch_qmatmul_q4k_q8k_multi(const uint8_t* const* w, float* const* y, cons
                                   int K, int order, hipStream_t s) {
     const int nb = K / 256;
     if (span_fits(nb)) {
-        const int R = span_rows_per_wave(total_rows(M, n));
+        const int R = span_rows_per_wave(total_rows(M, n), nb);
         const MultiArgs a = make_multi_args(w, y, M, n, R);
         if (a.first[kMulti] == 0) return;
         if (order == 0)
@@ -1423,7 +1431,7 @@ void launch_qmatmul_q4k_fused_multi(const uint8_t* const* w, float* const* y, co
                                     int K, int order, hipStream_t s) {
     const int nb = K / 256;
     if (span_fits(nb)) {
-        const int R = span_rows_per_wave(total_rows(M, n));
+        const int R = span_rows_per_wave(total_rows(M, n), 16);  // at any K: each workgroup quantizes x
         const MultiArgs a = make_multi_args(w, y, M, n, R);
         if (a.first[kMulti] == 0) return;
         if (order == 0)
@@ -1634,7 +1642,7 @@ static void launch_norm_span(const MultiArgs& a, const NormIn& nin, hipStream_t 
 
 void launch_q4k_norm_multi(const uint8_t* const* w, float* const* y, const int* M, int n, const NormIn& nin,
                            int order, hipStream_t s) {
-    const int R = span_rows_per_wave(total_rows(M, n));
+    const int R = span_rows_per_wave(total_rows(M, n), 16);
     const MultiArgs a = make_multi_args(w, y, M, n, R);
     if (a.first[kMulti] == 0) return;
     if (order == 0) {
@@ -1655,7 +1663,7 @@ static int launch_res(const uint8_t* w, int M, const float* x, const ResOut& ro,
 int launch_q4k_res(const uint8_t* w, int M, const float* x, int K, const ResOut& ro, int order, hipStream_t s) {
     if (K / 256 == 56)
         return order == 0 ? launch_res<0, 56, 1, 8, true>(w, M, x, ro, s) : launch_res<1, 56, 1, 8, true>(w, M, x, ro, s);
-    if (span_rows_per_wave(M) == 1)
+    if (span_rows_per_wave(M, 16) == 1)
         return order == 0 ? launch_res<0, 16, 1, 4, false>(w, M, x, ro, s) : launch_res<1, 16, 1, 4, false>(w, M, x, ro, s);
     return order == 0 ? launch_res<0, 16, 2, 4, false>(w, M, x, ro, s) : launch_res<1, 16, 2, 4, false>(w, M, x, ro, s);
 }

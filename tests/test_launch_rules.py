@@ -224,3 +224,25 @@ def test_padded_step_takes_the_faster_gate_and_up(launched, F, E, joint, apart):
     ls = launched("bpd_llama_step_gpu", llama.W_Q8_PAD64, *m._args(w, 0))
     t = apart if any(l.kernel == "k_swiglu" for l in ls) else joint
     assert t <= 1.1 * min(joint, apart), ls
+
+
+# ---------------------------------------------------------------- Q4_K spans
+
+# M, K, then us with one and with two rows per wave (cold weights), and of the kernel without spans
+SPAN_US = [
+    (33, 1024, 1.9, None, 2.13), (700, 512, 1.98, None, 2.35), (1001, 1024, 2.1, None, 2.39),
+    (2048, 2048, 2.38, None, 2.49), (3000, 256, 2.59, 3.2, 2.89), (3000, 1024, 2.76, 3.34, 2.98),
+    (3000, 2048, 2.87, 3.47, 3.08), (3000, 3072, 2.91, 3.7, 3.2), (4096, 512, 2.92, 3.16, 2.96),
+    (4096, 2048, 3.16, 3.59, 3.22), (4096, 3072, 3.32, 3.85, 3.38), (6144, 1024, 3.6, 3.82, 3.63),
+    (6144, 2048, 3.9, 3.97, 3.84), (6144, 3072, 4.05, 4.3, 4.06),
+]
+
+
+@pytest.mark.parametrize("M,K,one,two,before", SPAN_US)
+def test_short_span_rows_per_wave(launched, M, K, one, two, before):
+    for name in ("bpd_qmatmul_q4k_q8k_gpu", "bpd_qmatmul_q4k_q8k_gguf_gpu"):
+        l, = launched(name, W, X, OUT, M, K)
+        assert l.kernel == "k_q4k_q8k_gemv_span" and not l.args[3]
+        t = {1: one, 2: two}[l.args[2]]
+        assert t <= 1.05 * before, l
+        assert l.args[2] == 2 or l.grid[0] % 8 == 0, l  # else a line of outputs is written from 8 XCDs
