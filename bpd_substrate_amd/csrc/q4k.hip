@@ -1407,12 +1407,21 @@ static void launch_fused_span(const MultiArgs& a, const float* x, int nb, hipStr
 }
 
 // Longer rows up to K = 14336: one row per wave through a pass buffer, in workgroups of 8
-// waves.  From 257 to 511 of those some CUs run two and others one, and the 16-wave general
-// kernel is the faster one; us, that kernel in brackets: 1001x4352 4.2 (5.1), 2048x5632 4.2
-// (5.4), 33x8192 3.7 (4.8); 2560x8704 7.7 (6.4), 3072x9216 8.0 (7.0); 8192x8192 9.8 (10.4),
-// 5120x13824 13.2 (14.8).  (16 waves here as well: 2048x5632 5.3, 5120x13824 16.0.)
+// waves, two of which a CU runs at once; the general kernel's workgroups of 16 waves run one at
+// once.  So the time steps at every 2048 rows here and at every 4096 there.  Up to K = 8192 this is
+// the faster one everywhere but from 2049 to 4095 rows (us, the general kernel in brackets:
+// 1024x4352 4.4 (5.4), 3072x6144 5.9 (5.8), 5120x8192 8.3 (9.5), 28672x6144 22.3 (25.3)).  Beyond
+// it is when its last step is the first half of the other's: 2048x9216 5.8 (6.5), 3072x9216 8.4
+// (7.5), 6144x11008 11.5 (11.7), 7168x11008 13.6 (12.4), 10240x13824 19.6 (20.6), 16384x13824
+// 27.7 (27.6).  K = 14336, whose row length is known to the compiler, is 5 % better than its
+// neighbours (4096x14080 10.4, 4096x14336 9.8) and so keeps up where that last step is nearly
+// full: 3072 rows 9.6 (9.0), 4096 9.8 (10.1), 8192 15.8 (15.5), 12288 21.6 (22.0), 28672 45.7 (46.1).
+// (16 waves here as well: 2048x5632 5.3, 5120x13824 16.0.)
 static bool fused_span_long_fits(int rows, int nb) {
-    return nb > 16 && nb <= 56 && (rows <= 2048 || rows >= 4096 || nb == 56);
+    if (nb <= 16 || nb > 56) return false;
+    if (nb <= 32) return rows <= 2048 || rows >= 4096;
+    const int last = (rows - 1) % 4096 + 1;  // rows in the general kernel's last step
+    return last <= 2048 || (nb == 56 && last > 3840);
 }
 
 template <int ORDER>

@@ -246,3 +246,30 @@ def test_short_span_rows_per_wave(launched, M, K, one, two, before):
         t = {1: one, 2: two}[l.args[2]]
         assert t <= 1.05 * before, l
         assert l.args[2] == 2 or l.grid[0] % 8 == 0, l  # else a line of outputs is written from 8 XCDs
+
+
+# M, K, then us of the spans and of the general kernel, each quantizing x, and of the kernel that took
+# the shape before there were spans of any length
+FUSED_LONG_US = [
+    (33, 4352, 3.79, 4.54, 4.56), (2048, 4352, 4.43, 5.47, 5.9), (5120, 4352, 7.12, 8.73, 8.72),
+    (28672, 4352, 21.14, 24.27, 24.34), (512, 6144, 4.34, 5.35, 5.45), (3072, 6144, 5.88, 5.84, 6.15),
+    (8192, 6144, 9.09, 9.25, 9.34), (2048, 8192, 4.73, 5.54, 5.83), (4096, 8192, 6.91, 6.88, 6.84),
+    (7168, 8192, 9.98, 9.69, 9.96), (512, 8448, 5.53, 6.32, 6.52), (2048, 8448, 5.77, 6.51, 6.98),
+    (3072, 8448, 8.36, 7.4, 7.41), (4096, 8448, 8.49, 8.06, 8.08), (5120, 8448, 10.39, 11.21, 11.17),
+    (7168, 8448, 12.4, 11.37, 11.66), (11008, 8448, 16.61, 15.5, 15.57), (16384, 8448, 21.28, 20.12, 20.14),
+    (28672, 8448, 36.64, 33.09, 33.16), (4096, 9216, 8.65, 8.3, 8.31), (9216, 9216, 14.79, 15.47, 15.37),
+    (2048, 11008, 6.22, 7.39, 7.34), (4096, 11008, 8.93, 8.57, 8.55), (8192, 11008, 13.97, 13.05, 13.04),
+    (11008, 11008, 18.27, 17.47, 17.46), (5120, 13824, 13.17, 14.4, 14.36), (8192, 13824, 16.49, 15.38, 15.72),
+    (16384, 13824, 27.72, 27.64, 27.83), (2048, 14080, 7.28, 8.66, 8.59), (4096, 14080, 10.42, 9.92, 10.07),
+    (512, 14336, 5.89, 7.96, 5.89), (2048, 14336, 6.66, 8.38, 6.66), (2560, 14336, 9.64, 8.68, 9.64),
+    (3072, 14336, 9.63, 9.03, 9.63), (4096, 14336, 9.83, 10.06, 9.83), (7168, 14336, 15.49, 14.86, 15.49),
+    (5120, 14336, 12.6, 14.37, 12.6), (8192, 14336, 15.85, 15.54, 15.85), (28672, 14336, 45.71, 46.08, 45.71),
+]
+
+
+@pytest.mark.parametrize("M,K,span,general,before", FUSED_LONG_US)
+def test_long_fused_rows_take_a_measured_fast_form(launched, M, K, span, general, before):
+    l, = launched("bpd_qmatmul_q4k_q8k_fused_gpu", W, X, OUT, M, K)
+    t = {"k_q4k_fused_span": span, "k_q4k_fused_gemv": general}[l.kernel]
+    assert t <= 1.04 * min(span, general), l
+    assert t <= 1.04 * before, l
