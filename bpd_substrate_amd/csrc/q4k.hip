@@ -535,81 +535,71 @@ __device__ __forceinline__ XOps get_x(const uint8_t* __restrict__ xsrc, int b, i
     return o;
 }
 
-// Weight operands of one pass of gemv_rows: qs chunk and header dword of
-// G block-groups x R rows.
-template <int R, int G>
+// Weight operands of one pass of swiglu_rows: qs chunk and header dword of
+// G block-groups x 2 rows.
+template <int G>
 struct WideW {
-    uint4 qv[G][R];
-    uint32_t hw[G][R];
+    uint4 qv[G][2];
+    uint32_t hw[G][2];
 };
 
-// PAIR (R = 2): the wave's two rows are row row0 of w and row row0 of w1.
-template <int R, int G, bool PAIR = false>
-__device__ __forceinline__ void wide_load_g(WideW<R, G>& W, int g, const uint8_t* __restrict__ w, int M, int nb,
-                                            int row0, int t0, const uint8_t* __restrict__ w1 = nullptr) {
+// Group g of a pass: row `row` of w[0] (gate) and of w[1] (up).
+template <int G>
+__device__ __forceinline__ void wide_load_g(WideW<G>& W, int g, const uint8_t* const (&w)[2], int nb, int row, int t0) {
     const int lane = threadIdx.x & 63;
     const int q = lane >> 3, c = lane & 7;
     const int64_t row_bytes = (int64_t)nb * kQ4KBytes;
     const int b = (t0 + g) * 8 + q;
     const int bb = b < nb ? b : nb - 1;
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const uint8_t* base = PAIR && r == 1 ? w1 : w;
-        const int row = PAIR ? row0 : min(row0 + r, M - 1);
-        const uint8_t* blk = base + (int64_t)row * row_bytes + (int64_t)bb * kQ4KBytes;
+    for (int r = 0; r < 2; r++) {
+        const uint8_t* blk = w[r] + (int64_t)row * row_bytes + (int64_t)bb * kQ4KBytes;
         W.qv[g][r] = ld_u128(blk + 16 + 16 * c);
         W.hw[g][r] = ld_u32(blk + 4 * (c & 3));
     }
 }
 
-// One wave's R rows: each pass issues the loads of G block-groups x R rows (a
-// 16-byte qs load and a header dword per lane each) before computing any of
-// them, so every wave keeps its whole share of the stream in flight.  Rows past
-// M reuse row M-1 and slots past nb reuse block nb-1 (their results are
-// discarded), so every address stays in the tensors.  row0 < M.  With PRE the
-// weights of the first pass were loaded by the caller into `pre`.
-//
-// PAIR (R = 2): the rows are row0 of w (gate) and row0 of w1 (up), and the
-// wave stores y[row0] = (g / (1 + expf(-g))) * u, the SwiGLU of the two
-// (bench/bpd_cpu.c:5504-5507) on the bit-exact g and u.
 __device__ __forceinline__ float silu_mul(float g, float u) { return (g / (1.0f + expf_libm(-g))) * u; }
 
-template <int ORDER, int R, int G, bool LX, bool PRE, bool PAIR = false>
-__device__ __forceinline__ void gemv_rows(const uint8_t* __restrict__ w, const uint8_t* __restrict__ xsrc,
-                                          float* __restrict__ y, int M, int nb, int row0, const WideW<R, G>& pre,
-                                          const uint8_t* __restrict__ w1 = nullptr) {
+// One wave's gate row and up row from the Q8_K activation in LDS: y[row] = (g / (1 +
+// expf(-g))) * u, the SwiGLU of the two (bench/bpd_cpu.c:5504-5507) on the bit-exact g and u.
+// Each pass issues the loads of G block-groups x 2 rows (a 16-byte qs load and a header dword
+// per lane each) before computing any of them, so every wave keeps its whole share of the
+// stream in flight; the caller loaded the first pass into `pre`.  Slots past nb reuse block
+// nb-1 (their results are discarded), so every address stays in the tensors.
+template <int ORDER, int G>
+__device__ __forceinline__ void swiglu_rows(const uint8_t* const (&w)[2], const uint8_t* __restrict__ xl,
+                                            float* __restrict__ y, int nb, int row, const WideW<G>& pre) {
     const int lane = threadIdx.x & 63;
     const int q = lane >> 3, c = lane & 7;
     const int ngroups = (nb + 7) >> 3;
-    float s[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) s[r] = 0.0f;
+    float s[2] = {0.0f, 0.0f};
 
     for (int t0 = 0; t0 < ngroups; t0 += G) {
-        WideW<R, G> W;
+        WideW<G> W;
         XOps x[G];
         bool valid[G];
 #pragma unroll
         for (int g = 0; g < G; g++) {
             const int b = (t0 + g) * 8 + q;
             valid[g] = b < nb;
-            if (PRE && t0 == 0) {
+            if (t0 == 0) {
 #pragma unroll
-                for (int r = 0; r < R; r++) {
+                for (int r = 0; r < 2; r++) {
                     W.qv[g][r] = pre.qv[g][r];
                     W.hw[g][r] = pre.hw[g][r];
                 }
             } else {
-                wide_load_g<R, G, PAIR>(W, g, w, M, nb, row0, t0, w1);
+                wide_load_g<G>(W, g, w, nb, row, t0);
             }
-            x[g] = get_x<ORDER, LX>(xsrc, valid[g] ? b : nb - 1, c);
+            x[g] = get_x<ORDER, true>(xl, valid[g] ? b : nb - 1, c);
         }
         // every load of the pass is issued before any of its data is used
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int g = 0; g < G; g++) {
 #pragma unroll
-            for (int r = 0; r < R; r++) {
+            for (int r = 0; r < 2; r++) {
                 const float cb = block_contrib<ORDER>(bcast_header(W.hw[g][r]), W.qv[g][r], x[g], c);
                 if (valid[g]) s[r] = s[r] + cb;
             }
@@ -617,28 +607,27 @@ __device__ __forceinline__ void gemv_rows(const uint8_t* __restrict__ w, const u
     }
     // slot q lives in lanes 8q..8q+7: row_mirror pairs slots q and q^1, then the
     // four pair sums are lanes 0, 16, 32, 48
-    float out[R];
+    float out[2];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
+    for (int r = 0; r < 2; r++) {
         float v = s[r];
         v = v + dpp_f<0x140>(v);
         const float p01 = readlane_f(v, 0), p23 = readlane_f(v, 16);
         const float p45 = readlane_f(v, 32), p67 = readlane_f(v, 48);
         out[r] = (p01 + p23) + (p45 + p67);
-        if (!PAIR && lane == 0 && row0 + r < M) y[row0 + r] = out[r];
     }
-    if (PAIR && lane == 0) y[row0] = silu_mul(out[0], out[R - 1]);
+    if (lane == 0) y[row] = silu_mul(out[0], out[1]);
 }
 
 // ----------------------------------------------------------------------------
 // The same GEMV with 4 lanes per super-block: lane (bl = lane/4, c4 = lane%4)
 // takes qs chunks c4 and c4+4 of super-block 16t+bl, so the header broadcast,
 // the scale decode and the fp32 combine are shared by two chunks and a wave
-// pass covers 16 super-blocks.  The qs are loaded as in gemv_rows (instruction
+// pass covers 16 super-blocks.  The qs are loaded as in swiglu_rows (instruction
 // A: all 8 chunks of blocks 16t..16t+7, B: of blocks 16t+8..16t+15, chunk
 // 4(lane/32)+c4) and one v_permlane32_swap per dword pairs them up.  Integer
 // sums are the same integers and the fp32 order is the same order, so the
-// output equals gemv_rows bit for bit.  Fewer VALU per block pays off on
+// output equals the 8-lane mapping's bit for bit.  Fewer VALU per block pays off on
 // shorter matrices and on long rows.
 // ----------------------------------------------------------------------------
 template <int ORDER>
@@ -785,8 +774,8 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_q8k_gemv(const uint8_t* __rest
 // valid-block rule and the fp32 order are gemv4_rows's (and so gemv_rows's):
 // the bits are the same.  Weights must be 16-byte aligned (rows are then too).
 // Measured at 14336x4096 (graph of back-to-back launches over weights beyond
-// the MALL): 6.73 us against 7.36 for gemv_rows with per-lane chunk loads; the
-// same span in gemv_rows's 8-lane mapping 6.98.
+// the MALL): 6.73 us against 7.36 for the 8-lane mapping with per-lane chunk loads; the
+// same span in that mapping 6.98.
 // ----------------------------------------------------------------------------
 // PB (pass buffer): instead of a slot holding every load, the wave's LDS holds
 // one pass (16 super-blocks, 2,304 bytes), refilled from the staged loads
@@ -1215,14 +1204,15 @@ __global__ __launch_bounds__(64 * WPB) void k_q4k_fused_swiglu(const uint8_t* __
     const int row0 = has ? row : 0;
     XPre<1> P;
     x32_load<WPB, 1>(P, x, nb);
-    WideW<2, G> pre;
+    const uint8_t* const w[2] = {wg, wu};
+    WideW<G> pre;
 #pragma unroll
-    for (int g = 0; g < G; g++) wide_load_g<2, G, true>(pre, g, wg, M, nb, row0, 0, wu);
+    for (int g = 0; g < G; g++) wide_load_g<G>(pre, g, w, nb, row0, 0);
     __builtin_amdgcn_sched_barrier(0);
     x32_quantize<WPB, 1>(P, xl, nb);
     __syncthreads();
     if (!has) return;
-    gemv_rows<ORDER, 2, G, true, true, true>(wg, xl, y, M, nb, row0, pre, wu);
+    swiglu_rows<ORDER, G>(w, xl, y, nb, row0, pre);
 }
 
 template <int ORDER, int WPB>
