@@ -25,15 +25,6 @@ namespace bpdq {
 // its loads in flight allow.  NW waves of 16 rows per workgroup, NH more that only help
 // stage the activation row.
 // ----------------------------------------------------------------------------
-constexpr int kPadMulti = 3;
-struct PadW {
-    const uint8_t* w[kPadMulti];
-    float* y[kPadMulti];
-    int n[kPadMulti];
-    int first[kPadMulti + 1];  // workgroups before matrix i
-    uint8_t* yq;               // SwiGLU: Q8_0 blocks of y
-};
-
 constexpr int kPadG = 4;  // blocks per group
 constexpr int kPadX = 8;  // activation units in flight per thread
 
@@ -48,7 +39,7 @@ __device__ __forceinline__ PadRec pad_load(const uint8_t* p) {
 }
 
 template <int NW, int NH, int U, bool SWG>
-__global__ __launch_bounds__(64 * (NW + NH)) void k_pad_gemv(PadW pw, const uint8_t* __restrict__ Xq, int nb) {
+__global__ __launch_bounds__(64 * (NW + NH)) void k_pad_gemv(GemmW gw, const uint8_t* __restrict__ Xq, int nb) {
     static_assert(U % (2 * kPadG) == 0, "the activation slots alternate");
     static_assert(!SWG || (NW == 4 && NH == 0), "two gate and two up waves");
     constexpr int NT = 64 * (NW + NH);
@@ -58,10 +49,10 @@ __global__ __launch_bounds__(64 * (NW + NH)) void k_pad_gemv(PadW pw, const uint
     const int tid = threadIdx.x, lane = tid & 63, p = lane & 3, tok = blockIdx.y;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int bx = blockIdx.x;
-    const int mi = SWG ? wave >> 1 : (bx >= pw.first[1]) + (bx >= pw.first[2]);
-    const uint8_t* __restrict__ W = pw.w[mi];
-    const int N = pw.n[mi];
-    const int row0 = SWG ? bx * 32 + 16 * (wave & 1) : (bx - pw.first[mi]) * 16 * NW + 16 * min(wave, NW - 1);
+    const int mi = SWG ? wave >> 1 : (bx >= gw.first[1]) + (bx >= gw.first[2]);
+    const uint8_t* __restrict__ W = gw.w[mi];
+    const int N = gw.m[mi];
+    const int row0 = SWG ? bx * 32 + 16 * (wave & 1) : (bx - gw.first[mi]) * 16 * NW + 16 * min(wave, NW - 1);
     const int row = min(row0 + (lane >> 2), N - 1);  // rows past the end repeat the last one
     const int64_t stride = (int64_t)N * 64;
     const int base = min(row0, N - 1);
@@ -173,11 +164,11 @@ __global__ __launch_bounds__(64 * (NW + NH)) void k_pad_gemv(PadW pw, const uint
         if (tid < 32) {
             const float g = gu[tid], u = gu[32 + tid];
             const float v = (g / (1.0f + expf_libm(-g))) * u;
-            pw.y[0][bx * 32 + tid] = v;
-            q8_0_lane_store(v, pw.yq + (int64_t)bx * kQ80Bytes, tid);
+            gw.out[0][bx * 32 + tid] = v;
+            q8_0_lane_store(v, gw.yq + (int64_t)bx * kQ80Bytes, tid);
         }
     } else {
-        if (writes) pw.y[mi][(int64_t)tok * N + row] = y;
+        if (writes) gw.out[mi][(int64_t)tok * N + row] = y;
     }
 }
 
@@ -186,7 +177,7 @@ constexpr int kPadMaxNb = 2540;  // blocks whose activation fits in it
 constexpr size_t pad_lds(int nb) { return (size_t)(nb + kPadG) * 64; }
 
 template <int NW, int NH, int U, bool SWG>
-static bool launch_pad(const PadW& g, int blocks, int m_tokens, const uint8_t* Xq, int nb, hipStream_t s) {
+static bool launch_pad(const GemmW& g, int blocks, int m_tokens, const uint8_t* Xq, int nb, hipStream_t s) {
     const size_t lds = pad_lds(nb);
     if (nb > kPadMaxNb) return false;
     if (lds > 64 * 1024 - 512) {  // asked for once per process
@@ -201,21 +192,6 @@ static bool launch_pad(const PadW& g, int blocks, int m_tokens, const uint8_t* X
     }
     hipLaunchKernelGGL((k_pad_gemv<NW, NH, U, SWG>), dim3(blocks, m_tokens), dim3(64 * (NW + NH)), lds, s, g, Xq, nb);
     return true;
-}
-
-static PadW pad_args(const uint8_t* const* W, float* const* y, const int* N, int n, int R, int* blocks) {
-    PadW g{};
-    *blocks = 0;
-    for (int i = 0; i < kPadMulti; i++) {
-        const int q = i < n ? i : 0;
-        g.w[i] = W[q];
-        g.y[i] = y[q];
-        g.n[i] = N[q];
-        g.first[i] = *blocks;
-        if (i < n) *blocks += (N[i] + R - 1) / R;
-    }
-    g.first[kPadMulti] = *blocks;
-    return g;
 }
 
 // n <= 3 matrices of N[i] >= 1 rows: 64 rows per workgroup (4 waves), or 16 rows and three waves
@@ -239,8 +215,8 @@ bool launch_pad_gemv(const uint8_t* const* W, float* const* y, const int* N, int
     int64_t cells = 0;
     for (int i = 0; i < n; i++) cells += N[i];
     cells *= m_tokens;
-    int b16, b64;
-    const PadW g16 = pad_args(W, y, N, n, 16, &b16), g64 = pad_args(W, y, N, n, 64, &b64);
+    const GemmW g16 = gemm_args<16>(W, y, N, n), g64 = gemm_args<64>(W, y, N, n);
+    const int b16 = g16.first[kGemmMulti], b64 = g64.first[kGemmMulti];
     // 16-row workgroups per CU: 4 waves of 52 VGPRs, the activation in LDS
     const int64_t at_once = std::min<int64_t>(8, kPadMaxLds / pad_lds(nb));
     const bool fits = (int64_t)b16 * m_tokens <= 256 * at_once;
@@ -264,11 +240,11 @@ bool launch_pad_gemv(const uint8_t* const* W, float* const* y, const int* N, int
 bool launch_pad_swiglu(const uint8_t* Wg, const uint8_t* Wu, float* y, uint8_t* yq, int F, const uint8_t* Xq, int K,
                        hipStream_t s) {
     if (F <= 4096 && K >= 4096) return false;
-    PadW g{};
-    for (int i = 0; i < kPadMulti; i++) {
+    GemmW g{};
+    for (int i = 0; i < kGemmMulti; i++) {
         g.w[i] = i == 1 ? Wu : Wg;
-        g.y[i] = y;
-        g.n[i] = F;
+        g.out[i] = y;
+        g.m[i] = F;
     }
     g.yq = yq;
     return launch_pad<4, 0, 8, true>(g, F / 32, 1, Xq, K / 32, s);
