@@ -85,6 +85,61 @@ __device__ __forceinline__ float t_order_cell(const uint8_t* __restrict__ wrow, 
     return x86_add_sw(x86_add_sw(l0, l1, m & 16u), x86_add_sw(l2, l3, m & 32u), m & 64u);
 }
 
+// ROWS consecutive 34-byte rows of a wave in chunks of 16 blocks, each row's chunk as 34
+// 16-byte pieces at any address: loaded into registers (piece lane + 64 k of the chunk per lane)
+// and stored to the wave's LDS slot at a pitch of 544 bytes (136 dwords, 8 mod 64: the rows of a
+// column of quants fall in different banks).  Rows past the matrix repeat its last one.  A piece
+// past a row's end is the row's last 16 bytes; end() moves the last chunk's into place, zeros
+// behind.
+constexpr int kChunkBlocks = 16, kChunkPieces = 34, kChunkPitch = 16 * kChunkPieces;
+typedef uint32_t cu32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t cu32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
+
+template <int ROWS>
+struct RowChunks {
+    static constexpr int N = ROWS * kChunkPieces, PER = (N + 63) / 64;
+    typedef cu32x4 V[PER];
+    const uint8_t* base;
+    uint32_t off[PER], dst[PER];
+    int pc[PER], nch, last;  // this lane's pieces of a row; chunks; where a row's last 16 bytes start
+
+    __device__ __forceinline__ RowChunks(const uint8_t* W, int row0, int m_weight, int nb) {
+        const int64_t bpr = (int64_t)nb * kQ80Bytes;
+        const int first = min(row0, m_weight - 1), lane = threadIdx.x & 63;
+        base = W + first * bpr;
+        nch = (nb + kChunkBlocks - 1) / kChunkBlocks;
+        last = (int)bpr - 16;
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int f = min(lane + 64 * k, N - 1), r = f / kChunkPieces;
+            pc[k] = f % kChunkPieces;
+            off[k] = (uint32_t)((min(row0 + r, m_weight - 1) - first) * bpr);
+            dst[k] = (uint32_t)(r * kChunkPitch + 16 * pc[k]);
+        }
+    }
+    __device__ __forceinline__ void load(V& v, int c) const {  // chunks past the last: the last again
+        const int at = min(c, nch - 1) * kChunkPitch;
+#pragma unroll
+        for (int k = 0; k < PER; k++)
+            v[k] = *reinterpret_cast<const cu32x4_a1*>(base + (off[k] + (uint32_t)min(at + 16 * pc[k], last)));
+    }
+    __device__ __forceinline__ void end(V& v) const {  // v: chunk nch - 1
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int past = (nch - 1) * kChunkPitch + 16 * pc[k] - last;
+            if (past <= 0) continue;
+            const unsigned __int128 x = __builtin_bit_cast(unsigned __int128, v[k]);
+            v[k] = __builtin_bit_cast(cu32x4, past >= 16 ? (unsigned __int128)0 : x >> (8 * past));
+        }
+    }
+    __device__ __forceinline__ void store(uint8_t* slot, const V& v) const {
+#pragma unroll
+        for (int k = 0; k < PER; k++)
+            if (k < PER - 1 || N % 64 == 0 || (int)(threadIdx.x & 63) + 64 * k < N)
+                *reinterpret_cast<cu32x4*>(slot + dst[k]) = v[k];
+    }
+};
+
 // Up to kGemmMulti weight matrices that share the activation rows X (a prefill's
 // Q, K and V) in one launch: workgroup column bx takes row block bx - first[i]
 // of matrix i.

@@ -35,10 +35,7 @@ typedef int si32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t su32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t su32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
 
-constexpr int kSqPieces = 34;             // 16-byte pieces of a row's chunk of 16 blocks
-constexpr int kSqPitch = 16 * kSqPieces;  // 544 bytes: 136 dwords, 8 mod 64
-constexpr int kSqSlot = 16 * kSqPitch;    // a wave's 16 rows
-constexpr int kSqPer = (16 * kSqPieces + 63) / 64;
+constexpr int kSqSlot = 16 * kChunkPitch;  // a wave's 16 rows
 constexpr int kSqMaxLds = 160 * 1024;
 
 // blocks of the activation in LDS: whole groups of 4, zeros past the end (a zero block adds
@@ -115,44 +112,13 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_SQ(GemmW gw, const uint8_
     const int row0 = (bx - gw.first[mi]) * R + wave * 16, n0 = by * C;
     const int64_t bpr = (int64_t)nb * kQ80Bytes;
     const int nch = (nb + 15) / 16, nbp = sq_blocks(nb);
-    const int last = (int)bpr - 16;  // where a row's last 16 bytes start
-
-    // weights: rows past the end repeat the last one; a piece past a row's end is its last
-    // 16 bytes, moved into place (zeros behind) by wfix
-    const int base = min(row0, m_weight - 1);
-    const uint8_t* wbase = W + (int64_t)base * bpr;
-    uint32_t off[kSqPer], dst[kSqPer];
-    int pc[kSqPer];
-#pragma unroll
-    for (int k = 0; k < kSqPer; k++) {
-        const int f = min(lane + 64 * k, 16 * kSqPieces - 1), r = f / kSqPieces;
-        pc[k] = f % kSqPieces;
-        off[k] = (uint32_t)((min(row0 + r, m_weight - 1) - base) * bpr);
-        dst[k] = (uint32_t)(r * kSqPitch + 16 * pc[k]);
-    }
+    const RowChunks<16> rows(W, row0, m_weight, nb);
     uint8_t* xs = sqlds;
     uint16_t* xsc = reinterpret_cast<uint16_t*>(sqlds + (size_t)nbp * C * 32);
     uint8_t* slot = sqlds + (size_t)nbp * C * 34 + wave * kSqSlot;
-    const auto wload = [&](su32x4 (&v)[kSqPer], int c) {
-        const int at = min(c, nch - 1) * kSqPitch;
-#pragma unroll
-        for (int k = 0; k < kSqPer; k++)
-            v[k] = *reinterpret_cast<const su32x4_a1*>(wbase + (off[k] + (uint32_t)min(at + 16 * pc[k], last)));
-    };
-    const auto wfix = [&](su32x4 (&v)[kSqPer]) {  // chunk nch - 1
-#pragma unroll
-        for (int k = 0; k < kSqPer; k++) {
-            const int past = (nch - 1) * kSqPitch + 16 * pc[k] - last;
-            if (past <= 0) continue;
-            const unsigned __int128 x = __builtin_bit_cast(unsigned __int128, v[k]);
-            v[k] = __builtin_bit_cast(su32x4, past >= 16 ? (unsigned __int128)0 : x >> (8 * past));
-        }
-    };
-    const auto wstore = [&](const su32x4 (&v)[kSqPer]) {
+    const auto wstore = [&](const RowChunks<16>::V& v) {
         asm volatile("" ::: "memory");  // behind the reads of the previous chunk
-#pragma unroll
-        for (int k = 0; k < kSqPer; k++)
-            if (k < kSqPer - 1 || lane + 64 * k < 16 * kSqPieces) *reinterpret_cast<su32x4*>(slot + dst[k]) = v[k];
+        rows.store(slot, v);
         asm volatile("" ::: "memory");
     };
 
@@ -180,11 +146,11 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_SQ(GemmW gw, const uint8_
             if (h == 0) xsc[b * C + t] = i < nu ? (uint16_t)xh[u] : (uint16_t)0;
         }
     };
-    su32x4 wv[2][kSqPer];
+    RowChunks<16>::V wv[2];
     xload(tid);
     __builtin_amdgcn_sched_barrier(0);
-    wload(wv[0], 0);
-    wload(wv[1], 1);
+    rows.load(wv[0], 0);
+    rows.load(wv[1], 1);
     __builtin_amdgcn_sched_barrier(0);
     xstore(tid);
     for (int i0 = tid + XU * NT; i0 < nup; i0 += XU * NT) {
@@ -195,17 +161,17 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_SQ(GemmW gw, const uint8_
 
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     const int j = lane & 15, k = lane >> 4;
-    const uint8_t* wq = slot + j * kSqPitch + 8 * k;   // this lane's row, eight quants from 8 k
-    const uint8_t* wd = slot + j * kSqPitch + 34 * k;  // the scale of block k of a group of four
+    const uint8_t* wq = slot + j * kChunkPitch + 8 * k;   // this lane's row, eight quants from 8 k
+    const uint8_t* wd = slot + j * kChunkPitch + 34 * k;  // the scale of block k of a group of four
     const uint8_t* xq = xs + (j % C) * 32 + 8 * k;     // columns past C repeat tokens (not stored)
     const uint16_t* xd = xsc + k * C + j % C;
     SqOps o[2];
-    if (nch == 1) wfix(wv[0]);
+    if (nch == 1) rows.end(wv[0]);
     wstore(wv[0]);
-    wload(wv[0], 2);
+    rows.load(wv[0], 2);
     sq_read<C>(o[0], wq, wd, xq, xd, 0);
     // a whole chunk of 4 groups; the next chunk goes into the slot behind the last group's reads
-    const auto step = [&](su32x4 (&next)[kSqPer], int c) {
+    const auto step = [&](RowChunks<16>::V& next, int c) {
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             if (t < 3) {
@@ -213,9 +179,9 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_SQ(GemmW gw, const uint8_
             } else {
                 xq += 16 * C * 32;
                 xd += 16 * C;
-                if (c + 2 == nch) wfix(next);
+                if (c + 2 == nch) rows.end(next);
                 wstore(next);
-                wload(next, c + 3);
+                rows.load(next, c + 3);
                 sq_read<C>(o[0], wq, wd, xq, xd, 0);
             }
             __builtin_amdgcn_sched_barrier(0);

@@ -20,10 +20,9 @@ namespace bpdq {
 //    16 tokens as the exact fp32 value (|p_L| <= 65,536), so there is no
 //    int-to-float conversion.  Two of them (L = 2k, L = 2k+1) cover a Q8_0 block.
 //  - the same instruction with the two f16 scales at inner index 0 and zeros
-//    elsewhere gives RN(Ad*Bd) (exact: 11 x 11 bits) of two blocks x two column
-//    tiles at once.
-// A workgroup owns R = 16 WRN weight rows x C = 16 CT WCN tokens; each of its WRN x
-// WCN waves 16 rows x 16 CT tokens: 32 CT accumulators per lane.  A stage is 2 blocks
+//    elsewhere gives RN(Ad*Bd) (exact: 11 x 11 bits) of both blocks of a stage at once.
+// A workgroup owns R = 16 WRN weight rows x C = 16 WCN tokens; each of its WRN x
+// WCN waves 16 rows x 16 tokens: 32 accumulators per lane.  A stage is 2 blocks
 // (68 bytes of a row), staged by 4 threads per row: a thread loads half a block,
 // turns its 16 quants to f16 (0x6400 | (q ^ 0x80) is 1152 + q) and writes 32 bytes.
 // PF stages are in flight in registers, two LDS slots alternate, one barrier per
@@ -42,9 +41,9 @@ typedef uint32_t tu32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t tu32x4_a1 __attribute__((ext_vector_type(4), aligned(1)));
 typedef uint32_t tu32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
-template <int WRN, int WCN, int CT>
+template <int WRN, int WCN>
 struct TmGeo {
-    static constexpr int R = 16 * WRN, C = 16 * CT * WCN, ROWS = R + C;
+    static constexpr int R = 16 * WRN, C = 16 * WCN, ROWS = R + C;
     static constexpr int NT = 64 * WRN * WCN, UNITS = 4 * ROWS;  // staging threads (UNITS % 64 == 0)
     static constexpr int PASSES = (UNITS + NT - 1) / NT;
     static constexpr int PLANE = ROWS * 64 + 16;                 // bytes of one block's quants
@@ -111,11 +110,11 @@ __device__ __forceinline__ uint32_t tm_store(uint8_t* slot, const TmRaw& t, int 
     return has_m128(q[0]) | has_m128(q[1]) | has_m128(q[2]) | has_m128(q[3]);
 }
 
-template <int WRN, int WCN, int CT, int PF, bool AL>
+template <int WRN, int WCN, int PF, bool AL>
 __global__ __launch_bounds__(64 * WRN * WCN) void k_q8_0_gemm_TM(GemmW gw, const uint8_t* __restrict__ X, int m_tokens,
                                                                  int nb) {
-    using G = TmGeo<WRN, WCN, CT>;
-    static_assert(PF % 2 == 0 && (CT == 1 || CT == 2), "slot parity; one scale product per stage");
+    using G = TmGeo<WRN, WCN>;
+    static_assert(PF % 2 == 0, "slot parity");
     __shared__ __align__(16) uint8_t lds[2 * G::SLOT];
     __shared__ uint32_t m128[G::C];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -164,19 +163,17 @@ __global__ __launch_bounds__(64 * WRN * WCN) void k_q8_0_gemm_TM(GemmW gw, const
     load(raw[0], PF);
     lds_barrier();
 
-    float acc[CT][8][4];
+    float acc[8][4];
 #pragma unroll
-    for (int ct = 0; ct < CT; ct++)
+    for (int L = 0; L < 8; L++)
 #pragma unroll
-        for (int L = 0; L < 8; L++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[ct][L][r] = 0.0f;
+        for (int r = 0; r < 4; r++) acc[L][r] = 0.0f;
 
     const int j = lane & 15, k = lane >> 4;
     const int frag = j * 64 + 16 * (k ^ (j >> 2));  // this lane's chunk in a 16-row tile
-    const int arow = wr * 16, brow = G::R + wc * 16 * CT;
-    // scale operands: lane group k gives block k & 1, column tile k >> 1
-    const int asc = (k & 1) * G::ROWS + arow + j, bsc = (k & 1) * G::ROWS + brow + (CT == 2 ? 16 * (k >> 1) : 0) + j;
+    const int arow = wr * 16, brow = G::R + wc * 16;
+    // scale operands: lane group k gives block k & 1
+    const int asc = (k & 1) * G::ROWS + arow + j, bsc = (k & 1) * G::ROWS + brow + j;
     const tf32x16 zero = {0.0f};
 
     for (int s0 = 0; s0 < nst; s0 += PF) {
@@ -198,22 +195,19 @@ __global__ __launch_bounds__(64 * WRN * WCN) void k_q8_0_gemm_TM(GemmW gw, const
                 const uint4 fa = *reinterpret_cast<const uint4*>(slot + u * G::PLANE + arow * 64 + frag);
                 const h16x4 a0 = __builtin_bit_cast(h16x4, make_uint2(fa.x, fa.y));
                 const h16x4 a1 = __builtin_bit_cast(h16x4, make_uint2(fa.z, fa.w));
+                const uint4 fb = *reinterpret_cast<const uint4*>(slot + u * G::PLANE + brow * 64 + frag);
+                const h16x4 b0 = __builtin_bit_cast(h16x4, make_uint2(fb.x, fb.y));
+                const h16x4 b1 = __builtin_bit_cast(h16x4, make_uint2(fb.z, fb.w));
+                const tf32x16 p0 = __builtin_amdgcn_mfma_f32_16x16x4f16(a0, b0, zero, 0, 0, 0);
+                const tf32x16 p1 = __builtin_amdgcn_mfma_f32_16x16x4f16(a1, b1, zero, 0, 0, 0);
 #pragma unroll
-                for (int ct = 0; ct < CT; ct++) {
-                    const uint4 fb = *reinterpret_cast<const uint4*>(slot + u * G::PLANE + (brow + 16 * ct) * 64 + frag);
-                    const h16x4 b0 = __builtin_bit_cast(h16x4, make_uint2(fb.x, fb.y));
-                    const h16x4 b1 = __builtin_bit_cast(h16x4, make_uint2(fb.z, fb.w));
-                    const tf32x16 p0 = __builtin_amdgcn_mfma_f32_16x16x4f16(a0, b0, zero, 0, 0, 0);
-                    const tf32x16 p1 = __builtin_amdgcn_mfma_f32_16x16x4f16(a1, b1, zero, 0, 0, 0);
+                for (int g = 0; g < 4; g++)
 #pragma unroll
-                    for (int g = 0; g < 4; g++)
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const float d = delta[4 * (u + 2 * ct) + r];
-                            acc[ct][2 * g][r] = d * p0[4 * g + r] + acc[ct][2 * g][r];
-                            acc[ct][2 * g + 1][r] = d * p1[4 * g + r] + acc[ct][2 * g + 1][r];
-                        }
-                }
+                    for (int r = 0; r < 4; r++) {
+                        const float d = delta[4 * u + r];
+                        acc[2 * g][r] = d * p0[4 * g + r] + acc[2 * g][r];
+                        acc[2 * g + 1][r] = d * p1[4 * g + r] + acc[2 * g + 1][r];
+                    }
             }
             lds_barrier();
         }
@@ -223,34 +217,28 @@ __global__ __launch_bounds__(64 * WRN * WCN) void k_q8_0_gemm_TM(GemmW gw, const
     for (int ps = 0; ps < G::PASSES; ps++)
         if (bad[ps] != 0) m128[srow[ps] - G::R] = 1u;
     __syncthreads();
-    // register r of lane l: row 4 (l / 16) + r of the wave's 16, token l % 16 of column tile ct
+    // register r of lane l: row 4 (l / 16) + r of the wave's 16, token l % 16
+    const int tl = wc * 16 + j, tok = n0 + tl, r0 = m0 + arow + 4 * k;
+    if (tok >= m_tokens) return;
+    float y[4];
+    bool odd = m128[tl] != 0;
 #pragma unroll
-    for (int ct = 0; ct < CT; ct++) {
-        const int tl = wc * 16 * CT + 16 * ct + j, tok = n0 + tl;
-        if (tok >= m_tokens) continue;
-        const int r0 = m0 + arow + 4 * k;
-        float y[4];
-        bool odd = m128[tl] != 0;
+    for (int r = 0; r < 4; r++) {
+        y[r] = ((acc[0][r] + acc[4][r]) + (acc[2][r] + acc[6][r])) + ((acc[1][r] + acc[5][r]) + (acc[3][r] + acc[7][r]));
+        odd |= __builtin_isnan(y[r]);
+    }
+    if (odd) {  // the reference's own arithmetic: NaN bits, -128 activation quants
+        for (int r = 0; r < 4; r++)
+            if (r0 + r < m_weight && (m128[tl] != 0 || __builtin_isnan(y[r])))
+                y[r] = t_order_cell(W + (r0 + r) * bpr, kQ80Bytes, 2, X + tok * bpr, nb, r0 + r, tok, m_weight, m_tokens);
+    }
+    float* o = out + (int64_t)tok * m_weight + r0;
+    if ((reinterpret_cast<uintptr_t>(o) & 15) == 0 && r0 + 4 <= m_weight) {
+        *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
+    } else {
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const float(&a)[8][4] = acc[ct];
-            y[r] = ((a[0][r] + a[4][r]) + (a[2][r] + a[6][r])) + ((a[1][r] + a[5][r]) + (a[3][r] + a[7][r]));
-            odd |= __builtin_isnan(y[r]);
-        }
-        if (odd) {  // the reference's own arithmetic: NaN bits, -128 activation quants
-            for (int r = 0; r < 4; r++)
-                if (r0 + r < m_weight && (m128[tl] != 0 || __builtin_isnan(y[r])))
-                    y[r] = t_order_cell(W + (r0 + r) * bpr, kQ80Bytes, 2, X + tok * bpr, nb, r0 + r, tok, m_weight,
-                                        m_tokens);
-        }
-        float* o = out + (int64_t)tok * m_weight + r0;
-        if ((reinterpret_cast<uintptr_t>(o) & 15) == 0 && r0 + 4 <= m_weight) {
-            *reinterpret_cast<float4*>(o) = make_float4(y[0], y[1], y[2], y[3]);
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-                if (r0 + r < m_weight) o[r] = y[r];
-        }
+        for (int r = 0; r < 4; r++)
+            if (r0 + r < m_weight) o[r] = y[r];
     }
 }
 
@@ -270,18 +258,14 @@ __global__ __launch_bounds__(64 * WRN * WCN) void k_q8_0_gemm_TM(GemmW gw, const
 // ----------------------------------------------------------------------------
 typedef float tf32x4 __attribute__((ext_vector_type(4)));
 
-template <int NQ, int NW, int CB>
+template <int NQ, int NW>
 struct TqGeo {
-    static constexpr int C = 4 * NQ, R = 8 * NW, NT = 64 * NW;
-    static constexpr int PIECES = CB * 17 / 8;  // 16-byte pieces of a row's chunk
-    static constexpr int WP = 8 * PIECES, PER = (WP + 63) / 64;
-    static constexpr int PITCH = CB == 8 ? 288 : CB == 16 ? 544 : 1120;
+    static constexpr int C = 4 * NQ, R = 8 * NW, NT = 64 * NW, CB = kChunkBlocks;
     static constexpr int PLANE = C * 64 + 32;             // one block's activation quants
     static constexpr int XSLOT = CB * PLANE + CB * C * 4;  // quants, then the scales [block pair][token][2]
     static constexpr int UX = C * CB * 2, XP = (UX + NT - 1) / NT;
-    static constexpr int LDS = 2 * XSLOT + NW * 8 * PITCH;
-    static_assert(PITCH >= 16 * PIECES && PITCH % 16 == 0 && (PITCH / 32) % 2 == 1 && PITCH % 32 == 0 && CB % 8 == 0 &&
-                      XSLOT % 16 == 0, "LDS geometry");
+    static constexpr int LDS = 2 * XSLOT + NW * 8 * kChunkPitch;
+    static_assert((kChunkPitch / 32) % 2 == 1 && kChunkPitch % 32 == 0 && XSLOT % 16 == 0, "LDS geometry");
 };
 
 struct TqX {
@@ -340,9 +324,10 @@ __device__ __forceinline__ void tq_pair(const TqOps<NQ>& o, float (&acc)[NQ][4])
     }
 }
 
-template <int NQ, int NW, int CB>
+template <int NQ, int NW>
 __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_t* __restrict__ X, int m_tokens, int nb) {
-    using G = TqGeo<NQ, NW, CB>;
+    using G = TqGeo<NQ, NW>;
+    constexpr int CB = G::CB;
     __shared__ __align__(16) uint8_t lds[G::LDS];
     __shared__ uint32_t m128[G::C];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -356,36 +341,8 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
     const int row0 = (bx - gw.first[mi]) * G::R + wave * 8, n0 = by * G::C;
     const int64_t bpr = (int64_t)nb * kQ80Bytes;
     const int nch = (nb + CB - 1) / CB;
-    const int last = (int)bpr - 16;  // where a row's last 16 bytes start
-
-    // weights: piece k of this lane is piece f % PIECES of row f / PIECES of the chunk; a
-    // piece past the row's end is its last 16 bytes, moved into place (zeros behind) by wfix
-    const uint8_t* wbase = W + (int64_t)min(row0, m_weight - 1) * bpr;
-    uint32_t off[G::PER], dst[G::PER];
-    int pc[G::PER];
-#pragma unroll
-    for (int k = 0; k < G::PER; k++) {
-        const int f = min(lane + 64 * k, G::WP - 1), r = f / G::PIECES;
-        pc[k] = f % G::PIECES;
-        off[k] = (uint32_t)((min(row0 + r, m_weight - 1) - min(row0, m_weight - 1)) * bpr);
-        dst[k] = (uint32_t)(r * G::PITCH + 16 * pc[k]);
-    }
-    uint8_t* slot = lds + 2 * G::XSLOT + wave * 8 * G::PITCH;
-    const auto wload = [&](tu32x4 (&v)[G::PER], int c) {
-        const int at = min(c, nch - 1) * 16 * G::PIECES;
-#pragma unroll
-        for (int k = 0; k < G::PER; k++)
-            v[k] = *reinterpret_cast<const tu32x4_a1*>(wbase + (off[k] + (uint32_t)min(at + 16 * pc[k], last)));
-    };
-    const auto wfix = [&](tu32x4 (&v)[G::PER]) {  // chunk nch - 1
-#pragma unroll
-        for (int k = 0; k < G::PER; k++) {
-            const int past = (nch - 1) * 16 * G::PIECES + 16 * pc[k] - last;
-            if (past <= 0) continue;
-            const unsigned __int128 x = __builtin_bit_cast(unsigned __int128, v[k]);
-            v[k] = __builtin_bit_cast(tu32x4, past >= 16 ? (unsigned __int128)0 : x >> (8 * past));
-        }
-    };
+    const RowChunks<8> rows(W, row0, m_weight, nb);
+    uint8_t* slot = lds + 2 * G::XSLOT + wave * 8 * kChunkPitch;
     // activations: unit i is half i & 1 of block (i / 2) % CB of token i / (2 CB)
     TqX xr[G::XP];
     const auto xload = [&](int c) {
@@ -415,10 +372,10 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
         }
     };
 
-    tu32x4 wv[2][G::PER];
+    RowChunks<8>::V wv[2];
     xload(0);
-    wload(wv[0], 0);
-    wload(wv[1], 1);
+    rows.load(wv[0], 0);
+    rows.load(wv[1], 1);
     for (int i = tid; i < G::C; i += G::NT) m128[i] = 0u;
     xstore(0, 0);
     lds_barrier();
@@ -429,16 +386,14 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
 #pragma unroll
         for (int r = 0; r < 4; r++) acc[q][r] = 0.0f;
     const int j = lane & 3, L = (lane >> 2) & 7, rg = lane >> 5;
-    const uint8_t* wq = slot + (4 * rg + j) * G::PITCH + 4 * L;   // this lane's row, dword L
-    const uint8_t* wd = slot + (4 * rg + j) * G::PITCH;
+    const uint8_t* wq = slot + (4 * rg + j) * kChunkPitch + 4 * L;   // this lane's row, dword L
+    const uint8_t* wd = slot + (4 * rg + j) * kChunkPitch;
 
-    const auto step = [&](tu32x4 (&v)[G::PER], int xs, int c) {
-        if (c == nch - 1) wfix(v);
-#pragma unroll
-        for (int k = 0; k < G::PER; k++)
-            if (k < G::PER - 1 || G::WP % 64 == 0 || lane + 64 * k < G::WP) *reinterpret_cast<tu32x4*>(slot + dst[k]) = v[k];
+    const auto step = [&](RowChunks<8>::V& v, int xs, int c) {
+        if (c == nch - 1) rows.end(v);
+        rows.store(slot, v);
         xload(min(c + 1, nch - 1));  // before the weights: loads return in order
-        wload(v, c + 2);
+        rows.load(v, c + 2);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         const uint8_t* x = lds + xs * G::XSLOT;
         const uint8_t* xq = x + j * 64 + 8 * L;
@@ -498,21 +453,21 @@ __global__ __launch_bounds__(64 * NW) void k_q8_0_gemm_TQ(GemmW gw, const uint8_
     out[(int64_t)tok * m_weight + row] = y;
 }
 
-template <int WRN, int WCN, int CT, int PF, bool AL>
+template <int WRN, int WCN, int PF, bool AL>
 static void launch_tm(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq, int m_tokens,
                       int nb, hipStream_t s) {
-    using G = TmGeo<WRN, WCN, CT>;
+    using G = TmGeo<WRN, WCN>;
     const GemmW g = gemm_args<G::R>(W, out, M, n);
-    hipLaunchKernelGGL((k_q8_0_gemm_TM<WRN, WCN, CT, PF, AL>), dim3(g.first[kGemmMulti] * ((m_tokens + G::C - 1) / G::C)),
+    hipLaunchKernelGGL((k_q8_0_gemm_TM<WRN, WCN, PF, AL>), dim3(g.first[kGemmMulti] * ((m_tokens + G::C - 1) / G::C)),
                        dim3(G::NT), 0, s, g, Xq, m_tokens, nb);
 }
 
-template <int NQ, int NW, int CB>
+template <int NQ, int NW>
 static void launch_tq(const uint8_t* const* W, float* const* out, const int* M, int n, const uint8_t* Xq, int m_tokens,
                       int nb, hipStream_t s) {
-    using G = TqGeo<NQ, NW, CB>;
+    using G = TqGeo<NQ, NW>;
     const GemmW g = gemm_args<G::R>(W, out, M, n);
-    hipLaunchKernelGGL((k_q8_0_gemm_TQ<NQ, NW, CB>), dim3(g.first[kGemmMulti] * ((m_tokens + G::C - 1) / G::C)),
+    hipLaunchKernelGGL((k_q8_0_gemm_TQ<NQ, NW>), dim3(g.first[kGemmMulti] * ((m_tokens + G::C - 1) / G::C)),
                        dim3(G::NT), 0, s, g, Xq, m_tokens, nb);
 }
 
@@ -571,15 +526,15 @@ bool launch_q8_0_gemm_T_multi(const uint8_t* const* W, float* const* out, const 
     if (al4) least = std::min(least, tm64);
     if (gemv <= least) return false;
     if (least == tq1)
-        launch_tq<1, 4, 16>(W, out, M, n, Xq, m_tokens, nb, s);
+        launch_tq<1, 4>(W, out, M, n, Xq, m_tokens, nb, s);
     else if (least == tq2)
-        launch_tq<2, 4, 16>(W, out, M, n, Xq, m_tokens, nb, s);
+        launch_tq<2, 4>(W, out, M, n, Xq, m_tokens, nb, s);
     else if (least == tm32 && al4)
-        launch_tm<2, 4, 1, 4, true>(W, out, M, n, Xq, m_tokens, nb, s);
+        launch_tm<2, 4, 4, true>(W, out, M, n, Xq, m_tokens, nb, s);
     else if (least == tm32)
-        launch_tm<2, 4, 1, 4, false>(W, out, M, n, Xq, m_tokens, nb, s);
+        launch_tm<2, 4, 4, false>(W, out, M, n, Xq, m_tokens, nb, s);
     else
-        launch_tm<4, 4, 1, 4, true>(W, out, M, n, Xq, m_tokens, nb, s);
+        launch_tm<4, 4, 4, true>(W, out, M, n, Xq, m_tokens, nb, s);
     return true;
 }
 
