@@ -3,13 +3,23 @@
 For every shape the GPU tests use (and edge shapes: one row, spare waves in the
 last workgroup, K = 0, ragged tails) this recomputes, lane by lane, the byte
 ranges each kernel reads and writes and checks they stay inside the tensors.
-It mirrors the index formulas of bpd_substrate_amd/csrc/*.hip and the launch
-choices of their launchers; a change there must be mirrored here.  No GPU.
+It mirrors the index formulas of bpd_substrate_amd/csrc/*.hip; a change there must
+be mirrored here.  The launches of the quantized products (kernel, template
+arguments, grid, LDS) are those that the launchers themselves make.  No GPU.
 """
 import numpy as np
 import pytest
 
+from launches import Recorder
+
 Q4K, Q8K, Q80 = 144, 292, 34
+XS = 304                            # bytes of a Q8_K block quantized into LDS
+W, X, OUT = 0x100000, 0x200000, 0x300000  # never read: aligned as a torch tensor is
+
+
+@pytest.fixture(scope="module")
+def launched(tmp_path_factory):
+    return Recorder(str(tmp_path_factory.mktemp("launches")))
 
 
 def lanes():
@@ -17,21 +27,6 @@ def lanes():
 
 
 # ---------------------------------------------------------------- Q4_K x Q8_K GEMV
-
-def span_rows_per_wave(rows):
-    """span_rows_per_wave() in q4k.hip."""
-    return 1 if rows <= 2048 else 2
-
-
-def q4k_gemv_shape(rows, nb):
-    """(kind, R, G, WPB) as launch_gemv_order() in q4k.hip picks it for 16-byte
-    aligned weights (kind 2: k_q4k_q8k_gemv_span)."""
-    if nb == 16:
-        return (2, span_rows_per_wave(rows), 1, 4)
-    if nb > 16:
-        return (1, 2, 1, 4)
-    return (1, 1, 1, 8) if rows <= 8192 else (0, 2, 2, 4)
-
 
 def x_accesses(c):
     """(offset, bytes) of every Q8_K access load_x makes for chunk c (both element maps)."""
@@ -52,7 +47,8 @@ def q6x_accesses(c, order):
 
 
 def check_wide(M, nb, row0, R, G):
-    w_size, x_size = M * nb * Q4K, nb * Q8K
+    """wide_load_g / get_x of swiglu_rows: row row0 of each of the two matrices."""
+    w_size, x_size = M * nb * Q4K, nb * XS
     l = lanes()
     q, c = l >> 3, l & 7
     for t0 in range(0, (nb + 7) >> 3, G):
@@ -63,45 +59,59 @@ def check_wide(M, nb, row0, R, G):
                 base = min(row0 + r, M - 1) * nb * Q4K + bb * Q4K
                 assert (base + 16 + 16 * c + 16).max() <= w_size and base.min() >= 0
                 assert (base + 4 * (c & 3) + 4).max() <= w_size
-            for off, size in x_accesses(c):
-                assert np.max(bb * Q8K + off + size) <= x_size and np.min(bb * Q8K + off) >= 0
+            assert np.max(bb * XS + 288 + 4) <= x_size
 
 
-def check_span(M, nb, row0, R, joint=True):
-    """span_issue / span_rows of Span<NB=nb, R, JOINT> in q4k.hip for the wave
-    whose first row is row0 of an M-row matrix (joint: R consecutive rows as one
-    span; otherwise R one-row spans of different matrices, here rows row0 of R
-    matrices of M rows): the 16-byte pieces (clamped to the tensor), the slot of
-    whole loads, the 4-lane mapping's LDS reads (block clamped to nb-1), the
-    load count each pass waits for, and span_load_x's Q8_K reads."""
+def check_span(M, nb, row0, R, joint=True, NB=None, pass_buffer=False):
+    """span_segs / span_issue / span_rows of Span<NB, R, joint> in q4k.hip, rows of nb <= NB
+    super-blocks, for the wave whose first row is row0 of an M-row matrix (joint: R consecutive
+    rows as one span, nb == NB; otherwise R one-row spans): the 16-byte pieces (clamped to the
+    segment), the slot of whole loads, or with pass_buffer each pass's pieces copied into a
+    16-block buffer and read back there, the 4-lane mapping's LDS reads (block clamped to
+    nb-1), the load count each pass waits for, and the Q8_K reads."""
+    NB = nb if NB is None else NB
+    assert nb <= NB and (nb == NB or not joint)
     w_size, x_size = M * nb * Q4K, nb * Q8K
     segs = 1 if joint else R
-    seg_pieces = (R if joint else 1) * nb * 9
+    seg_pieces = (R if joint else 1) * NB * 9
     seg_loads = (seg_pieces + 63) // 64
     loads = segs * seg_loads
-    slot = loads * 64 * 16
+    slot = 16 * Q4K if pass_buffer else loads * 64 * 16
     l = lanes()
     bl, c4 = l >> 2, l & 3
+    np_ = min(R, M - row0) * NB * 9 if joint else nb * 9
     for g in range(segs):
-        np_ = min(R, M - row0) * nb * 9 if joint else nb * 9
-        span = row0 * nb * Q4K
+        span = row0 * nb * Q4K if joint else min(row0 + g, M - 1) * nb * Q4K
         for u in range(seg_loads):
             p = np.minimum(l + 64 * u, np_ - 1)
             assert (span + 16 * p).min() >= 0 and (span + 16 * p + 16).max() <= w_size
-            assert (16 * (l + 64 * (g * seg_loads + u)) + 16).max() <= slot
+            assert pass_buffer or (16 * (l + 64 * (g * seg_loads + u)) + 16).max() <= slot
     for r in range(R):
         for t in range((nb + 15) // 16):
-            end = min(16 * t + 16, nb)
-            need = ((r * nb + end) * 9 + 63) // 64 if joint else r * seg_loads + (end * 9 + 63) // 64
-            assert need <= loads
-            row_off = r * nb * Q4K if joint else r * seg_loads * 1024
             bb = np.minimum(16 * t + bl, nb - 1)
+            if pass_buffer:
+                p0 = ((r * NB if joint else 0) + 16 * t) * 9
+                n = min(16, NB - 16 * t) * 9
+                held = np.zeros(16 * 9, bool)
+                for u in range(seg_loads):
+                    q = l + 64 * u - p0
+                    ok = (q >= 0) & (q < n)
+                    assert (16 * q[ok] + 16 <= slot).all()
+                    held[q[ok]] = True
+                off = bb - 16 * t
+                assert (off >= 0).all() and ((off * Q4K + 144) <= slot).all()
+                for k in range(9):  # every piece of every block read was written by this pass
+                    assert held[off * 9 + k].all()
+                continue
+            end = min(16 * t + 16, NB)
+            need = ((r * NB + end) * 9 + 63) // 64 if joint else r * seg_loads + (end * 9 + 63) // 64
+            assert need <= loads
+            row_off = r * NB * Q4K if joint else r * seg_loads * 1024
             blk = row_off + bb * Q4K
             # every piece the pass reads lies in a load it waited for
             assert ((blk + 144) <= need * 1024).all()
-            assert (blk + 16).max() <= slot
             assert (blk + 16 + 16 * c4 + 16).max() <= slot and (blk + 80 + 16 * c4 + 16).max() <= slot
-    for t in range((nb + 15) // 16):
+    for t in range((NB + 15) // 16):  # span_load_x: all NB blocks' slots, clamped to nb
         b = np.minimum(16 * t + bl, nb - 1)
         for c in (c4, c4 + 4):
             for off, size in x_accesses(c):
@@ -129,80 +139,91 @@ def check_four(M, nb, row0, R):
                 assert np.max(bb * Q8K + off + size) <= x_size and np.min(bb * Q8K + off) >= 0
 
 
-@pytest.mark.parametrize("M,K", [(4096, 4096), (14336, 4096), (4096, 14336), (1024, 4096), (1, 256), (5, 512),
-                                 (13, 2304), (9, 2304), (3, 0), (64, 1024), (77, 512), (6144, 4096), (28672, 4096),
-                                 (8193, 4096), (17, 4352), (2, 14336)])
-@pytest.mark.parametrize("force", [None, (0, 2, 2, 4), (1, 1, 1, 8), (1, 2, 1, 4), (1, 1, 1, 16), (2, 2, 1, 4),
-                                   (2, 1, 1, 4)])
-def test_q4k_q8k_gemv_in_bounds(M, K, force):
-    nb = K // 256
-    if nb == 0:
-        return  # no block-group pass runs: the kernels read nothing and write y = +0.0
-    if force is not None and force[0] == 2 and nb != 16:
-        return  # the span kernel is instantiated for K = 4096 only
-    kind, R, G, WPB = force or q4k_gemv_shape(M, nb)
-    waves = (M + R - 1) // R
-    grid = (waves + WPB - 1) // WPB
-    for blk in sorted({0, grid - 1}):
-        for wave in range(WPB):
-            row0 = (blk * WPB + wave) * R
-            if row0 >= M:
-                continue
-            if kind == 0:
-                check_wide(M, nb, row0, R, G)
-            elif kind == 1:
-                check_four(M, nb, row0, R)
-            else:
-                check_span(M, nb, row0, R)
-            for r in range(R):
-                if row0 + r < M:
-                    assert (row0 + r) * 4 + 4 <= M * 4
+def check_fused_quantization(l, nb, WPB, IT, lds):
+    """x32_load / x32_quantize: every Q8_K block of x quantized by one thread row, inside x and LDS."""
+    assert IT * 4 * WPB >= nb, "some Q8_K block would never be quantized"
+    tid = np.arange(64 * WPB)
+    gq, li = tid >> 4, tid & 15
+    for it in range(IT):
+        b = np.minimum(it * 4 * WPB + gq, nb - 1)
+        assert ((b * 256 + 16 * li + 16) <= nb * 256).all() and (b >= 0).all()
+        bw = it * 4 * WPB + gq
+        ok = bw < nb
+        assert ((bw[ok] * XS + 16 * li[ok] + 16) <= lds).all()
+        assert ((bw[ok] * XS + 288 + 4) <= lds).all()
 
 
-@pytest.mark.parametrize("Ms", [[4096, 1024, 1024], [4096, 1024, 1024, 13], [1], [7, 2048], [14336, 14336]])
-def test_q4k_multi_span_in_bounds(Ms):
-    """k_q4k_q8k_multi_span / k_q4k_fused_span at K = 4096: every wave of every
-    matrix (waves past the last row read row 0 of a non-empty matrix)."""
-    nb = 16
-    R = span_rows_per_wave(sum(Ms))
+def check_q4k(l, Ms, nb):
+    """One launch of a Q4_K product over matrices of Ms rows."""
+    k, a = l.kernel, l.args
+    if k in ("k_q4k_q8k_gemv_span", "k_q4k_q8k_multi_span", "k_q4k_fused_span"):
+        NB, R, joint, WPB = a[1:5]
+        pb = k == "k_q4k_fused_span" and bool(a[5])
+        rows = lambda M, r0: check_span(M, nb, r0, R, bool(joint), NB, pb)
+        if k == "k_q4k_fused_span":
+            check_fused_quantization(l, nb, WPB, (NB + 4 * WPB - 1) // (4 * WPB), NB * XS)
+            slot = 16 * Q4K if pb else (1 if joint else R) * (((R if joint else 1) * NB * 9 + 63) // 64) * 1024
+            assert WPB * slot + NB * XS <= 160 * 1024
+    elif k in ("k_q4k_q8k_gemv", "k_q4k_q8k_gemv_multi"):
+        R, WPB = a[1:3]
+        rows = lambda M, r0: check_four(M, nb, r0, R)
+    else:
+        assert k == "k_q4k_fused_gemv", l
+        R, WPB, IT = a[1:4]
+        rows = lambda M, r0: check_four(M, nb, r0, R)
+        assert l.lds == nb * XS
+        check_fused_quantization(l, nb, WPB, IT, l.lds)
+    assert l.block[0] == 64 * WPB
+    waves = sum((M + R - 1) // R for M in Ms)
+    assert l.grid[0] * WPB >= waves  # waves past the last return, or (fused) read row 0 of a matrix
     for M in Ms:
-        for row0 in range(0, M, R):
-            check_span(M, nb, row0, R)
-        check_span(M, nb, 0, R)
+        for r0 in sorted({0, R * ((M - 1) // R), R * ((M - 1) // (2 * R))} if M else ()):
+            rows(M, r0)
 
 
-@pytest.mark.parametrize("nb,R,M", [(56, 1, 1), (56, 1, 7), (56, 1, 4096), (16, 2, 16384), (16, 2, 28672),
-                                    (16, 2, 16385)])
-def test_q4k_fused_span_pass_buffer_in_bounds(nb, R, M):
-    """k_q4k_fused_span<ORDER, NB, R, WPB, PB = true> (K = 14336 one row per wave; K = 4096
-    from 16,384 rows, two rows per wave): the rows' pieces as loads, each pass's pieces
-    copied into a 16-block buffer and read back there."""
-    buf = 16 * Q4K
-    for row0 in sorted({0, ((M - 1) // R) * R}):
-        check_span(M, nb, row0, R)  # global reads and x reads are those of the slot form
-        l = lanes()
-        bl = l >> 2
-        pieces = R * nb * 9
-        covered = np.zeros(pieces, bool)
-        for r in range(R):
-            for t in range((nb + 15) // 16):
-                p0, n = (r * nb + 16 * t) * 9, min(16, nb - 16 * t) * 9
-                for u in range((pieces + 63) // 64):
-                    q = l + 64 * u - p0
-                    ok = (q >= 0) & (q < n)
-                    assert (16 * q[ok] + 16 <= buf).all()
-                    covered[(l + 64 * u)[ok & (l + 64 * u < pieces)]] = True
-                bb = np.minimum(16 * t + bl, nb - 1) - 16 * t
-                assert (bb >= 0).all() and ((bb * Q4K + 144) <= buf).all()
-                assert ((bb * Q4K + 144) <= n * 16).all()  # only the pass's own pieces are read
-        assert covered.all()
+@pytest.mark.parametrize("M,K", [(4096, 4096), (14336, 4096), (4096, 14336), (1024, 4096), (1, 256), (5, 512),
+                                 (13, 2304), (9, 2304), (64, 1024), (77, 512), (6144, 4096), (28672, 4096),
+                                 (8193, 4096), (17, 4352), (2, 14336), (12289, 3840), (12288, 3840), (3, 16384),
+                                 (4097, 8192), (1, 8448), (4096, 14080), (2049, 6144), (16385, 4096), (7, 65536)])
+@pytest.mark.parametrize("entry", ["q4k_q8k", "q4k_q8k_gguf", "q4k_q8k_fused"])
+def test_q4k_products_in_bounds(launched, M, K, entry):
+    if entry == "q4k_q8k_fused" and K > 16384:
+        return  # quantized to memory first
+    l = [l for l in launched(f"bpd_qmatmul_{entry}_gpu", W, X, OUT, M, K) if not l.kernel.startswith("k_quant")]
+    assert len(l) == 1
+    check_q4k(l[0], [M], K // 256)
+
+
+@pytest.mark.parametrize("nb", [1, 7, 15, 16, 17, 32, 33, 55, 56, 57, 64])
+@pytest.mark.parametrize("Ms", [[4096, 1024, 1024], [4096, 1024, 1024, 13], [1], [7, 2048], [14336, 14336], [1, 0, 5]])
+@pytest.mark.parametrize("entry", ["multi", "fused_multi"])
+def test_q4k_multi_products_in_bounds(launched, Ms, nb, entry):
+    n = len(Ms)
+    w, y, m = np.full(n, W, np.int64), np.full(n, OUT, np.int64), np.array(Ms, np.int32)
+    l = launched(f"bpd_qmatmul_q4k_q8k_{entry}_gpu", w.ctypes.data, y.ctypes.data, m.ctypes.data, n, X, nb * 256)
+    l = [l for l in l if not l.kernel.startswith("k_quant")]
+    assert len(l) == 1
+    check_q4k(l[0], Ms, nb)
 
 
 @pytest.mark.parametrize("M", [1, 5, 512, 14336])
-def test_q4k_swiglu_span_in_bounds(M):
-    """k_q4k_swiglu_span: row r of gate and of up as two one-row spans."""
+@pytest.mark.parametrize("nb", [1, 7, 12, 16])
+def test_q4k_swiglu_span_in_bounds(M, nb):
+    """k_q4k_swiglu_span (Span<16, 2, false>): row r of gate and of up as two one-row spans of
+    two matrices; here both are row r of the same matrix."""
     for row in sorted({0, M - 1, M // 2}):
-        check_span(M, 16, row, 2, joint=False)
+        check_span(M, nb, row, 1, joint=False, NB=16)
+        seg_loads = (16 * 9 + 63) // 64
+        assert ((1 * seg_loads) * 1024 + nb * Q4K) <= 2 * seg_loads * 1024  # the up row's half of the slot
+
+
+@pytest.mark.parametrize("M", [1, 5, 512])
+@pytest.mark.parametrize("nb", [17, 56, 64])
+def test_q4k_fused_swiglu_in_bounds(M, nb):
+    """k_q4k_fused_swiglu<.., G = 2, WPB = 16>: K > 4096, one row of gate and of up per wave."""
+    check_fused_quantization(None, nb, 16, 1, nb * XS)
+    for row in sorted({0, M - 1}):
+        check_wide(M, nb, row, 1, 2)
 
 
 @pytest.mark.parametrize("M", [1, 7, 64, 14336])
@@ -309,6 +330,52 @@ def test_q6k_span_long_in_bounds(M):
     assert covered.all()
 
 
+@pytest.mark.parametrize("M,K", [(1, 2304), (33, 2560), (10720, 3072), (8191, 4352), (8192, 4352), (8193, 4352),
+                                 (4096, 4096), (9, 14336), (3072, 9216), (32003, 5120), (5, 23296)])
+def test_q6k_stream_in_bounds(launched, M, K):
+    """k_q6k_q8k_gemv_stream: rows at any 2-byte address (K = 4096 and 14336 off the 16-byte grid), R
+    rows per wave of np passes; the last pass of a row is its last 1,680 bytes, pieces from `lead`."""
+    w = W if K not in (4096, 14336) else W + 2
+    l, = launched("bpd_qmatmul_q6k_q8k_gpu", w, X, OUT, M, K)
+    assert l.kernel == "k_q6k_q8k_gemv_stream"
+    Q6, nb, WPB, AHEAD, REC, PP = 210, K // 256, l.args[1], 4, 20, 105
+    PASS, buf = 8 * Q6, 8 * Q6 + 16
+    assert l.lds == nb * 8 * REC * 4 + WPB * buf <= 64 * 1024
+    R = -(-M // (l.grid[0] * WPB))
+    np_ = (nb + 7) >> 3
+    tail = nb - 8 * (np_ - 1)
+    lead, row_bytes = PASS - tail * Q6, nb * Q6
+    assert np_ >= 2 and 1 <= tail <= 8
+    l_ = lanes()
+    q = l_ >> 3
+    for row0 in sorted({0, R, R * ((M - 1) // R), R * (l.grid[0] * WPB - 1)}):
+        total = max(min(R, M - row0), 0) * np_
+        lrow, lt, li = min(row0, M - 1) * row_bytes, 0, 0
+        for _ in range(total + 2 * AHEAD):  # as many loads as any wave issues
+            end = lt == np_ - 1
+            lo = lead >> 4 if end else 0
+            hi = PP - 1 if li < total else lo
+            base = lrow + lt * PASS - (lead if end else 0)
+            for u in range(2):
+                a = base + 16 * np.minimum(np.maximum(l_ + 64 * u, lo), hi)
+                assert a.min() >= lrow and (a + 16).max() <= lrow + row_bytes <= M * row_bytes
+            li += 1
+            if li < total:
+                lrow += row_bytes if end else 0
+                lt = 0 if end else lt + 1
+    # a pass in the buffer: the pieces of every block read are stored, the spare slot is the 106th
+    for end in (False, True):
+        qq = np.minimum(q, tail - 1) if end else q
+        blk = (lead if end else 0) + qq * Q6
+        assert (blk // 16 >= (lead >> 4 if end else 0)).all() and (blk + Q6 <= PASS).all()
+        assert 16 * min(63 + 64, PP) + 16 <= buf
+        t = np_ - 1 if end else np_ - 2
+        assert (((8 * t + qq) * 8 + 7) * REC + 18 < nb * 8 * REC).all()
+    # x records: each once
+    i = np.concatenate([np.arange(64 * WPB) + i0 for i0 in range(0, nb * 8, 64 * WPB)])
+    assert set(range(nb * 8)) <= set(i.tolist())
+
+
 # ---------------------------------------------------------------- dequant
 
 @pytest.mark.parametrize("nb", [1, 7, 33, 65536, 4096])
@@ -338,26 +405,7 @@ def v_lds(nb, nw):
     return (32 * v_xpitch(nb) + nb) * 4 + nw * V_SLOT
 
 
-def q8_wide_config(mw, mt, nb):
-    """(NW, XR) of k_q8_0_gemv_V as launch_wide() in q8_0.hip picks it for a
-    16-byte aligned W, or None."""
-    if nb == 0 or nb % 32 != 0:
-        return None
-    waves = -(-mw // V_ROWS) * mt
-    if waves < 256:
-        return None
-    xr = lambda nw: next((x for x in (4, 8, 16, 32) if nb * 8 <= x * 64 * nw), None)
-    nw = 4
-    XR = xr(nw)
-    if XR is None:
-        nw = 8
-        XR = xr(nw)
-    if XR is None or v_lds(nb, nw) > 160 * 1024:
-        return None
-    return nw, XR
-
-
-def check_wide_q8(mw, mt, nb, w_size, x_size, out_size):
+def check_wide_q8(l, mw, mt, nb, w_size, x_size, out_size):
     """k_q8_0_gemv_V: lane l of wave w in workgroup g (rows row0 = 2(g*NW + w) ..)
     reads 16-byte piece f = min(l + 64k, 135) (k < 3, every lane) -- row f/68,
     bytes 1088c + 16(f%68) of that row (rows past mw re-read row mw-1) -- for
@@ -370,7 +418,8 @@ def check_wide_q8(mw, mt, nb, w_size, x_size, out_size):
     x dwords at (4L + q)*(nb/4 + 4) + 8c + b16/4 and four products at
     (4row + q)*12 + b16/4; the activation is quant dword min(i, 8nb-1) and scale
     min(j, nb-1)."""
-    NW, XR = q8_wide_config(mw, mt, nb)
+    NW, XR = l.args
+    assert nb * 8 <= XR * 64 * NW and l.lds == v_lds(nb, NW)
     NT, bpr, nch, xp = 64 * NW, nb * Q80, nb // 32, v_xpitch(nb)
     l = np.arange(64)
     groups = -(-mw // (V_ROWS * NW))
@@ -418,22 +467,6 @@ def check_wide_q8(mw, mt, nb, w_size, x_size, out_size):
     assert v_lds(nb, NW) <= 160 * 1024
 
 
-def q8_gemv_config(mw, mt, K):
-    nb = K // 32
-    waves = (mw + 7) // 8
-    if nb == 0:
-        return None
-    if q8_wide_config(mw, mt, nb) is not None:
-        return ("wide", 0, 0)
-    if nb * 36 > 64 * 1024:
-        return ("plain", 4, 1)
-    if waves * mt >= 1024:
-        return ("pipelined", 4, 16)
-    if nb * 36 + 2 * 64 * 36 * 4 <= 64 * 1024:
-        return ("producer", 5, 32)
-    return ("pipelined", 2, 32)
-
-
 def check_producer(mw, mt, nb, layout, w_size):
     """k_q8_0_gemv_TP: producer lane p of workgroup g reads block min(c*32 + p%32,
     nb-1) of row min(8g + p/32, mw-1) for chunks c < nch, bytes [blk, blk+34)
@@ -467,31 +500,46 @@ def check_producer(mw, mt, nb, layout, w_size):
                                      (4096, 4, 4096), (4096, 2, 14336), (512, 1, 8192),
                                      (4100, 1, 4096), (1024, 1, 14336), (2048, 1, 4096), (512, 1, 65536),
                                      (513, 1, 3072), (28672, 1, 4096), (4097, 3, 1024)])
-def test_q8_0_gemv_T_in_bounds(mw, mt, K):
-    cfg = q8_gemv_config(mw, mt, K)
+def test_q8_0_T_in_bounds(launched, mw, mt, K):
     nb = K // 32
+    for w in (W, W + 16, W + 4, W + 1):  # every alignment that the launcher looks at
+        l, = launched("bpd_qmatmul_q8_0_dispatch_gpu", w, X, OUT, mw, mt, K)
+        check_q8_0_T(l, mw, mt, nb, w - W)
+
+
+def check_q8_0_T(l, mw, mt, nb, misaligned):
     bpr = nb * Q80
     w_size, x_size, out_size = mw * bpr, mt * bpr, mw * mt * 4
-    if cfg is None:
+    if l.kernel == "k_q8_0_gemm_TM":
+        assert not l.args[3] or misaligned % 4 == 0
+        check_tm(l, [mw], mt, nb)
         return
-    kind, WPB, U = cfg
-    if kind == "wide":
-        check_wide_q8(mw, mt, nb, w_size, x_size, out_size)
+    if l.kernel == "k_q8_0_gemm_TQ":
+        check_tq(l, [mw], mt, nb)
         return
-    if kind == "producer":
-        check_producer(mw, mt, nb, 0, w_size)
+    assert l.grid[1] == mt
+    if l.kernel == "k_q8_0_gemv_V":
+        assert misaligned % 16 == 0
+        check_wide_q8(l, mw, mt, nb, w_size, x_size, out_size)
+        return
+    if l.kernel == "k_q8_0_gemv_TP":
+        assert l.lds == nb * 36 and l.lds + 2 * 64 * 36 * 4 <= 64 * 1024
+        check_producer(mw, mt, nb, l.args[0], w_size)
         for tok in range(mt):
             assert tok * bpr + (nb - 1) * Q80 + 2 + 28 + 4 <= x_size
         return
-    waves = (mw + 7) // 8
-    grid = (waves + WPB - 1) // WPB if kind == "pipelined" else (waves + 3) // 4
+    if l.kernel == "k_q8_0_gemm_T":
+        check_plain(l, mw, nb, w_size)
+        return
+    assert l.kernel == "k_q8_0_gemv_T", l
+    U, WPB = l.args
+    assert l.lds == nb * 36 <= 64 * 1024 and l.grid[0] * WPB * 8 >= mw
     l = lanes()
     L = l & 7
-    for blk in sorted({0, grid - 1}):
+    waves = (mw + 7) // 8
+    for blk in sorted({0, (waves + WPB - 1) // WPB - 1}):
         for wave in range(WPB):
             row = (blk * WPB + wave) * 8 + (l >> 3)
-            if kind == "plain":
-                continue
             row0 = min((blk * WPB + wave) * 8, mw - 1)
             doff = (np.maximum(np.minimum(row, mw - 1), row0) - row0) * bpr
             assert doff.min() >= 0
@@ -506,6 +554,215 @@ def test_q8_0_gemv_T_in_bounds(mw, mt, K):
                 assert tok * bpr + (nb - 1) * Q80 + 2 + 28 + 4 <= x_size
                 ok = row < mw
                 assert ((tok * mw + row[ok]) * 4 + 4).max(initial=0) <= out_size
+
+
+def check_plain(l, mw, nb, w_size):
+    """k_q8_0_gemm_T<LAYOUT>: 8 rows per wave, rows past the last clamped, whole waves past it return."""
+    layout = l.args[0]
+    assert l.grid[0] * 32 >= mw
+    for row in {0, mw - 1}:
+        at = row * (nb * Q80 if layout == 0 else 64) + (nb - 1) * (Q80 if layout == 0 else mw * 64)
+        assert at + (2 if layout == 0 else 4) + 28 + 4 <= w_size
+
+
+# ---------------------------------------------------------------- Q8_0, several activation rows
+
+CHUNK, PIECES, PITCH = 16, 34, 544
+
+
+def check_row_chunks(ROWS, row0, M, nb):
+    """RowChunks<ROWS> for the wave whose first row is row0: every load inside its matrix, and
+    the slot holds the rows' chunk with zeros behind their end (run on bytes, not only ranges)."""
+    bpr = nb * Q80
+    w = np.frombuffer(np.random.default_rng(M + nb).bytes(M * bpr), np.uint8)
+    N, per = ROWS * PIECES, (ROWS * PIECES + 63) // 64
+    first, last, nch = min(row0, M - 1), bpr - 16, (nb + CHUNK - 1) // CHUNK
+    assert (min(ROWS, M) * bpr) < 2 ** 32 and last >= 0
+    for c in sorted({0, nch - 1, max(nch - 2, 0)}):
+        slot = np.full(ROWS * PITCH, 0xAA, np.uint8)
+        for k in range(per):
+            for lane in range(64):
+                f = min(lane + 64 * k, N - 1)
+                r, pc = f // PIECES, f % PIECES
+                off = (min(row0 + r, M - 1) - first) * bpr
+                a = first * bpr + off + min(c * PITCH + 16 * pc, last)
+                assert 0 <= a and a + 16 <= M * bpr
+                v = w[a:a + 16].copy()
+                if c == nch - 1:
+                    past = min(c * PITCH + 16 * pc - last, 16)
+                    if past > 0:
+                        v = np.concatenate([v[past:], np.zeros(past, np.uint8)])
+                if k < per - 1 or N % 64 == 0 or lane + 64 * k < N:
+                    slot[r * PITCH + 16 * pc:r * PITCH + 16 * pc + 16] = v
+        for r in range(ROWS):
+            row = w[min(row0 + r, M - 1) * bpr:][:bpr][c * PITCH:(c + 1) * PITCH]
+            want = np.zeros(PITCH, np.uint8)
+            want[:row.size] = row
+            assert (slot[r * PITCH:(r + 1) * PITCH] == want).all(), (r, c)
+
+
+def panels(Ms, R):
+    return sum((M + R - 1) // R for M in Ms)
+
+
+def wave_first_rows(M, R, rows):
+    """First rows of the waves (of `rows` rows) of the first and of the last workgroup of R."""
+    last = (M + R - 1) // R - 1
+    return sorted({bx * R + w for bx in (0, last) for w in range(0, R, rows)})
+
+
+def check_tm(l, Ms, T, nb):
+    """k_q8_0_gemm_TM<WRN, WCN, PF, AL>."""
+    WRN, WCN, PF, AL = l.args
+    R, C = 16 * WRN, 16 * WCN
+    ROWS, NT, UNITS = R + C, 64 * WRN * WCN, 4 * (R + C)
+    PLANE = ROWS * 64 + 16
+    bpr, nst = nb * Q80, (nb + 1) // 2
+    assert l.block[0] == NT and l.grid[0] == panels(Ms, R) * ((T + C - 1) // C)
+    assert 2 * (2 * PLANE + 2 * ROWS * 4) + 4 * C <= 64 * 1024 and UNITS % 64 == 0
+    unit = np.arange((UNITS + NT - 1) // NT * NT)
+    unit = unit[unit < UNITS]
+    row, p = unit >> 2, unit & 3
+    assert row.max() == ROWS - 1
+    # a stage in LDS: every byte of two blocks' quants and every scale written once
+    q = np.zeros((2, PLANE), int)
+    sc = np.zeros((2, ROWS), int)
+    u, h, swz = p >> 1, p & 1, (row >> 2) & 3
+    for e in (0, 1):
+        at = row * 64 + 16 * ((2 * h + e) ^ swz)
+        assert (at + 16 <= PLANE).all()
+        for i in range(16):
+            np.add.at(q, (u, at + i), 1)
+    assert (q[:, :ROWS * 64] == 1).all()
+    if AL:
+        np.add.at(sc, (p[p < 2], row[p < 2]), 1)
+    else:
+        np.add.at(sc, (u[h == 0], row[h == 0]), 1)
+    assert (sc == 1).all()
+    # ... where lane (j, k) of a 16-row tile reads chunk k
+    j, k = lanes() & 15, lanes() >> 4
+    for tile in range(0, ROWS, 16):
+        assert (j * 64 + 16 * (k ^ (j >> 2)) == 64 * j + 16 * (k ^ (((tile + j) >> 2) & 3))).all()
+    # the loads of stage st (clamped), and that they are the quants and scales meant
+    for st in range(0, nst + PF + 1):
+        if AL:
+            assert nb % 2 == 0
+            s = min(st, nst - 1) * 68 + 16 * np.arange(4) + np.array([0, 0, 4, 4])
+            e = s + np.array([16, 16, 12, 12])
+            assert (s % 4 == 0).all() and (e % 4 == 0).all() and (s + 16 <= bpr).all() and (e + 4 <= bpr).all()
+            base = min(st, nst - 1) * 68
+            assert (s + np.array([2, 2, 0, 0]) == base + np.array([2, 18, 36, 52])).all()
+            assert s[0] == base and e[1] + 2 == base + 34  # the two scales
+        else:
+            b = np.minimum(2 * st + (np.arange(4) >> 1), nb - 1)
+            assert (b * Q80 + 2 + 16 * (np.arange(4) & 1) + 16 <= bpr).all()
+    # outputs: each cell of the tile by one lane register
+    cells = np.zeros((R, C), int)
+    for wave in range(WRN * WCN):
+        wr, wc = wave // WCN, wave % WCN
+        for r in range(4):
+            np.add.at(cells, (wr * 16 + 4 * k + r, wc * 16 + j), 1)
+    assert (cells == 1).all()
+
+
+def check_tq(l, Ms, T, nb):
+    """k_q8_0_gemm_TQ<NQ, NW>."""
+    NQ, NW = l.args
+    C, R, NT = 4 * NQ, 8 * NW, 64 * NW
+    PLANE = C * 64 + 32
+    XSLOT, UX = CHUNK * PLANE + CHUNK * C * 4, C * CHUNK * 2
+    assert l.block[0] == NT and l.grid[0] == panels(Ms, R) * ((T + C - 1) // C)
+    assert 2 * XSLOT + NW * 8 * PITCH + 4 * C <= 64 * 1024
+    for M in Ms:
+        for row0 in wave_first_rows(M, R, 8):
+            check_row_chunks(8, row0, M, nb)
+    # activation units: every half block of every token once, loads inside a row, stores inside a slot
+    i = np.arange(UX)
+    t, b = i // (2 * CHUNK), (i >> 1) % CHUNK
+    assert t.max() < C and len({(x, y, z) for x, y, z in zip(t.tolist(), b.tolist(), (i & 1).tolist())}) == UX
+    at = b * PLANE + t * 64 + 32 * (i & 1)
+    assert (at + 32 <= CHUNK * PLANE).all() and (at % 16 == 0).all()
+    assert (2 * ((b >> 1) * C + t) + (b & 1) < CHUNK * C).all()
+    for c in range((nb + CHUNK - 1) // CHUNK + 1):
+        assert (np.minimum(c * CHUNK + b, nb - 1) * Q80 + 2 + 16 + 16 <= nb * Q80).all()
+    # operand reads of a block pair
+    l_ = lanes()
+    jj, L, rg = l_ & 3, (l_ >> 2) & 7, l_ >> 5
+    for tt in range(CHUNK // 2):
+        w = (4 * rg + jj) * PITCH + 4 * L + 68 * tt
+        assert (w + 36 + 4 <= (4 * rg + jj + 1) * PITCH).all() and (w + 8 <= 8 * PITCH).all()
+        for n in range(NQ):
+            assert (jj * 64 + 8 * L + (2 * tt + 1) * PLANE + 256 * n + 8 <= CHUNK * PLANE).all()
+            assert (jj + tt * C + 4 * n < CHUNK * C // 2).all()
+    # the cell that lane L of (row group, token) stores
+    cells = np.zeros((8, C), int)
+    n, r = L >> 2, L & 3
+    ok = n < NQ
+    np.add.at(cells, ((4 * rg + r)[ok], (4 * n + jj)[ok]), 1)
+    assert (cells == 1).all()
+
+
+def check_sq(l, Ms, T, nb):
+    """k_q8_0_gemm_SQ<C, NW>."""
+    C, NW = l.args
+    R, NT, XU = 16 * NW, 64 * NW, 4
+    nbp, nch = (nb + 3) // 4 * 4, (nb + 15) // 16
+    assert l.block[0] == NT and l.grid[0] == panels(Ms, R) * ((T + C - 1) // C)
+    assert l.lds == nbp * C * 34 + NW * 16 * PITCH <= 160 * 1024
+    for M in Ms:
+        for row0 in wave_first_rows(M, R, 16)[:: max(1, NW // 2)]:
+            check_row_chunks(16, row0, M, nb)
+    # activation units: all of whole groups of 4 blocks, each once, in batches of XU * NT
+    nu, nup = 2 * C * nb, 2 * C * nbp
+    i = np.concatenate([np.arange(NT) + i0 + u * NT for i0 in range(0, nup, XU * NT) for u in range(XU)])
+    s = np.minimum(i, nu - 1)
+    assert (s // (2 * C) * Q80 + 2 + 16 * ((s // C) & 1) + 16 <= nb * Q80).all()
+    i = i[i < nup]
+    assert len(set(i.tolist())) == nup == i.size
+    t, h, b = i % C, (i // C) & 1, i // (2 * C)
+    assert ((b * C + t) * 32 + 16 * h + 16 <= nbp * C * 32).all() and (b * C + t < nbp * C).all()
+    # operand reads of group tt of a chunk: weights in the row's chunk, activation blocks below nbp
+    l_ = lanes()
+    j, k = l_ & 15, l_ >> 4
+    for c in range(nch):
+        for tt in range(min(4, (nb - 16 * c + 3) // 4)):
+            assert (8 * k + 34 * (4 * tt + 3) + 2 + 8 <= PITCH).all() and (8 * k + 34 * (4 * tt + 2) + 12 <= PITCH).all()
+            assert (34 * k + 136 * tt + 2 <= PITCH).all()
+            blk = 16 * c + 4 * tt
+            assert (blk + 3 < nbp) and (((blk + 3) * C + j % C) * 32 + 8 * k + 8 <= nbp * C * 32).all()
+            assert ((blk + k) * C + j % C < nbp * C).all()
+
+
+FEW = [(4096, 8, 4096), (4096, 16, 4128), (14336, 3, 32), (8193, 2, 4096), (33, 600, 64), (1057, 40, 1440),
+       (4099, 65, 4128), (4099, 65, 4096), (2047, 130, 544), (32000, 5, 96), (128, 512, 4096), (20000, 65, 1440),
+       (300, 300, 4096), (4100, 5, 14336)]
+
+
+@pytest.mark.parametrize("M,T,K", FEW)
+def test_q8_0_few_tokens_T_in_bounds(launched, M, T, K):
+    for w in (W, W + 1):
+        l, = launched("bpd_qmatmul_q8_0_dispatch_gpu", w, X, OUT, M, T, K)
+        check_q8_0_T(l, M, T, K // 32, w - W)
+
+
+@pytest.mark.parametrize("M,T,K", FEW + [(1, 1, 32), (5, 3, 64), (16, 1, 160), (65, 4, 544), (2048, 16, 28672),
+                                         (11584, 9, 16256), (70, 1, 256)])
+def test_q8_0_few_tokens_S_in_bounds(launched, M, T, K):
+    l, = launched("bpd_qmatmul_q8_0_dispatch_s_gpu", W, X, OUT, M, T, K)
+    if l.kernel == "k_q8_0_gemm_SQ":
+        check_sq(l, [M], T, K // 32)
+
+
+def test_q8_0_few_tokens_forms_are_all_replayed(launched):
+    """The shapes above reach every form of the three kernels."""
+    seen = set()
+    for M, T, K in FEW:
+        for w in (W, W + 1):
+            seen |= {(l.kernel, *l.args) for l in launched("bpd_qmatmul_q8_0_dispatch_gpu", w, X, OUT, M, T, K)}
+        seen |= {(l.kernel, *l.args) for l in launched("bpd_qmatmul_q8_0_dispatch_s_gpu", W, X, OUT, M, T, K)}
+    assert {("k_q8_0_gemm_TQ", 1, 4), ("k_q8_0_gemm_TQ", 2, 4), ("k_q8_0_gemm_TM", 2, 4, 4, 0),
+            ("k_q8_0_gemm_TM", 2, 4, 4, 1), ("k_q8_0_gemm_TM", 4, 4, 4, 1), ("k_q8_0_gemm_SQ", 4, 4),
+            ("k_q8_0_gemm_SQ", 8, 4), ("k_q8_0_gemm_SQ", 16, 4), ("k_q8_0_gemm_SQ", 16, 8)} <= seen, seen
 
 
 # ---------------------------------------------------------------- Q8_0 S-order GEMM (MFMA)
@@ -532,29 +789,6 @@ def test_q8_0_gemm_S_in_bounds(mw, mt, K):
                     assert wa.min() >= 0 and (wa + 34).max() <= mw * bpr
                     assert xa.min() >= 0 and (xa + 34).max() <= mt * bpr
                     assert u.max() < 4 and rr.max() < 128
-
-
-# ---------------------------------------------------------------- fused Q8_K quantization prologue
-
-def fused_config(rows, nb):
-    """(WPB, IT) of launch_qmatmul_q4k_fused_multi in q4k.hip."""
-    return (4, 1) if nb <= 16 else (16, 1)
-
-
-@pytest.mark.parametrize("rows", [1, 300, 8192, 8193, 14336, 28672])
-def test_fused_quantization_covers_x_and_stays_in_bounds(rows):
-    for nb in range(1, 65):  # fused_max_k() = 64 * 256
-        WPB, IT = fused_config(rows, nb)
-        assert IT * 4 * WPB >= nb, "some Q8_K block would never be quantized"
-        tid = np.arange(64 * WPB)
-        gq, li = tid >> 4, tid & 15
-        for it in range(IT):
-            b = np.minimum(it * 4 * WPB + gq, nb - 1)
-            assert ((b * 256 + 16 * li + 16) <= nb * 256).all() and (b >= 0).all()
-            bw = it * 4 * WPB + gq
-            ok = bw < nb
-            assert ((bw[ok] * 304 + 16 * li[ok] + 16) <= nb * 304).all()
-            assert ((bw[ok] * 304 + 288 + 4) <= nb * 304).all()
 
 
 # ---------------------------------------------------------------- Q8_0 S-order GEMM, coalesced staging
@@ -694,34 +928,56 @@ def test_q6k_gemv_in_bounds(M, K, order):
                 assert min(row0 + r, M - 1) < M
 
 
-@pytest.mark.parametrize("mw,mt,K", [(4096, 1, 14336), (14336, 1, 4096), (13, 3, 160), (8, 1, 32), (9, 2, 64), (7, 5, 128)])
-def test_q8_pad64_gemv_in_bounds(mw, mt, K):
-    """k_q8_0_gemv_T<.., 1> / k_q8_0_gemm_T<1>: W records (b, n) at (b*mw + n)*64."""
-    cfg = q8_gemv_config(mw, mt, K)
-    if cfg is None:
-        return
+def check_pad(l, Ms, nb):
+    """k_pad_gemv<NW, NH, U, SWG>: records, loads past a row's end, the activation in LDS and the
+    spare blocks that the read ahead reaches."""
+    NW, NH, U, SWG = l.args
+    NT, R = 64 * (NW + NH), 32 if SWG else 16 * NW
+    assert l.block[0] == NT and l.grid[0] == (Ms[0] // 32 if SWG else panels(Ms, R))
+    assert l.lds == (nb + 4) * 64 <= 160 * 1024
+    lane = lanes()
+    p = lane & 3
+    for N in Ms:
+        for row0 in wave_first_rows(N, R, 16):
+            base = min(row0, N - 1)
+            off = (np.minimum(row0 + (lane >> 2), N - 1) - base) * 64 + 8 * p
+            assert off.min() >= 0
+            for issued in (0, 1, nb - 1, nb, nb + U):  # wnext stops at the last block
+                at = base * 64 + min(issued, nb - 1) * N * 64 + off
+                assert at.min() >= 0 and (at + 12).max() <= nb * N * 64 and (8 * p + 12 <= 36).all()
+    # activation units, 8 per thread and batch: dwords 2p, 2p + 1 of block i / 4
+    i = np.concatenate([np.arange(NT) + i0 + k * NT for i0 in range(0, 4 * nb, 8 * NT) for k in range(8)])
+    s = np.minimum(i, 4 * nb - 1)
+    assert ((s >> 2) * Q80 + 6 + 8 * (s & 3) + 4 <= nb * Q80).all()
+    i = i[i < 4 * nb]
+    assert i.size == 4 * nb == len(set(i.tolist()))
+    # reads: groups of 4 blocks, the next group ahead of each
+    reads = {0, 1, 2, 3}
+    b = 0
+    while b + U <= nb:
+        reads |= {b + u + 4 + g for u in range(0, U, 4) for g in range(4)}
+        b += U
+    reads |= {b + u for u in range(U) if b + u < nb}
+    assert max(reads) < nb + 4 and set(range(nb)) <= reads
+
+
+PAD = [(4096, 1, 14336), (14336, 1, 4096), (13, 3, 160), (8, 1, 32), (9, 2, 64), (7, 5, 128), (5120, 1, 1024),
+       (2048, 4, 40960), (3000, 1, 96), (12289, 1, 224), (33, 2, 90000 // 32 * 32), (4097, 1, 16384), (6145, 3, 544)]
+
+
+@pytest.mark.parametrize("mw,mt,K", PAD)
+def test_q8_pad64_gemv_in_bounds(launched, mw, mt, K):
+    """W records (b, n) at (b*mw + n)*64."""
     nb = K // 32
-    w_size = nb * mw * 64
-    kind, WPB, U = cfg
-    if kind == "producer":
-        check_producer(mw, mt, nb, 1, w_size)
-        return
-    waves = (mw + 7) // 8
-    grid = (waves + WPB - 1) // WPB if kind == "pipelined" else (waves + 3) // 4
-    l = lanes()
-    L = l & 7
-    for blk in sorted({0, grid - 1}):
-        for wave in range(WPB):
-            row = (blk * WPB + wave) * 8 + (l >> 3)
-            row0 = min((blk * WPB + wave) * 8, mw - 1)
-            doff = (np.maximum(np.minimum(row, mw - 1), row0) - row0) * 64
-            voff = doff + 4 + 4 * L
-            for b0 in range(0, nb + 2 * U, U):
-                for u in range(U):
-                    b = min(b0 + u, nb - 1)
-                    base = row0 * 64 + b * mw * 64
-                    assert (base + voff + 4).max() <= w_size and (base + doff).min() >= 0
-                    assert (base + doff + 2).max() <= w_size
+    l, = launched("bpd_qmatmul_q8_pad64_gpu", W, X, OUT, mw, mt, K)
+    assert l.grid[1] == mt
+    if l.kernel == "k_pad_gemv":
+        check_pad(l, [mw], nb)
+    elif l.kernel == "k_q8_0_gemm_T":
+        check_plain(l, mw, nb, nb * mw * 64)
+    else:
+        assert l.kernel == "k_q8_0_gemv_TP" and l.args[0] == 1 and l.lds + 2 * 64 * 36 * 4 <= 64 * 1024
+        check_producer(mw, mt, nb, 1, nb * mw * 64)
 
 
 @pytest.mark.parametrize("N,K", [(1, 32), (7, 96), (300, 4096)])
@@ -915,7 +1171,7 @@ def test_folded_norm_partials_fit_their_buffers(E, F):
     def grid(M, K):
         if K // 256 == 56:
             return (M + 7) // 8
-        R = span_rows_per_wave(M)
+        R = 1 if M <= 2048 else 2
         return ((M + R - 1) // R + 3) // 4
     for K in (E, F):
         g = grid(E, K)
