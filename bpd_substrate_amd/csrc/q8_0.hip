@@ -335,8 +335,6 @@ __device__ __forceinline__ void tp_gemv(const uint8_t* __restrict__ W, const uin
     p.rowbase = W + (int64_t)row * (LAYOUT == 0 ? (int64_t)nb * kQ80Bytes : 64);
     p.bstride = LAYOUT == 0 ? kQ80Bytes : (int64_t)m_weight * 64;
     const int nch = (nb + kTpChunk - 1) / kTpChunk;
-    // loads return in order, so: chunk 0, then the activation row (the first
-    // barrier waits for it), then the rest of the prefetch
     // the activation row first (an L2 hit for every workgroup but the first few),
     // then the weight prefetch: loads return in order, so staging issued after
     // the prefetch would wait for all of it

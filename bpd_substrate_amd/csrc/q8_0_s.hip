@@ -14,8 +14,14 @@ namespace bpdq {
 // blocks in order, S_b the exact dot of the cell's two blocks.  k_q8_0_gemm_SH stages 128
 // tokens for any token count and waits for one half-stage of 4 blocks at a time, so a few
 // tokens cost what 128 do and every 4 blocks a memory round trip: 14336x8, K = 4096, 46 us
-// there, 18 here (62 MB at 3.5 TB/s; a wave alone on its SIMD issues an instruction every 5
-// cycles, 34 VALU and MFMA of them per 4 blocks, and that bounds it).  Here the workgroup puts
+// there, 18 here (62 MB at 3.5 TB/s; 128256x1 230 and 103 us, 5.4 TB/s).  What bounds it: the
+// memory where the launch fills the chip; with few rows, a wave's own instructions.  For any C a
+// wave issues 57 VALU and MFMA instructions per 4 blocks (16 conversions, 16 multiplications, 16
+// additions, 4 realignments, 5 MFMA), about 290 cycles at the 5 cycles that a wave alone on its
+// SIMD needs for each; 4096x1 (64 workgroups, one wave per SIMD) takes 13.6 us with C = 4 and 17.6
+// with C = 16, 660 and 960 cycles per 4 blocks beyond the launch and the staging: the rest is
+// operand reads from LDS (lanes of equal tokens share them) and the staging of the next chunk,
+// not taken apart further.  Here the workgroup puts
 // its C activation rows into LDS once; after that barrier each wave runs by itself over its
 // 16 rows: chunks of 16 blocks as 16-byte pieces, two chunks in flight in registers, through
 // its own LDS slot (a wave's LDS operations execute in order, so the next chunk is written
