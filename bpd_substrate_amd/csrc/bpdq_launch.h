@@ -98,7 +98,8 @@ bool launch_pad_gemv(const uint8_t* const* W, float* const* y, const int* N, int
 // Up to 3 matrices sharing one activation row: y[i][N[i]].
 void launch_q8_pad64_multi(const uint8_t* const* W, float* const* y, const int* N, int n, const uint8_t* Xq, int K,
                            hipStream_t s);
-// Gate and up with SwiGLU and the Q8_0 blocks of y; false (nothing launched) if K does not fit.
+// Gate and up with SwiGLU and the Q8_0 blocks of y; false (nothing launched) if K does not fit or two
+// products and k_swiglu are faster.
 bool launch_pad_swiglu(const uint8_t* Wg, const uint8_t* Wu, float* y, uint8_t* yq, int F, const uint8_t* Xq, int K,
                        hipStream_t s);
 
